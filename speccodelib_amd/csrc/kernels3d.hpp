@@ -75,9 +75,20 @@ struct ZOffR {
 };
 __device__ inline ZOffR zoffr(const Tile& t) { return ZOffR{(uint32_t)t.base, (uint32_t)t.rs, (uint32_t)t.bs, t.sh}; }
 
+// The spherical truncation k^2 >= kc2 as the passes of one axis see it: a
+// (kx, ky) column with kx^2 + ky^2 >= kc2 holds no kept mode, and neither
+// does a kx with kx^2 >= kc2.  Where a field is known to be zero there (the
+// z-inverse of a truncated state), or only its kept modes are used
+// afterwards (the RHS of a step's last stage), the y- and x-passes leave
+// those columns out: at the 2/3 radius 65% of the (kx, ky) columns and a
+// third of the kx.  Nothing is read from or written to them.
+template <class R>
+__host__ __device__ inline bool col_cut(int kx, int ky, R kc2) {
+  return (R)(kx * kx + ky * ky) >= kc2;
+}
+
 template <int CW, int AXIS>
-__device__ inline Tile col_tile(const Geom& g, int wg, int c) {
-  const int xtn = g.mx / CW;
+__device__ inline Tile col_tile(const Geom& g, int wg, int c, int xtn) {
   Tile t;
   if constexpr (AXIS == 1) {
     const int nmain = xtn * g.nz;
@@ -120,6 +131,23 @@ __device__ inline Tile col_tile(const Geom& g, int wg, int c) {
     }
   }
   return t;
+}
+
+template <int CW, int AXIS>
+__device__ inline Tile col_tile(const Geom& g, int wg, int c) {
+  return col_tile<CW, AXIS>(g, wg, c, g.mx / CW);
+}
+
+// The tiles of a y-pass that leaves out the columns of the truncation:
+// nkx = number of kept kx; the first tiles of every z hold them, the tail
+// tiles only run when kx = nx/2 is kept.
+template <int CW>
+__host__ __device__ inline int ycut_tiles(const Geom& g, int nkx) {
+  return (min(nkx, g.mx) + CW - 1) / CW;
+}
+template <int CW>
+inline int ycut_grid(const Geom& g, int nkx) {
+  return ycut_tiles<CW>(g, nkx) * g.nz + (nkx > g.mx ? (g.nz + CW - 1) / CW : 0);
 }
 
 // Main tiles plus tail tiles; a partial last tail tile (batch count not a
@@ -175,10 +203,56 @@ __device__ inline int xcd_swizzle(int b, int G) {
   return (b & 7) * (G8 >> 3) + (b >> 3);
 }
 
-// Pure batched column FFT, in place, one field per blockIdx.y.
-template <class R, int N, int AXIS, int DIR>
+// p[o] where in, else 0.  Not a branch: a lane that is out reads the entry at
+// rest instead (one its line has anyway), so that the loads of a line go out
+// together; a branch per load made the small grids' passes slower.
+template <class R>
+__device__ inline cpx<R> ld_or_zero(const cpx<R>* p, int64_t o, int64_t rest, bool in) {
+  const cpx<R> v = p[in ? o : rest];
+  return in ? v : mk<R>(0, 0);
+}
+
+// The truncation a y- or x-pass with CUT runs with: its radius squared and
+// the number of kept kx (infinite and nx/2 + 1: all).  The variants without
+// it are for the passes that are never cut: at 32^3 a pass is bound by its
+// instruction count and fetch, and steps were 12% slower without them.
+template <class R>
+struct Cut {
+  R kc2;
+  int nkx;
+};
+
+// Tile order of a z-pass that leaves tiles out: the left-out tiles are those
+// of the large |ky|, so contiguous ranges of y per XCD (xcd_swizzle) would
+// leave two of the eight idle.  Block b takes a tile of a y with y mod 8 =
+// b mod 8 instead, so each XCD gets every 8th y.
+template <int CW>
+__device__ inline int zcut_swizzle(const Geom& g, int b) {
+  const int xtn = g.mx / CW;
+  if (b >= xtn * g.ny) return b;
+  const int i = b >> 3;
+  return ((i / xtn) * 8 + (b & 7)) * xtn + i % xtn;
+}
+
+// Whether no column of z-pass tile wg holds a kept mode.
+template <class R, int CW>
+__device__ inline bool zcut_tile(const Geom& g, int wg, R kc2) {
+  const int xtn = g.mx / CW;
+  if (wg < xtn * g.ny) return col_cut<R>(wg % xtn * CW, kwave(wg / xtn, g.ny), kc2);
+  const int y = (wg - xtn * g.ny) * CW;
+  int least = 1 << 20;
+#pragma unroll
+  for (int c = 0; c < CW; ++c) least = min(least, abs(kwave(y + c, g.ny)));
+  return col_cut<R>(g.mx, least, kc2);
+}
+
+// Pure batched column FFT, in place, one field per blockIdx.y.  CUT (AXIS 1):
+// modes beyond the truncation are taken as zero (inverse) or not stored
+// (forward); grid of ycut_grid.  At 512^3, 3 fields: inverse 627 -> 438 us,
+// forward 626 -> 358 us.
+template <class R, int N, int AXIS, int DIR, bool CUT = false>
 __global__ __launch_bounds__((ColCfg<R, N>::BS)) void k_colfft(cpx<R>* __restrict__ f0, int64_t fstride, Geom g,
-                                                              const cpx<R>* __restrict__ tw, int tws) {
+                                                              const cpx<R>* __restrict__ tw, int tws, Cut<R> cut) {
   using CC = ColCfg<R, N>;
   constexpr int CW = CC::CW, E = CC::E, T = CC::T;
   __shared__ cpx<R> lds[lds_pad(N) * CW];
@@ -186,14 +260,26 @@ __global__ __launch_bounds__((ColCfg<R, N>::BS)) void k_colfft(cpx<R>* __restric
   for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
   const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
   cpx<R>* f = f0 + (int64_t)blockIdx.y * fstride;
-  const Tile t = col_tile<CW, AXIS>(g, xcd_swizzle(blockIdx.x, gridDim.x), c);
+  Tile t = col_tile<CW, AXIS>(g, xcd_swizzle(blockIdx.x, gridDim.x), c, CUT ? ycut_tiles<CW>(g, cut.nkx) : g.mx / CW);
+  if (CUT && t.kx >= cut.nkx) t.ok = false;
   cpx<R> v[E];
 #pragma unroll
-  for (int m = 0; m < E; ++m) v[m] = t.ok ? f[t.off(rt + T * m)] : mk<R>(0, 0);
+  for (int m = 0; m < E; ++m) {
+    const int j = rt + T * m;
+    if constexpr (CUT && DIR > 0) {
+      v[m] = ld_or_zero(f, t.off(j), t.base, t.ok && !col_cut<R>(t.kx, kwave(j, N), cut.kc2));
+    } else {
+      v[m] = t.ok ? f[t.off(j)] : mk<R>(0, 0);
+    }
+  }
   Line<R, N, E, DIR>::run(v, lds, rt, twl, 1, ColIdx<CW>{c});
   if (!t.ok) return;
 #pragma unroll
-  for (int m = 0; m < E; ++m) f[t.off(Line<R, N, E, DIR>::out_pos(m, rt))] = v[m];
+  for (int m = 0; m < E; ++m) {
+    const int j = Line<R, N, E, DIR>::out_pos(m, rt);
+    if (CUT && DIR < 0 && col_cut<R>(t.kx, kwave(j, N), cut.kc2)) continue;
+    f[t.off(j)] = v[m];
+  }
 }
 
 // z-inverse of a velocity column held in registers (slot m = index
@@ -203,6 +289,8 @@ __global__ __launch_bounds__((ColCfg<R, N>::BS)) void k_colfft(cpx<R>* __restric
 // five transforms, stored to w[0..4] (u, then w_x, w_y) at stride ws.
 // w_z = i (kx u_y - ky u_x) needs no kz, so the y-inverse builds it from
 // the transformed u_x, u_y (k_yinv_vort) and one field less crosses HBM.
+// live: false on the lanes whose column holds no kept mode (col_cut): all of
+// it is zero, and nothing is stored (the y-inverse takes it as zero).
 // Offsets are 32-bit (ZOff).  PARK (1024-thread workgroups, one per CU at the
 // 128-VGPR cap, and 1024-point lines, one 512-thread workgroup per CU at
 // 2 waves per SIMD: LDS to spare in both): Uz waits in park (E BS entries,
@@ -211,7 +299,7 @@ __global__ __launch_bounds__((ColCfg<R, N>::BS)) void k_colfft(cpx<R>* __restric
 template <class R, int N, int E, int CW, bool PARK, int ZS>
 __device__ inline void zinv_store(cpx<R> (&ux)[E], cpx<R> (&uy)[E], cpx<R> (&uz)[E], cpx<R>* lds, cpx<R>* park,
                                   const cpx<R>* twl, int rt, int c, R kx, R ky, int nz, ZOff<ZS> zo,
-                                  cpx<R>* __restrict__ w, int64_t ws) {
+                                  cpx<R>* __restrict__ w, int64_t ws, bool live = true) {
   constexpr int T = N / E, BS = CW * T;
   using L = Line<R, N, E, +1>;
   // An empty asm that "changes" the base offset: the store addresses below
@@ -223,32 +311,36 @@ __device__ inline void zinv_store(cpx<R> (&ux)[E], cpx<R> (&uy)[E], cpx<R> (&uz)
   const int slot = rt * CW + c;
   cpx<R> d[E];
   L::run(uz, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+  auto store = [&](int f, auto&& val) {
+    if (!live) return;
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    (w + 2 * ws)[off(m)] = uz[m];
-    if constexpr (PARK) park[m * BS + slot] = uz[m];
+    for (int m = 0; m < E; ++m) (w + f * ws)[off(m)] = val(m);
+  };
+  store(2, [&](int m) { return uz[m]; });
+  if constexpr (PARK) {
+#pragma unroll
+    for (int m = 0; m < E; ++m) park[m * BS + slot] = uz[m];
   }
   auto Uz = [&](int m) { return PARK ? park[m * BS + slot] : uz[m]; };
 #pragma unroll
   for (int m = 0; m < E; ++m) d[m] = kz(m) * uy[m];
   L::run(d, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
-#pragma unroll
-  for (int m = 0; m < E; ++m) (w + 3 * ws)[off(m)] = mul_i(ky * Uz(m) - d[m]);
+  store(3, [&](int m) { return mul_i(ky * Uz(m) - d[m]); });
   L::run(uy, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
-#pragma unroll
-  for (int m = 0; m < E; ++m) (w + ws)[off(m)] = uy[m];
+  store(1, [&](int m) { return uy[m]; });
 #pragma unroll
   for (int m = 0; m < E; ++m) d[m] = kz(m) * ux[m];
   L::run(d, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
-#pragma unroll
-  for (int m = 0; m < E; ++m) (w + 4 * ws)[off(m)] = mul_i(d[m] - kx * Uz(m));
+  store(4, [&](int m) { return mul_i(d[m] - kx * Uz(m)); });
   L::run(ux, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
-#pragma unroll
-  for (int m = 0; m < E; ++m) w[off(m)] = ux[m];
+  store(0, [&](int m) { return ux[m]; });
 }
 
 // ZINV: z-inverse of the stage state s (3 fields at stride sstride) into
-// w[0..4] (stride wstride), see zinv_store.
+// w[0..4] (stride wstride), see zinv_store.  Its stores are conditional
+// (on t.ok, always true here) as those of k_zfwd_rhs are: with the same
+// blocks around the same arithmetic the compiler contracts both alike, so a
+// chain started here continues the bits of one that ran on.
 template <class R, int N, int CWZ, int EZ = 0, int ZS = 0>
 __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zinv_vort(const cpx<R>* __restrict__ s,
                                                                      int64_t sstride, cpx<R>* __restrict__ w,
@@ -273,27 +365,36 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zinv_vort(const
     ux[m] = ld_once<R, (CW >= 16)>(s + o);
   }
   zinv_store<R, N, E, CW, PARK, ZS>(ux, uy, uz, lds, park, twl, rt, c, (R)t.kx, (R)kwave(t.oth, g.ny), g.nz, zo, w,
-                                    wstride);
+                                    wstride, t.ok);
 }
 
 // YINV (u_x, u_y and w_z): y-inverse of fields 0 and 1 (u_x, u_y) and of
 // w_z = i (kx Uy - ky Ux), formed before the transform while ky is still a
 // spectral index, into field 5; in place at stride fs.  Fields 2..4 (u_z,
-// w_x, w_y) take the plain column kernel.
-template <class R, int N>
+// w_x, w_y) take the plain column kernel.  CUT: as k_colfft's (512^3: 582 ->
+// 399 us).
+template <class R, int N, bool CUT = false>
 __global__ __launch_bounds__((ColCfg<R, N>::BS)) void k_yinv_vort(cpx<R>* __restrict__ W, int64_t fs, Geom g,
-                                                                const cpx<R>* __restrict__ tw, int tws) {
+                                                                const cpx<R>* __restrict__ tw, int tws, Cut<R> cut) {
   using CC = ColCfg<R, N>;
   constexpr int CW = CC::CW, E = CC::E, T = CC::T;
   __shared__ cpx<R> lds[lds_pad(N) * CW];
   __shared__ cpx<R> twl[N];  // first read after a barrier inside the transform
   for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
   const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
-  const Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, gridDim.x), c);
+  Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, gridDim.x), c, CUT ? ycut_tiles<CW>(g, cut.nkx) : g.mx / CW);
+  if (CUT && t.kx >= cut.nkx) t.ok = false;
   using L = Line<R, N, E, +1>;
   auto load = [&](cpx<R>(&v)[E], int f) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = t.ok ? W[t.off(rt + T * m) + f * fs] : mk<R>(0, 0);
+    for (int m = 0; m < E; ++m) {
+      const int j = rt + T * m;
+      if constexpr (CUT) {
+        v[m] = ld_or_zero(W + f * fs, t.off(j), t.base, t.ok && !col_cut<R>(t.kx, kwave(j, N), cut.kc2));
+      } else {
+        v[m] = t.ok ? W[t.off(j) + f * fs] : mk<R>(0, 0);
+      }
+    }
   };
   auto store = [&](cpx<R>(&v)[E], int f) {
     if (!t.ok) return;
@@ -374,6 +475,91 @@ __device__ inline cpx<R> stage_apply(const StageIn<R>& in, cpx<R> a, I o, cpx<R>
   return out;
 }
 
+// The three velocity components of a mode at once (fields fs apart): one
+// branch per condition for all of them, so their loads go out together.
+// cut: the mode is beyond the truncation of the step's end, where the new v
+// is 0 whatever du and the history hold, so neither is kept there; vcut: v
+// is known to be 0 there (the solver's own last step wrote it) and is not
+// read.  NT: nontemporal loads (whole-line accesses only, ld_once).
+template <int MODE, bool NT, class R>
+__device__ inline void stage_load3(StageIn<R> (&in)[3], uint32_t o, int64_t fs, const cpx<R>* V, const cpx<R>* DU,
+                                   const cpx<R>* S, bool cut, bool vcut) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q) in[q] = {mk<R>(0, 0), mk<R>(0, 0)};
+  if (MODE < 4 && !(cut && vcut)) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) in[q].v = ld_once<R, NT>(V + q * fs + o);
+  }
+  if (MODE > 1 && !cut) {
+    const cpx<R>* const H = MODE == 7 ? S : DU;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      if constexpr (MODE >= 5) in[q].v = ld_once<R, NT>(V + q * fs + o);
+      if constexpr (MODE != 5) in[q].h = ld_once<R, NT>(H + q * fs + o);
+    }
+  }
+}
+
+// stage_apply's arithmetic.  s: the new stage state (MODE 1..3) or the new v
+// (MODE 4); du: the new accumulator (MODE 1..3, only used where not cut).
+template <class R>
+struct StageOut {
+  cpx<R> s, du;
+};
+template <int MODE, class R>
+__device__ inline StageOut<R> stage_math(const StageIn<R>& in, cpx<R> a, R em1, R x, bool cut) {
+  const cpx<R> v = in.v;
+  if constexpr (MODE == 1) {
+    const cpx<R> u = v + ((R)1 / (R)6) * a, q = v + (R)0.5 * a;
+    return {q + em1 * q, u + expm1_r((R)2 * x) * u};
+  } else if constexpr (MODE == 2 || MODE == 3) {
+    const cpx<R> q = ((R)1 / (R)3) * a;
+    const cpx<R> du = in.h + (q + em1 * q);
+    const cpx<R> ev = v + em1 * v;
+    if constexpr (MODE == 2) return {ev + (R)0.5 * a, du};
+    const cpx<R> u = ev + a;
+    return {u + em1 * u, du};
+  } else {
+    return {cut ? mk<R>(0, 0) : in.h + ((R)1 / (R)6) * a, mk<R>(0, 0)};
+  }
+}
+
+// A non-finite new v raises the sticky flag *nf (read first, so that a field
+// full of NaN does not make every lane an atomic).
+template <class R>
+__device__ inline void flag_nonfinite(unsigned* nf, cpx<R> v) {
+  if (nf && !(isfinite(v.x) && isfinite(v.y)) && *(volatile unsigned*)nf == 0u) atomicOr(nf, 1u);
+}
+
+// stage_math of the three components of a mode with its stores: DU and S (only
+// where store_s), or V.  cut, vcut: as stage_load3; with vcut the zeros of v
+// beyond the cut stand.
+template <int MODE, class R>
+__device__ inline void stage_apply3(const StageIn<R> (&in)[3], const cpx<R> (&a)[3], cpx<R> (&out)[3], uint32_t o,
+                                    int64_t fs, cpx<R>* V, cpx<R>* DU, cpx<R>* S, R em1, R x, bool cut, bool store_s,
+                                    unsigned* nf, bool vcut) {
+  StageOut<R> r[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    r[q] = stage_math<MODE, R>(in[q], a[q], em1, x, cut);
+    out[q] = r[q].s;
+  }
+  if (MODE < 4 && !cut) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) (DU + q * fs)[o] = r[q].du;
+  }
+  if (MODE < 4 && store_s) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) (S + q * fs)[o] = r[q].s;
+  }
+  if (MODE >= 4 && !(cut && vcut)) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) (V + q * fs)[o] = r[q].s;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) flag_nonfinite(nf, r[q].s);
+  }
+}
+
 // Parameters of the fused ZFWD epilogue.
 template <class R>
 struct RhsParams {
@@ -383,6 +569,9 @@ struct RhsParams {
   R kc2;        // 2/3 cut: zero where k2 >= kc2
   int forced;   // 0 none, 1 force(), 2 force_heli()
   int dealias;  // 1: zero k2 >= kc2 in the RHS as well
+  int trunc = 0;  // leave out what lies beyond kc2 and is not used (trunc_pays)
+  int vcut = 0;   // v is 0 where k2 >= kc2 (the solver's own last step wrote it)
+  int scut = 0;   // the new stage state is 0 where k2 >= kc2 (v truncated, RHS truncated)
   unsigned* nonfinite = nullptr;  // sticky flag set by stage 4 on a non-finite v (null: no check)
   const double* ab = nullptr;     // IF-AB2 (MODE 5..7): the step's coefficients on the device (AB_*)
 };
@@ -423,6 +612,42 @@ __device__ inline cpx<R> ab_apply(const StageIn<R>& in, cpx<R> a, I o, cpx<R>* V
   return out;
 }
 
+// ab_apply's arithmetic.
+template <class R>
+struct AbWeights {
+  R dt, cS, cek, cdel;
+};
+template <int MODE, class R>
+__device__ inline cpx<R> ab_math(const StageIn<R>& in, cpx<R> a, const AbWeights<R>& w, R e1, R e2, bool cut) {
+  const cpx<R> v = in.v;
+  cpx<R> y;
+  if constexpr (MODE == 5) y = v + w.dt * a;
+  else if constexpr (MODE == 6) y = w.cS * (in.h + e2 * in.h) + w.cek * v + w.cdel * a;
+  else y = v + w.cS * a + w.cek * (in.h + e2 * in.h);
+  return cut ? mk<R>(0, 0) : y + e1 * y;
+}
+// ab_math of the three components of a mode with its stores.  over: k2 >=
+// kcut^2, where the history is never used and not kept; vcut: as stage_apply3.
+template <int MODE, class R>
+__device__ inline void ab_apply3(const StageIn<R> (&in)[3], const cpx<R> (&a)[3], cpx<R> (&out)[3], uint32_t o,
+                                 int64_t fs, cpx<R>* V, cpx<R>* DU, cpx<R>* S, const AbWeights<R>& w, R e1, R e2,
+                                 bool cut, unsigned* nf, bool over, bool vcut) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q) out[q] = ab_math<MODE, R>(in[q], a[q], w, e1, e2, cut);
+  if (!over) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      if constexpr (MODE == 5) (DU + q * fs)[o] = in[q].v;
+      if constexpr (MODE != 6) (S + q * fs)[o] = a[q];
+    }
+  }
+  if (!(over && vcut)) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) (V + q * fs)[o] = out[q];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) flag_nonfinite(nf, out[q]);
+  }
+}
 
 // ZFWD: z-forward of the three transformed products + forcing + the
 // pointwise part of symmetrize + projection (+ optional RHS truncation),
@@ -444,7 +669,10 @@ __device__ inline cpx<R> ab_apply(const StageIn<R>& in, cpx<R> a, I o, cpx<R>* V
 // (zinv_store), so that RHS needs no z-inverse pass of its own; S is then
 // stored only where the forcing reads it (k2 < fk2).  Each workgroup reads
 // all of its columns of W before it writes them.
-template <class R, int N, int MODE, int CWZ, int EZ = 0, bool FUSED = false, int ZS = 0>
+//
+// TR: the variant that can leave out what lies beyond the truncation; p.trunc
+// says whether it does.
+template <class R, int N, int MODE, int CWZ, int EZ = 0, bool FUSED = false, int ZS = 0, bool TR = true>
 __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>* W, int64_t fstride, cpx<R>* V,
                                                                     cpx<R>* DU, cpx<R>* S, const cpx<R>* st,
                                                                     const double* __restrict__ coef, RhsParams<R> p,
@@ -455,11 +683,35 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
   __shared__ cpx<R> twl[N];  // this line length's twiddles; first read after a barrier
   for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
   const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
-  const Tile t = col_tile<CW, 2>(g, xcd_swizzle(blockIdx.x, gridDim.x), c);
+  // MODE 4 and up end a step, so only the modes inside the truncation count:
+  // columns without any (col_cut) are neither read nor transformed, and their
+  // z-inverse is not stored (the next y-inverse leaves them out).  With
+  // scut (RHS truncated as well) the same holds for every stage.
+  const bool trunc = TR && p.trunc, vcut = TR && p.vcut;
+  const bool scut = trunc && (MODE >= 4 || (MODE > 0 && p.scut));
+  const bool ncut = trunc && (MODE >= 4 || p.dealias);
+  const int wg = scut ? zcut_swizzle<CW>(g, blockIdx.x) : xcd_swizzle(blockIdx.x, gridDim.x);
+  const Tile t = col_tile<CW, 2>(g, wg, c);
   // 32-bit in-field offsets: the three components go through their own
   // base pointers, so a thread keeps one 32-bit offset per slot instead of
   // 64-bit ones (which spilled).
   const ZOff<ZS> zo = zoff<ZS>(t);
+  if (scut && zcut_tile<R, CW>(g, wg, p.kc2)) {
+    if (MODE >= 4 && !vcut) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) {
+        const uint32_t o = zo.at(rt + T * m);
+        V[o] = mk<R>(0, 0);
+        (V + fstride)[o] = mk<R>(0, 0);
+        (V + 2 * fstride)[o] = mk<R>(0, 0);
+      }
+    }
+    return;
+  }
+  const bool ccut = col_cut<R>(t.kx, kwave(t.oth, g.ny), p.kc2);
+  const bool nin = !(ncut && ccut);   // the products of this column are read
+  // the new state of this column is not all zero (t.ok: always true, see k_zinv_vort)
+  const bool live = TR ? !(scut && ccut) : t.ok;
   cpx<R>* const W1 = W + fstride;
   cpx<R>* const W2 = W + 2 * fstride;
   // 1024-thread workgroups (and 1024-point lines) run one per CU, which
@@ -469,13 +721,17 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
   constexpr bool PARK = CC::BS >= 1024 || (N >= 1024 && sizeof(R) == 4);
   __shared__ cpx<R> park[PARK ? E * CC::BS : 1];
   cpx<R> nx_[E], ny_[E], nz_[E];
+  auto load = [&](cpx<R>(&v)[E], const cpx<R>* w, const ZOff<ZS>& zz) {
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const uint32_t o = zo.at(rt + T * m);
-    nx_[m] = ld_once<R, (CW >= 16)>(W + o);
-    ny_[m] = ld_once<R, (CW >= 16)>(W1 + o);
-    if constexpr (!PARK) nz_[m] = ld_once<R, (CW >= 16)>(W2 + o);
-  }
+    for (int m = 0; m < E; ++m) v[m] = mk<R>(0, 0);
+    if (nin) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) v[m] = ld_once<R, (CW >= 16)>(w + zz.at(rt + T * m));
+    }
+  };
+  load(nx_, W, zo);
+  load(ny_, W1, zo);
+  if constexpr (!PARK) load(nz_, W2, zo);
   using L = Line<R, N, E, -1>;
   L::run(nx_, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
   if constexpr (PARK) {
@@ -483,10 +739,8 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
     ZOff<ZS> zn = zo;
     asm volatile("" : "+v"(zn.ob));
 #pragma unroll
-    for (int m = 0; m < E; ++m) {
-      park[m * CC::BS + threadIdx.x] = nx_[m];
-      nz_[m] = ld_once<R, (CW >= 16)>(W2 + zn.at(rt + T * m));
-    }
+    for (int m = 0; m < E; ++m) park[m * CC::BS + threadIdx.x] = nx_[m];
+    load(nz_, W2, zn);
   }
   L::run(ny_, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
   // The stage update's loads (v, du or the AB2 history) of all three
@@ -498,12 +752,8 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
     const int z = L::out_pos(m, rt);
     const int iy = kwave(t.oth, g.ny), iz = kwave(z, g.nz);
     const int ik2 = t.kx * t.kx + iy * iy + iz * iz;
-    // MODE 4 reads du only inside the cut
-    const bool cut = (ik2 == 0 ? std::numeric_limits<R>::min() : (R)ik2) >= p.kc2;
-    const uint32_t o = zz.at(z);
-    dst[0] = stage_load<MODE, R, uint32_t, NT>(o, V, DU, S, cut);
-    dst[1] = stage_load<MODE, R, uint32_t, NT>(o, V + fstride, DU + fstride, S + fstride, cut);
-    dst[2] = stage_load<MODE, R, uint32_t, NT>(o, V + 2 * fstride, DU + 2 * fstride, S + 2 * fstride, cut);
+    const bool cut = (MODE == 4 || trunc) && (ik2 == 0 ? std::numeric_limits<R>::min() : (R)ik2) >= p.kc2;
+    stage_load3<MODE, NT, R>(dst, zz.at(z), fstride, V, DU, S, cut, vcut);
   };
   L::run(nz_, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
   // the epilogue recomputes its offsets (not kept live from the loads)
@@ -519,13 +769,11 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
     fa = (R)coef[0];
     fb = (R)coef[1];
   }
-  R ab_dt = 0, ab_dto = 0, ab_s = 0, ab_ek = 0, ab_del = 0;
+  R ab_dto = 0;
+  AbWeights<R> ab{};
   if constexpr (MODE >= 5) {
-    ab_dt = (R)p.ab[AB_DT];
     ab_dto = (R)p.ab[AB_DTO];
-    ab_s = (R)p.ab[AB_S];
-    ab_ek = (R)p.ab[AB_EK];
-    ab_del = (R)p.ab[AB_DELTA];
+    ab = {(R)p.ab[AB_DT], (R)p.ab[AB_S], (R)p.ab[AB_EK], (R)p.ab[AB_DELTA]};
   }
   // With the park, the new x stage state goes back to its park slot (just
   // read) until the z-inverse, which keeps 2E registers free here.
@@ -581,14 +829,15 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
       W2[o] = d;
     } else if constexpr (MODE >= 5) {
       const R xk = -p.nu * k2;
-      const R e1 = expm1_r(xk * ab_dt);
+      const R e1 = expm1_r(xk * ab.dt);
       const R e2 = MODE == 5 ? (R)0 : expm1_r(xk * ab_dto);
-      const bool cut = k2 >= p.kc2 || ik2 == 0;
-      keep_x(m, ab_apply<MODE, R>(in[0], a, o, V, DU, S, ab_dt, ab_s, ab_ek, ab_del, e1, e2, cut, p.nonfinite));
-      ny_[m] = ab_apply<MODE, R>(in[1], b, o, V + fstride, DU + fstride, S + fstride, ab_dt, ab_s, ab_ek, ab_del, e1,
-                                 e2, cut, p.nonfinite);
-      nz_[m] = ab_apply<MODE, R>(in[2], d, o, V + 2 * fstride, DU + 2 * fstride, S + 2 * fstride, ab_dt, ab_s, ab_ek,
-                                 ab_del, e1, e2, cut, p.nonfinite);
+      const bool cut = k2 >= p.kc2 || ik2 == 0, over = trunc && k2 >= p.kc2;
+      const cpx<R> n[3] = {a, b, d};
+      cpx<R> out[3];
+      ab_apply3<MODE, R>(in, n, out, o, fstride, V, DU, S, ab, e1, e2, cut, p.nonfinite, over, vcut);
+      keep_x(m, out[0]);
+      ny_[m] = out[1];
+      nz_[m] = out[2];
     } else {
       // E = exp(x), x = -nu k2 dt/2.  E is within 1e-3 of 1 for most modes,
       // where FP32 spacing (6e-8) makes a rounded E or E*E a biased factor
@@ -596,13 +845,14 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
       // to the rounding of the result.
       const R x = -p.nu * k2 * p.dt / (R)2;
       const R em1 = expm1_r(x);
-      const bool cut = k2 >= p.kc2;
+      const bool cut = (MODE == 4 || trunc) && k2 >= p.kc2;
       const bool store_s = !FUSED || (p.forced && k2 < p.fk2);
-      keep_x(m, stage_apply<MODE, R>(in[0], p.dt * a, o, V, DU, S, em1, x, cut, store_s, p.nonfinite));
-      ny_[m] = stage_apply<MODE, R>(in[1], p.dt * b, o, V + fstride, DU + fstride, S + fstride, em1, x, cut, store_s,
-                                    p.nonfinite);
-      nz_[m] = stage_apply<MODE, R>(in[2], p.dt * d, o, V + 2 * fstride, DU + 2 * fstride, S + 2 * fstride, em1, x,
-                                    cut, store_s, p.nonfinite);
+      const cpx<R> n[3] = {p.dt * a, p.dt * b, p.dt * d};
+      cpx<R> out[3];
+      stage_apply3<MODE, R>(in, n, out, o, fstride, V, DU, S, em1, x, cut, store_s, p.nonfinite, vcut);
+      keep_x(m, out[0]);
+      ny_[m] = out[1];
+      nz_[m] = out[2];
     }
   }
   if constexpr (FUSED && MODE > 0) {
@@ -610,7 +860,7 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
 #pragma unroll
       for (int m = 0; m < E; ++m) nx_[m] = park[m * CC::BS + threadIdx.x];
     }
-    zinv_store<R, N, E, CW, PARK, ZS>(nx_, ny_, nz_, lds, park, twl, rt, c, kx, ky, g.nz, zo, W, fstride);
+    zinv_store<R, N, E, CW, PARK, ZS>(nx_, ny_, nz_, lds, park, twl, rt, c, kx, ky, g.nz, zo, W, fstride, live);
   }
 }
 
@@ -872,29 +1122,33 @@ __device__ inline void row_c2r_prep(cpx<R> (&v)[8], const cpx<R> (&x)[8], cpx<R>
 
 // After the length-M forward FFT of packed reals (z: Z[rt + T*m]):
 // X[k] = (Zk + conj Z_{M-k})/2 - (i/2) exp(-2 pi i k/nx) (Zk - conj Z_{M-k}),
-// k = 0..M-1 to the main row, X[M] = Re Z0 - Im Z0 to nyq.
-template <class R, int M>
+// k = 0..M-1 to the main row, X[M] = Re Z0 - Im Z0 to nyq.  CUT: only the
+// entries k < kout (k = M: nyq) are stored.
+template <class R, int M, bool CUT = false>
 __device__ inline void row_r2c_post(const cpx<R> (&z)[8], cpx<R>* mainrow, cpx<R>* nyqp, int rt, const cpx<R>* tw,
-                                    int twsN) {
+                                    int twsN, int kout = M + 1) {
   constexpr int T = M / 8;
 #pragma unroll
   for (int m = 0; m < 8; ++m) {
     const int k = rt + T * m;
     const cpx<R> zk = z[m], zc = conj(row_partner<R, M>(z, m, rt));
     const cpx<R> s = zk + zc, d = zk - zc;
-    mainrow[k] = (R)0.5 * (s - mul_i(tw[k * twsN] * d));
+    const cpx<R> x = (R)0.5 * (s - mul_i(tw[k * twsN] * d));
+    if (!CUT || k < kout) mainrow[k] = x;
   }
-  if (rt == 0) *nyqp = mk<R>(z[0].x - z[0].y, (R)0);
+  if (rt == 0 && (!CUT || M < kout)) *nyqp = mk<R>(z[0].x - z[0].y, (R)0);
 }
 
 // XPASS: per row, c2r of 6 fields, u x w * scale, r2c of 3, in place into
 // fields 0..2.  Fields at W + f*fstride.  TAPE: u, w in physical space also
 // to tape (stride fstride, the layout k_row_c2r leaves: the adjoint's record
-// of the forward).
-template <class R, int M, bool TAPE = false>
+// of the forward).  CUT: entries k >= kin of the inputs are taken as zero (the
+// state is truncated) and entries k >= kout of the outputs not stored (only
+// the kept modes are used); k = M is the kx = nx/2 entry.
+template <class R, int M, bool TAPE = false, bool CUT = false>
 __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_convec(cpx<R>* W, int64_t fstride, Geom g, R scale,
                                                                  const cpx<R>* __restrict__ tw, int twsM, int twsN,
-                                                                 cpx<R>* __restrict__ tape) {
+                                                                 cpx<R>* __restrict__ tape, int kin, int kout) {
   using C = RowCfg<R, M>;
   constexpr int T = C::TPR;
   __shared__ cpx<R> lds[C::RPW * lds_pad(M)];
@@ -920,8 +1174,11 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_convec(cpx<R>* W, in
     for (int f = 0; f < 6; ++f) {
       const cpx<R>* base = W + f * fstride;
 #pragma unroll
-      for (int m = 0; m < 8; ++m) raw[f][m] = base[row * M + rt + T * m];
-      xm[f] = rt == 0 ? base[g.nmain + row] : mk<R>(0, 0);
+      for (int m = 0; m < 8; ++m) {
+        const int k = rt + T * m;
+        raw[f][m] = CUT ? ld_or_zero(base, row * M + k, row * M, k < kin) : base[row * M + k];
+      }
+      xm[f] = rt == 0 && (!CUT || M < kin) ? base[g.nmain + row] : mk<R>(0, 0);
     }
     cpx<R> a[6][8];
 #pragma unroll
@@ -948,7 +1205,7 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_convec(cpx<R>* W, in
     for (int f = 0; f < 3; ++f) {
       cpx<R>* base = W + f * fstride;
       LF::run(p[f], lrow, rt, twM, 1, LinIdx{});
-      row_r2c_post<R, M>(p[f], base + row * M, base + g.nmain + row, rt, twN, 1);
+      row_r2c_post<R, M, CUT>(p[f], base + row * M, base + g.nmain + row, rt, twN, 1, kout);
     }
   }
 }

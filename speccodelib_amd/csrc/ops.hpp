@@ -16,9 +16,12 @@ struct AdjLayout;
 template <class R>
 struct Ops {
   using C = cpx<R>;
-  static int32_t colfft(const scl_plan3d& pl, C* f0, int64_t fstride, int nf, int axis, int dir);
+  // kc2 > 0 (here and below, y- and x-passes): only the modes inside the
+  // truncation k^2 < kc2 are there (inverse) or wanted (forward); infinite:
+  // all of them, by the same kernels as with a truncation
+  static int32_t colfft(const scl_plan3d& pl, C* f0, int64_t fstride, int nf, int axis, int dir, R kc2 = 0);
   static int32_t zinv_vort(const scl_plan3d& pl, const C* s, int64_t sstride, C* w, int64_t wstride);
-  static int32_t yinv_vort(const scl_plan3d& pl, C* W, int64_t fstride);
+  static int32_t yinv_vort(const scl_plan3d& pl, C* W, int64_t fstride, R kc2 = 0);
   // fused (mode 1..4): also z-inverse the new stage state (mode 4: the new
   // v) into W[0..4] for the next RHS (k_zfwd_rhs FUSED)
   static int32_t zfwd_rhs(const scl_plan3d& pl, int mode, C* W, int64_t fstride, C* V, C* DU, C* S, const C* st,
@@ -49,7 +52,8 @@ struct Ops {
                             int type, double* coef);
   static int32_t herm_fix(const scl_plan3d& pl, const FieldPtrs<R>& fp);
   // tape (optional): u, w in physical space (k_row_convec TAPE)
-  static int32_t row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape = nullptr);
+  static int32_t row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape = nullptr, R kc2_in = 0,
+                            R kc2_out = 0);
   static int32_t row_c2r(const scl_plan3d& pl, C* W, int64_t fstride, int nf);
   static int32_t row_r2c(const scl_plan3d& pl, C* W, int64_t fstride, int nf);
   static int32_t ref_to_split(const scl_plan3d& pl, const C* ref, C* f);

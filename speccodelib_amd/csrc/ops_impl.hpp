@@ -74,8 +74,16 @@ static int32_t check_cols(const Geom& g) {
   return SCL_OK;
 }
 
+// The truncation of radius^2 kc2 (0: none) for the y- and x-passes.
 template <class R>
-int32_t Ops<R>::colfft(const scl_plan3d& pl, C* f0, int64_t fstride, int nf, int axis, int dir) {
+static Cut<R> cut_of(const Geom& g, R kc2) {
+  Cut<R> c{kc2 > 0 ? kc2 : std::numeric_limits<R>::infinity(), 0};
+  while (c.nkx <= g.mx && !col_cut<R>(c.nkx, 0, c.kc2)) ++c.nkx;
+  return c;
+}
+
+template <class R>
+int32_t Ops<R>::colfft(const scl_plan3d& pl, C* f0, int64_t fstride, int nf, int axis, int dir, R kc2) {
   const Geom& g = pl.g;
   const int n = axis == 1 ? g.ny : g.nz;
   return with_line<R>(n, [&](auto NC) -> int32_t {
@@ -85,14 +93,22 @@ int32_t Ops<R>::colfft(const scl_plan3d& pl, C* f0, int64_t fstride, int nf, int
     const dim3 blk(CC::BS);
     const cpx<R>* tw = twp<R>(pl);
     const int tws = pl.L / N;
-    if (axis == 1) {
+    auto go = [&](auto kern, dim3 grd, Cut<R> cut) {
+      hipLaunchKernelGGL(kern, grd, blk, 0, pl.stream, f0, fstride, g, tw, tws, cut);
+    };
+    const Cut<R> cut = cut_of<R>(g, kc2);
+    if (axis == 1 && kc2 > 0) {
+      const dim3 grd(ycut_grid<CC::CW>(g, cut.nkx), nf);
+      if (dir < 0) go(k_colfft<R, N, 1, -1, true>, grd, cut);
+      else go(k_colfft<R, N, 1, 1, true>, grd, cut);
+    } else if (axis == 1) {
       const dim3 grd(col_grid<CC::CW, 1>(g), nf);
-      if (dir < 0) hipLaunchKernelGGL((k_colfft<R, N, 1, -1>), grd, blk, 0, pl.stream, f0, fstride, g, tw, tws);
-      else hipLaunchKernelGGL((k_colfft<R, N, 1, 1>), grd, blk, 0, pl.stream, f0, fstride, g, tw, tws);
+      if (dir < 0) go(k_colfft<R, N, 1, -1>, grd, cut);
+      else go(k_colfft<R, N, 1, 1>, grd, cut);
     } else {
       const dim3 grd(col_grid<CC::CW, 2>(g), nf);
-      if (dir < 0) hipLaunchKernelGGL((k_colfft<R, N, 2, -1>), grd, blk, 0, pl.stream, f0, fstride, g, tw, tws);
-      else hipLaunchKernelGGL((k_colfft<R, N, 2, 1>), grd, blk, 0, pl.stream, f0, fstride, g, tw, tws);
+      if (dir < 0) go(k_colfft<R, N, 2, -1>, grd, cut);
+      else go(k_colfft<R, N, 2, 1>, grd, cut);
     }
     return check_launch("colfft");
   });
@@ -103,16 +119,21 @@ int32_t Ops<R>::colfft(const scl_plan3d& pl, C* f0, int64_t fstride, int nf, int
 // kernel (one field live, twice the waves per CU; measured 1193 vs 1237 us
 // per RHS at 512^3 for one kernel doing all six).
 template <class R>
-int32_t Ops<R>::yinv_vort(const scl_plan3d& pl, C* W, int64_t fstride) {
+int32_t Ops<R>::yinv_vort(const scl_plan3d& pl, C* W, int64_t fstride, R kc2) {
   const Geom& g = pl.g;
   return with_line<R>(g.ny, [&](auto NC) -> int32_t {
     constexpr int N = decltype(NC)::value;
     using CC = ColCfg<R, N>;
     SCL_CHECK((check_cols<R, N>(g)));
-    hipLaunchKernelGGL((k_yinv_vort<R, N>), dim3(col_grid<CC::CW, 1>(g)), dim3(CC::BS), 0, pl.stream, W, fstride, g,
-                       twp<R>(pl), pl.L / N);
+    const Cut<R> cut = cut_of<R>(g, kc2);
+    if (kc2 > 0)
+      hipLaunchKernelGGL((k_yinv_vort<R, N, true>), dim3(ycut_grid<CC::CW>(g, cut.nkx)), dim3(CC::BS), 0, pl.stream, W,
+                         fstride, g, twp<R>(pl), pl.L / N, cut);
+    else
+      hipLaunchKernelGGL((k_yinv_vort<R, N>), dim3(col_grid<CC::CW, 1>(g)), dim3(CC::BS), 0, pl.stream, W, fstride, g,
+                         twp<R>(pl), pl.L / N, cut);
     SCL_CHECK(check_launch("yinv_vort"));
-    return colfft(pl, W + 2 * fstride, fstride, 3, 1, 1);
+    return colfft(pl, W + 2 * fstride, fstride, 3, 1, 1, kc2);
   });
 }
 
@@ -195,8 +216,15 @@ int32_t Ops<R>::zfwd_rhs(const scl_plan3d& pl, int mode, C* W, int64_t fstride, 
       auto launch = [&](auto MC, auto FC, auto ZC) {
         constexpr int MODE = decltype(MC)::value, ZS = decltype(ZC)::value;
         constexpr bool FUSED = decltype(FC)::value != 0;
-        hipLaunchKernelGGL((k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS>), grd, blk, 0, pl.stream, W, fstride, V, DU, S, st,
-                           coef, p, g, tw, tws);
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, grd, blk, 0, pl.stream, W, fstride, V, DU, S, st, coef, p, g, tw, tws);
+        };
+        // short lines come in both variants: their grids can be so small
+        // that the instructions of the unused one are felt (Cut)
+        if constexpr (N <= 64) {
+          if (!p.trunc) return go(k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS, false>);
+        }
+        go(k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS>);
       };
       auto by_zs = [&](auto MC, auto FC) {
         if (g.zs == 3) launch(MC, FC, IC<3>{});
@@ -367,8 +395,9 @@ int32_t Ops<R>::herm_fix(const scl_plan3d& pl, const FieldPtrs<R>& fp) {
 }
 
 template <class R>
-int32_t Ops<R>::row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape) {
+int32_t Ops<R>::row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape, R kc2_in, R kc2_out) {
   const Geom& g = pl.g;
+  const int kin = cut_of<R>(g, kc2_in).nkx, kout = cut_of<R>(g, kc2_out).nkx;
   const R scale = (R)1 / (R)((double)g.nx * g.ny * g.nz);
   return with_half<R>(g.mx, [&](auto MC) -> int32_t {
     constexpr int M = decltype(MC)::value;
@@ -387,11 +416,12 @@ int32_t Ops<R>::row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape)
       const int64_t groups = g.nrow / RC::RPW;
       const int64_t grid = std::min<int64_t>(groups, (int64_t)resident * pl.ncu);
       hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(RC::BS), 0, pl.stream, W, fstride, g, scale, twp<R>(pl),
-                         pl.L / M, pl.L / g.nx, tape);
+                         pl.L / M, pl.L / g.nx, tape, kin, kout);
       return check_launch("row_convec");
     };
-    if (tape) return go(IC<1>{}, k_row_convec<R, M, true>);
-    return go(IC<0>{}, k_row_convec<R, M, false>);
+    const bool cut = kc2_in > 0 || kc2_out > 0;
+    if (tape) return cut ? go(IC<3>{}, k_row_convec<R, M, true, true>) : go(IC<1>{}, k_row_convec<R, M, true>);
+    return cut ? go(IC<2>{}, k_row_convec<R, M, false, true>) : go(IC<0>{}, k_row_convec<R, M, false>);
   });
 }
 
