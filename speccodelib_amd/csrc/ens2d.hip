@@ -3,7 +3,9 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <limits>
+#include <mutex>
 #include <vector>
 
 #include "ic.hpp"
@@ -127,6 +129,8 @@ struct scl_ens2d {
   // size group (SCL_ENS2D_FORK=1), whose concurrent groups slow each other.
   bool fork_groups = false;
   double* diag = nullptr;
+  void* pin = nullptr;  // pinned host memory of the member copies
+  std::mutex pin_use;
   int ncu = 256;
   int64_t steps = 0;
   double time = 0.0;
@@ -380,28 +384,57 @@ int32_t locate(const scl_ens2d& e, int ug, int j, const Group** gr, int* b) {
   return SCL_OK;
 }
 
-// Host reference layout (lx1, ly) <-> split layout of member b, field f.
-int32_t copy_member(const scl_ens2d& e, const Group& gr, int b, int f, void* host, bool to_device) {
-  const size_t es = e.esize();
-  const int n = gr.n, mx = n / 2, lx1 = mx + 1;
-  char* dbase = reinterpret_cast<char*>(gr.base) + (size_t)f * gr.fs() * es;
-  char* dmain = dbase + (size_t)b * n * mx * es;
-  char* dnyq = dbase + ((size_t)gr.g.nmain + (size_t)b * n) * es;
-  char* h = reinterpret_cast<char*>(host);
-  if (to_device) {
-    SCL_HIP(hipMemcpy2DAsync(dmain, mx * es, h, lx1 * es, mx * es, n, hipMemcpyHostToDevice, e.stream));
-    SCL_HIP(hipMemcpy2DAsync(dnyq, es, h + mx * es, lx1 * es, es, n, hipMemcpyHostToDevice, e.stream));
-  } else {
-    SCL_HIP(hipMemcpy2DAsync(h, lx1 * es, dmain, mx * es, mx * es, n, hipMemcpyDeviceToHost, e.stream));
-    SCL_HIP(hipMemcpy2DAsync(h + mx * es, lx1 * es, dnyq, es, es, n, hipMemcpyDeviceToHost, e.stream));
+// Pinned host memory for one member of the largest size, made on the first
+// copy and kept with the ensemble; the caller holds e.pin_use.
+template <class R>
+int32_t pinned(scl_ens2d& e, cpx<R>** out) {
+  if (!e.pin) {
+    const size_t n = *std::max_element(e.sizes.begin(), e.sizes.end());
+    if (hipHostMalloc(&e.pin, (n / 2 + 1) * n * e.esize(), 0) != hipSuccess) {
+      (void)hipGetLastError();
+      e.pin = nullptr;
+      return set_error("pinned host allocation failed"), SCL_ENOMEM;
+    }
   }
-  SCL_HIP(hipStreamSynchronize(e.stream));
+  *out = static_cast<cpx<R>*>(e.pin);
   return SCL_OK;
 }
 
-// turb_2d.f90's wz(my, mx2) (C = 2 conj(D), see Turb2DP) <-> the host
-// reference layout (lx1, ly) of the normalised coefficients D.  On the way
-// in, symmetrize (turb_2d.f90:569-590): row ky = -n/2 and k = 0 zeroed, the
+// Host reference layout (lx1, ly) <-> split layout of member b, field f; with
+// turb (to the host only) turb_2d.f90's wz(my, mx2).  One kernel changes the
+// layout between the device field and pinned memory, and the CPU copies that
+// to or from the caller's array.  With a copy per row into pageable memory,
+// 100 steps of 256 members (192 of 256^2, 48 of 512^2, 16 of 1024^2) and their
+// read-back took 1489 ms, 190 of them the steps; this way 240 ms (turb_2d,
+// 7 of 128^2 and 3 of 512^2, 200 steps: 59 to 24 ms).
+template <class R>
+int32_t copy_member(scl_ens2d& e, const Group& gr, int b, int f, void* host, bool to_device, bool turb = false) {
+  using C = cpx<R>;
+  const std::lock_guard<std::mutex> hold(e.pin_use);
+  C* pin = nullptr;
+  SCL_CHECK(pinned<R>(e, &pin));
+  C* const fld = gr.field<R>(f);
+  const int n = gr.n, mx = n / 2;
+  const size_t entries = (size_t)(turb ? mx : mx + 1) * n;
+  const dim3 grd((unsigned)((entries + 255) / 256));
+  if (to_device) {
+    std::memcpy(pin, host, entries * sizeof(C));
+    hipLaunchKernelGGL((k_member_in<R>), grd, dim3(256), 0, e.stream, (const C*)pin, gr.g, b, fld);
+  } else if (turb) {
+    hipLaunchKernelGGL((k_member_out_turb<R>), dim3(mx / 16, (n + 63) / 64), dim3(256), 0, e.stream, (const C*)fld,
+                       gr.g, b, pin);
+  } else {
+    hipLaunchKernelGGL((k_member_out<R>), grd, dim3(256), 0, e.stream, (const C*)fld, gr.g, b, pin);
+  }
+  SCL_CHECK(check_launch("copy_member"));
+  SCL_HIP(hipStreamSynchronize(e.stream));
+  if (!to_device) std::memcpy(host, pin, entries * sizeof(C));
+  return SCL_OK;
+}
+
+// turb_2d.f90's wz(my, mx2) (C = 2 conj(D), see Turb2DP) -> the host
+// reference layout (lx1, ly) of the normalised coefficients D, with
+// symmetrize (turb_2d.f90:569-590): row ky = -n/2 and k = 0 zeroed, the
 // kx = 0 column averaged with its mirror for 1 <= y <= n/2 - 2.
 template <class R>
 void turb_in(const cpx<R>* wz, int n, std::vector<cpx<R>>& h) {
@@ -416,37 +449,25 @@ void turb_in(const cpx<R>* wz, int n, std::vector<cpx<R>>& h) {
   for (int y = 1; y <= n / 2 - 2; ++y) h[(size_t)(n - y) * lx1] = conj(h[(size_t)y * lx1]);
 }
 
-template <class R>
-void turb_out(const std::vector<cpx<R>>& h, int n, cpx<R>* wz) {
-  const int mx2 = n / 2, lx1 = mx2 + 1;
-  for (int x = 0; x < mx2; ++x)
-    for (int y = 0; y < n; ++y) wz[(size_t)x * n + y] = (R)2 * conj(h[(size_t)y * lx1 + x]);
-}
-
 template <class F>
 int32_t with_prec(int prec, F&& f) {
   return prec == SCL_SP ? f(float{}) : f(double{});
 }
 
 // Member copies in the layout of the ensemble's scheme.
-int32_t put_member(const scl_ens2d& e, const Group& gr, int b, int f, const void* w) {
-  if (e.p.scheme != 1) return copy_member(e, gr, b, f, const_cast<void*>(w), true);
+int32_t put_member(scl_ens2d& e, const Group& gr, int b, int f, const void* w) {
   return with_prec(e.prec, [&](auto zero) -> int32_t {
     using R = decltype(zero);
+    if (e.p.scheme != 1) return copy_member<R>(e, gr, b, f, const_cast<void*>(w), true);
     std::vector<cpx<R>> h;
     turb_in<R>(static_cast<const cpx<R>*>(w), gr.n, h);
-    return copy_member(e, gr, b, f, h.data(), true);
+    return copy_member<R>(e, gr, b, f, h.data(), true);
   });
 }
 
-int32_t take_member(const scl_ens2d& e, const Group& gr, int b, int f, void* w) {
-  if (e.p.scheme != 1) return copy_member(e, gr, b, f, w, false);
+int32_t take_member(scl_ens2d& e, const Group& gr, int b, int f, void* w) {
   return with_prec(e.prec, [&](auto zero) -> int32_t {
-    using R = decltype(zero);
-    std::vector<cpx<R>> h((size_t)(gr.n / 2 + 1) * gr.n);
-    SCL_CHECK(copy_member(e, gr, b, f, h.data(), false));
-    turb_out<R>(h, gr.n, static_cast<cpx<R>*>(w));
-    return SCL_OK;
+    return copy_member<decltype(zero)>(e, gr, b, f, w, false, e.p.scheme == 1);
   });
 }
 
@@ -496,10 +517,10 @@ void initialize2d(std::vector<double>& w, int n, int32_t seed, double k0, double
 }
 
 template <class R>
-int32_t upload_member_f64(const scl_ens2d& e, const Group& gr, int b, const std::vector<double>& w) {
+int32_t upload_member_f64(scl_ens2d& e, const Group& gr, int b, const std::vector<double>& w) {
   std::vector<R> h(w.size());
   for (size_t i = 0; i < w.size(); ++i) h[i] = (R)w[i];
-  return copy_member(e, gr, b, F_WS, h.data(), true);
+  return copy_member<R>(e, gr, b, F_WS, h.data(), true);
 }
 
 void destroy_groups(scl_ens2d& e) {
@@ -630,6 +651,7 @@ extern "C" int32_t scl_ens2d_destroy(scl_ens2d* e) {
   drop_graph(*e);
   destroy_groups(*e);
   if (e->diag) (void)hipFree(e->diag);
+  if (e->pin) (void)hipHostFree(e->pin);
   if (e->fork) (void)hipEventDestroy(e->fork);
   if (e->t0) (void)hipEventDestroy(e->t0);
   if (e->t1) (void)hipEventDestroy(e->t1);
@@ -689,7 +711,7 @@ extern "C" int32_t scl_ens2d_rhs(scl_ens2d* e, int32_t group, int32_t member, co
     return take_member(*e, *gr, b, F_NA, rhs);
   }
   SCL_CHECK(e->prec == SCL_SP ? stage<float>(*e, *gr, 0, e->stream) : stage<double>(*e, *gr, 0, e->stream));
-  return copy_member(*e, *gr, b, F_W, rhs, false);
+  return take_member(*e, *gr, b, F_W, rhs);
 }
 
 extern "C" int32_t scl_ens2d_step(scl_ens2d* e, int32_t nsteps) {

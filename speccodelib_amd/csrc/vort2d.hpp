@@ -488,6 +488,55 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
   }
 }
 
+// Member b of a batch (field f) -> the host layout (lx1, ly) of the copies,
+// in one contiguous block.  out is pinned host memory: the stores go over the
+// host link as they are made, whole rows at a time, and no row is a copy of
+// its own.
+template <class R>
+__global__ __launch_bounds__(256) void k_member_out(const cpx<R>* __restrict__ f, Geom g, int b,
+                                                    cpx<R>* __restrict__ out) {
+  const int n = g.ny, lx1 = g.mx + 1;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n * lx1) return;
+  const int y = i / lx1, x = i % lx1;
+  const int64_t row = (int64_t)b * n + y;
+  out[i] = x < g.mx ? f[row * g.mx + x] : f[g.nmain + row];
+}
+
+// The same the other way.
+template <class R>
+__global__ __launch_bounds__(256) void k_member_in(const cpx<R>* __restrict__ in, Geom g, int b,
+                                                   cpx<R>* __restrict__ f) {
+  const int n = g.ny, lx1 = g.mx + 1;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n * lx1) return;
+  const int y = i / lx1, x = i % lx1;
+  const int64_t row = (int64_t)b * n + y;
+  f[x < g.mx ? row * g.mx + x : g.nmain + row] = in[i];
+}
+
+// Member b -> turb_2d.f90's wz(my, mx2) (C = 2 conj(D), the kx = n/2 column
+// left out): a transpose, in tiles of 16 x by 64 y through LDS so that loads
+// run along x and the stores to host memory along y.  The padding entry of a
+// tile row keeps its columns off one another's banks.
+template <class R>
+__global__ __launch_bounds__(256) void k_member_out_turb(const cpx<R>* __restrict__ f, Geom g, int b,
+                                                         cpx<R>* __restrict__ out) {
+  constexpr int TX = 16, TY = 64;
+  __shared__ cpx<R> tile[TX][TY + 1];
+  const int n = g.ny;
+  const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY;
+  for (int i = threadIdx.x; i < TX * TY; i += 256) {
+    const int x = i % TX, y = i / TX;
+    if (y0 + y < n) tile[x][y] = f[((int64_t)b * n + y0 + y) * g.mx + x0 + x];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < TX * TY; i += 256) {
+    const int y = i % TY, x = i / TY;
+    if (y0 + y < n) out[(int64_t)(x0 + x) * n + y0 + y] = (R)2 * conj(tile[x][y]);
+  }
+}
+
 // Per-member FP64 sums in a fixed order: out[2b] = sum' |w|^2/k^2 (twice the
 // kinetic energy's half-plane sum, as spectral_dns_2d.f90:125-128 with
 // kx = 0 halved), out[2b+1] = sum' |w|^2.  One workgroup per member.
