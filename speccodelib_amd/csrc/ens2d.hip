@@ -134,6 +134,7 @@ struct scl_ens2d {
   int ncu = 256;
   int64_t steps = 0;
   double time = 0.0;
+  bool truncated = false;  // scheme 0: every member's state is zero beyond the 2/3 cut
   int total_members() const {
     int t = 0;
     for (int m : members) t += m;
@@ -145,8 +146,9 @@ struct scl_ens2d {
 namespace {
 
 template <class R>
-Rhs2D<R> rhs_params(const scl_ens2d& e, int n) {
+Rhs2D<R> rhs_params(const scl_ens2d& e, int n, bool trunc) {
   Rhs2D<R> r;
+  r.trunc = trunc;
   r.dt = (R)e.p.dt;
   r.fk2min = (R)(e.p.fkmin * e.p.fkmin);
   r.fk2max = (R)(e.p.fkmax * e.p.fkmax);
@@ -160,6 +162,14 @@ Rhs2D<R> rhs_params(const scl_ens2d& e, int n) {
   r.rate.n_hyper = e.p.n_hyper;
   r.rate.n_hypo = e.p.n_hypo;
   return r;
+}
+
+// What a pass keeps: the modes inside the 2/3 cut, or all of them.
+template <class R>
+Cut<R> cut2d(const scl_ens2d& e, const Group& gr, bool trunc) {
+  Cut<R> c{trunc ? rhs_params<R>(e, gr.n, true).kc2 : std::numeric_limits<R>::infinity(), 0};
+  while (c.nkx <= gr.g.mx && !col_cut<R>(c.nkx, 0, c.kc2)) ++c.nkx;
+  return c;
 }
 
 // Workgroups of the x-pass: persistent (as many as can be resident) or one
@@ -180,24 +190,24 @@ int64_t row_grid_size(const scl_ens2d& e, const Group& gr) {
 }
 
 template <class R>
-int32_t yinv_launch(const Group& gr, const cpx<R>* src, int shift, hipStream_t st) {
+int32_t yinv_launch(const Group& gr, const cpx<R>* src, int shift, hipStream_t st, Cut<R> cut) {
   const cpx<R>* tw = reinterpret_cast<const cpx<R>*>(gr.tw);
   return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
     constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
-    hipLaunchKernelGGL((k_yinv2d<R, N, E, CW>), dim3(col_grid<CW, 1>(gr.g)), dim3(Col2D<R, N, E, CW>::BS), 0, st,
-                       src, gr.field<R>(F_W), gr.fs(), gr.g, tw, 1, shift);
+    hipLaunchKernelGGL((k_yinv2d<R, N, E, CW>), dim3(ycut_grid<CW>(gr.g, cut.nkx)), dim3(Col2D<R, N, E, CW>::BS), 0,
+                       st, src, gr.field<R>(F_W), gr.fs(), gr.g, tw, 1, shift, cut);
     return check_launch("yinv2d");
   });
 }
 
 template <class R>
-int32_t row_launch(const scl_ens2d& e, const Group& gr, hipStream_t st) {
+int32_t row_launch(const scl_ens2d& e, const Group& gr, hipStream_t st, Cut<R> cut) {
   const cpx<R>* tw = reinterpret_cast<const cpx<R>*>(gr.tw);
   return with_row2d<R>(gr.n / 2, [&](auto MC) -> int32_t {
     constexpr int M = decltype(MC)::value;
     const R scale = (R)1 / (R)((double)gr.n * gr.n);
     hipLaunchKernelGGL((k_row_adv2d<R, M>), dim3((unsigned)row_grid_size<R, M>(e, gr)), dim3(RowCfg<R, M>::BS), 0,
-                       st, gr.field<R>(F_W), gr.fs(), gr.g, scale, tw, 2, 1);
+                       st, gr.field<R>(F_W), gr.fs(), gr.g, scale, tw, 2, 1, cut.nkx);
     return check_launch("row_adv2d");
   });
 }
@@ -205,9 +215,11 @@ int32_t row_launch(const scl_ens2d& e, const Group& gr, hipStream_t st) {
 // One RHS evaluation (mode 0) or IF-RK4 stage (modes 1..4) of a group.
 // primed: W[0..2] already hold the y-inverse of the stage vorticity (the
 // previous stage was fused); fuse: the y-forward also y-inverses the new
-// stage vorticity into W[0..2] (k_yfwd2d FUSED), for the next stage.
+// stage vorticity into W[0..2] (k_yfwd2d FUSED), for the next stage.  trunc:
+// the step's state is zero beyond the 2/3 cut, which its passes leave out.
 template <class R>
-int32_t stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st, bool primed = false, bool fuse = false) {
+int32_t stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st, bool primed = false, bool fuse = false,
+              bool trunc = false) {
   using C = cpx<R>;
   C* W = gr.field<R>(F_W);
   C* WS = gr.field<R>(F_WS);
@@ -216,18 +228,20 @@ int32_t stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st, boo
   const C* sin = mode <= 1 ? WS : S;
   const C* tw = reinterpret_cast<const C*>(gr.tw);
   const int64_t fs = gr.fs();
-  const Rhs2D<R> rp = rhs_params<R>(e, gr.n);
+  const Rhs2D<R> rp = rhs_params<R>(e, gr.n, trunc);
+  const Cut<R> cut = cut2d<R>(e, gr, trunc);
   if (fuse && mode < 1) return set_error("fused 2D stage: mode %d is not a stage 1..4", mode), SCL_EINVAL;
-  if (!primed) SCL_CHECK(yinv_launch<R>(gr, sin, 0, st));
-  SCL_CHECK(row_launch<R>(e, gr, st));
+  if (!primed) SCL_CHECK(yinv_launch<R>(gr, sin, 0, st, cut));
+  SCL_CHECK(row_launch<R>(e, gr, st, cut));
   return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
     constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
-    const dim3 grd(col_grid<CW, 1>(gr.g)), blk(Col2D<R, N, E, CW>::BS);
+    const dim3 grd(ycut_grid<CW>(gr.g, cut.nkx)), blk(Col2D<R, N, E, CW>::BS);
     if (fuse)
-      hipLaunchKernelGGL((k_yfwd2d<R, N, E, CW, true>), grd, blk, 0, st, W, fs, WS, ACC, S, sin, mode, rp, gr.g, tw, 1);
+      hipLaunchKernelGGL((k_yfwd2d<R, N, E, CW, true>), grd, blk, 0, st, W, fs, WS, ACC, S, sin, mode, rp, gr.g, tw, 1,
+                         cut.nkx);
     else
       hipLaunchKernelGGL((k_yfwd2d<R, N, E, CW, false>), grd, blk, 0, st, W, fs, WS, ACC, S, sin, mode, rp, gr.g, tw,
-                         1);
+                         1, cut.nkx);
     return check_launch("yfwd2d");
   });
 }
@@ -256,8 +270,9 @@ int32_t turb_stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st
   const C* tw = reinterpret_cast<const C*>(gr.tw);
   const Turb2DP<R> tp = turb_params<R>(e, gr.n);
   for (int half = 0; half < 2; ++half) {
-    SCL_CHECK(yinv_launch<R>(gr, gr.field<R>(F_WS), half, st));
-    SCL_CHECK(row_launch<R>(e, gr, st));
+    const Cut<R> all = cut2d<R>(e, gr, false);
+    SCL_CHECK(yinv_launch<R>(gr, gr.field<R>(F_WS), half, st, all));
+    SCL_CHECK(row_launch<R>(e, gr, st, all));
     SCL_CHECK(with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
       constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
       hipLaunchKernelGGL((k_yfwd2d_turb<R, N, E, CW>), dim3(col_grid<CW, 1>(gr.g)), dim3(Col2D<R, N, E, CW>::BS), 0,
@@ -275,16 +290,19 @@ int turb_mode(int64_t step) { return step == 0 ? TURB_STEP0 : step == 1 ? TURB_S
 // y-inverse, every later one gets it from the previous stage's fused
 // y-forward, and the last stage is not fused (the chain leaves no state in
 // W).  The kx = 0 column is made Hermitian in the same workgroup, so the
-// chain gives the same results as separate stages.
+// chain gives the same results as separate stages.  Scheme 0's passes leave
+// out what lies beyond the 2/3 cut, where the state is zero from the end of
+// its first step on (the caller says with trunc whether it is); the first
+// step takes the state as it was set.
 template <class R>
-int32_t group_steps(const scl_ens2d& e, const Group& gr, hipStream_t st, int nsteps, int64_t first) {
+int32_t group_steps(const scl_ens2d& e, const Group& gr, hipStream_t st, int nsteps, int64_t first, bool trunc) {
   if (e.p.scheme == 1) {
     for (int s = 0; s < nsteps; ++s) SCL_CHECK(turb_stage<R>(e, gr, turb_mode(first + s), st));
     return SCL_OK;
   }
   for (int s = 0; s < nsteps; ++s)
     for (int mode = 1; mode <= 4; ++mode)
-      SCL_CHECK(stage<R>(e, gr, mode, st, s > 0 || mode > 1, s < nsteps - 1 || mode < 4));
+      SCL_CHECK(stage<R>(e, gr, mode, st, s > 0 || mode > 1, s < nsteps - 1 || mode < 4, trunc || s > 0));
   return SCL_OK;
 }
 
@@ -294,14 +312,15 @@ int32_t group_steps(const scl_ens2d& e, const Group& gr, hipStream_t st, int nst
 // through events, which graph capture turns into graph edges) and the
 // branches join once, at the end.
 // first: the index of the first step (scheme 1 bootstraps on steps 0, 1).
-int32_t launch_steps(scl_ens2d& e, int nsteps, int64_t first) {
+// trunc: as group_steps.
+int32_t launch_steps(scl_ens2d& e, int nsteps, int64_t first, bool trunc) {
   const bool fork = e.fork_groups && !e.p.per_member && e.groups.size() > 1;
   if (fork) SCL_HIP(hipEventRecord(e.fork, e.stream));
   for (auto& gr : e.groups) {
     hipStream_t st = fork ? gr.stream : e.stream;
     if (fork) SCL_HIP(hipStreamWaitEvent(st, e.fork, 0));
-    SCL_CHECK(e.prec == SCL_SP ? group_steps<float>(e, gr, st, nsteps, first)
-                               : group_steps<double>(e, gr, st, nsteps, first));
+    SCL_CHECK(e.prec == SCL_SP ? group_steps<float>(e, gr, st, nsteps, first, trunc)
+                               : group_steps<double>(e, gr, st, nsteps, first, trunc));
     if (fork) {
       SCL_HIP(hipEventRecord(gr.done, st));
       SCL_HIP(hipStreamWaitEvent(e.stream, gr.done, 0));
@@ -320,11 +339,12 @@ void drop_graph(scl_ens2d& e) {
 }
 
 // Graph i of e (0: one step, 1: a chunk of e.chunk steps), built on first
-// use; scheme 1 graphs hold IF-AB2 steps only.
+// use; scheme 0 graphs hold steps of truncated states, scheme 1 graphs IF-AB2
+// steps only.
 int32_t graph_exec(scl_ens2d& e, int i, hipGraphExec_t* out) {
   if (!e.exec[i]) {
     SCL_HIP(hipStreamBeginCapture(e.stream, hipStreamCaptureModeThreadLocal));
-    const int32_t st = launch_steps(e, i ? e.chunk : 1, 2);
+    const int32_t st = launch_steps(e, i ? e.chunk : 1, 2, true);
     hipGraph_t g = nullptr;
     const hipError_t ce = hipStreamEndCapture(e.stream, &g);
     if (st != SCL_OK) {
@@ -348,8 +368,16 @@ int32_t run_steps(scl_ens2d& e, int nsteps) {
   if (nsteps < 0) return set_error("nsteps < 0"), SCL_EINVAL;
   // scheme 1: the two bootstrap steps run eagerly
   for (; nsteps > 0 && e.p.scheme == 1 && e.steps < 2; --nsteps) {
-    SCL_CHECK(launch_steps(e, 1, e.steps));
+    SCL_CHECK(launch_steps(e, 1, e.steps, true));
     advance_clock(e, 1);
+  }
+  // scheme 0: so does the first step of a state that was set, and it leaves
+  // every member's state truncated
+  if (nsteps > 0 && e.p.scheme == 0 && !e.truncated) {
+    SCL_CHECK(launch_steps(e, 1, e.steps, false));
+    advance_clock(e, 1);
+    e.truncated = true;
+    --nsteps;
   }
   int done = 0;
   if (e.p.use_graph) {
@@ -363,7 +391,7 @@ int32_t run_steps(scl_ens2d& e, int nsteps) {
       for (; done < nsteps; ++done) SCL_HIP(hipGraphLaunch(x, e.stream));
     }
   } else {
-    SCL_CHECK(launch_steps(e, nsteps, e.steps));
+    SCL_CHECK(launch_steps(e, nsteps, e.steps, true));
     done = nsteps;
   }
   advance_clock(e, done);
@@ -665,6 +693,7 @@ extern "C" int32_t scl_ens2d_set_member(scl_ens2d* e, int32_t group, int32_t mem
   const Group* gr;
   int b;
   SCL_CHECK(locate(*e, group, member, &gr, &b));
+  e->truncated = false;
   SCL_CHECK(put_member(*e, *gr, b, F_WS, w));
   // scheme 1: a new state starts turb_2d.f90's bootstrap again (its restart
   // reads wz and runs istep = 0, 1 first)
@@ -683,6 +712,7 @@ extern "C" int32_t scl_ens2d_get_member(scl_ens2d* e, int32_t group, int32_t mem
 extern "C" int32_t scl_ens2d_initialize(scl_ens2d* e, int32_t seed0, double k0, double energy) {
   if (!e) return set_error("null argument"), SCL_EINVAL;
   if (!(k0 > 0) || !(energy > 0)) return set_error("k0 and energy must be > 0"), SCL_EINVAL;
+  e->truncated = false;
   std::vector<double> w;
   int q = 0;
   for (int ug = 0; ug < (int)e->sizes.size(); ++ug)
@@ -703,6 +733,7 @@ extern "C" int32_t scl_ens2d_rhs(scl_ens2d* e, int32_t group, int32_t member, co
   const Group* gr;
   int b;
   SCL_CHECK(locate(*e, group, member, &gr, &b));
+  e->truncated = false;
   SCL_CHECK(put_member(*e, *gr, b, F_WS, w));
   if (e->p.scheme == 1) {
     e->steps = 0;
@@ -842,8 +873,8 @@ extern "C" int32_t scl_ens2d_tune(scl_ens2d* e, int32_t reps, double* best_ms) {
           for (int c = 0; c < ng && st == SCL_OK; ++c) {
             const Group& gr = e->groups[e->first[ug] + c];
             auto steps = [&](int k) -> int32_t {
-              return e->prec == SCL_SP ? group_steps<float>(*e, gr, e->stream, k, first)
-                                       : group_steps<double>(*e, gr, e->stream, k, first);
+              return e->prec == SCL_SP ? group_steps<float>(*e, gr, e->stream, k, first, e->truncated)
+                                       : group_steps<double>(*e, gr, e->stream, k, first, e->truncated);
             };
             float t = 0;
             auto timed = [&]() -> int32_t {

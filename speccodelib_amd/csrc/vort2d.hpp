@@ -72,6 +72,10 @@ struct Rhs2D {
   R eps;             // forcing amplitude
   R kc2;             // 2/3 cut: zero where k^2 >= kc2
   int forced;
+  // w and the stage vorticity are zero beyond the cut (the right-hand side is
+  // cut, so all of a step is once its initial state is): nothing out there is
+  // read, transformed or written
+  int trunc;
   Rate2D<R> rate;
 };
 
@@ -127,21 +131,26 @@ __device__ inline cpx<R> half_cell_phase(int s, int n) {
 // fstride.  shift: the fields are taken at points moved by half a cell along
 // x and y, the spectrum times exp(-i pi (kx + ky)/N) (the phase shift of
 // turb_2d.f90:369-371, in the normalised coefficients of the real field).
+// cut: modes beyond it are taken as zero, and only its nkx columns stored.
 template <class R, int N, int E, int CW>
 __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yinv2d(const cpx<R>* __restrict__ s,
                                                                    cpx<R>* __restrict__ w, int64_t fstride, Geom g,
                                                                    const cpx<R>* __restrict__ tw, int tws,
-                                                                   int shift) {
+                                                                   int shift, Cut<R> cut) {
   using CC = Col2D<R, N, E, CW>;
   constexpr int T = CC::T;
   __shared__ cpx<R> lds[lds_pad(N) * CW];
   __shared__ cpx<R> twl[N];  // first read after a barrier inside the transform
   for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
   const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
-  const Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, gridDim.x), c);
+  Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, gridDim.x), c, ycut_tiles<CW>(g, cut.nkx));
+  if (t.kx >= cut.nkx) t.ok = false;
   cpx<R> o[E];
 #pragma unroll
-  for (int m = 0; m < E; ++m) o[m] = t.ok ? s[t.base + (int64_t)(rt + T * m) * t.rs] : mk<R>(0, 0);
+  for (int m = 0; m < E; ++m) {
+    const int j = rt + T * m;
+    o[m] = ld_or_zero(s, t.base + (int64_t)j * t.rs, t.base, t.ok && !col_cut<R>(t.kx, kwave(j, N), cut.kc2));
+  }
   if (shift) {
 #pragma unroll
     for (int m = 0; m < E; ++m) o[m] = o[m] * conj(half_cell_phase<R>(t.kx + kwave(rt + T * m, N), N));
@@ -150,10 +159,13 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yinv2d(const cpx<R
 }
 
 // XPASS: per row, c2r of u, v, w; u w and v w times scale; r2c of both
-// into work fields 0 and 1.  Persistent grid over groups of RPW rows.
+// into work fields 0 and 1.  Persistent grid over groups of RPW rows.  Entries
+// k >= nkx of the inputs are taken as zero and those of the outputs not
+// stored (the truncation; nx/2 + 1: all of them).
 template <class R, int M>
 __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int64_t fstride, Geom g, R scale,
-                                                                const cpx<R>* __restrict__ tw, int twsM, int twsN) {
+                                                                const cpx<R>* __restrict__ tw, int twsM, int twsN,
+                                                                int nkx) {
   using C = RowCfg<R, M>;
   constexpr int T = C::TPR;
   __shared__ cpx<R> lds[C::RPW * lds_pad(M)];
@@ -175,8 +187,11 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int
     for (int f = 0; f < 3; ++f) {
       const cpx<R>* base = W + f * fstride;
 #pragma unroll
-      for (int m = 0; m < 8; ++m) raw[f][m] = base[row * M + rt + T * m];
-      xm[f] = rt == 0 ? base[g.nmain + row] : mk<R>(0, 0);
+      for (int m = 0; m < 8; ++m) {
+        const int k = rt + T * m;
+        raw[f][m] = ld_or_zero(base, row * M + k, row * M, k < nkx);
+      }
+      xm[f] = rt == 0 && M < nkx ? base[g.nmain + row] : mk<R>(0, 0);
     }
     cpx<R> a[3][8];
 #pragma unroll
@@ -197,7 +212,7 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int
     for (int f = 0; f < 2; ++f) {
       cpx<R>* base = W + f * fstride;
       LF::run(p[f], lrow, rt, twM, 1, LinIdx{});
-      row_r2c_post<R, M>(p[f], base + row * M, base + g.nmain + row, rt, twN, 1);
+      row_r2c_post<R, M, true>(p[f], base + row * M, base + g.nmain + row, rt, twN, 1, nkx);
     }
   }
 }
@@ -219,11 +234,15 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int
 // y-inverse (yinv2d_store) goes to W[0..2] for the next RHS, which then
 // needs no y-inverse pass; S is stored only in the forced band, where the
 // forcing reads it.
+// p.trunc: the tiles of the nkx kept kx only, and of them only the modes
+// inside the cut go through memory: at the 2/3 radius a third of the tiles and
+// 65% of the state, accumulator and stage entries are left out (16 members of
+// 1024^2, FP32: 180 -> 93 us; 48 of 512^2: 90 -> 56; 192 of 256^2: 70 -> 46).
 template <class R, int N, int E, int CW, bool FUSED = false>
 __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d(cpx<R>* W, int64_t fstride, cpx<R>* WS,
                                                                    cpx<R>* ACC, cpx<R>* S, const cpx<R>* st, int mode,
                                                                    Rhs2D<R> p, Geom g,
-                                                                   const cpx<R>* __restrict__ tw, int tws) {
+                                                                   const cpx<R>* __restrict__ tw, int tws, int nkx) {
   using CC = Col2D<R, N, E, CW>;
   constexpr int T = CC::T;
   __shared__ cpx<R> lds[lds_pad(N) * CW];
@@ -231,9 +250,10 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d(cpx<R>* W, 
   for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
   const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
   const int wg = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int xtn = g.mx / CW;
+  const int xtn = ycut_tiles<CW>(g, nkx);
   const bool kx0_tile = wg < xtn * g.nz && wg % xtn == 0;  // uniform over the workgroup
-  const Tile t = col_tile<CW, 1>(g, wg, c);
+  Tile t = col_tile<CW, 1>(g, wg, c, xtn);
+  if (t.kx >= nkx) t.ok = false;
   using L = Line<R, N, E, -1>;
   cpx<R> f0[E], f1[E];
 #pragma unroll
@@ -260,7 +280,9 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d(cpx<R>* W, 
     const R k2 = ik2 == 0 ? tiny : (R)ik2;
     return p.forced && k2 >= p.fk2min && k2 <= p.fk2max;
   };
+  auto left_out = [&](int y) { return p.trunc && col_cut<R>(ikx, kwave(y, N), p.kc2); };
   auto put = [&](uint32_t y, cpx<R> v1, cpx<R> v2) {
+    if (left_out(y)) return;
     const int64_t o = t.base + (int64_t)y * t.rs;
     if (mode == 0) {
       W[o] = v1;
@@ -280,6 +302,7 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d(cpx<R>* W, 
     acc = wv;
     if (mode == 0 || !t.ok) return;
     const int y = L::out_pos(m, rt);
+    if (left_out(y)) return;
     const int iky = kwave(y, N);
     const int ik2 = ikx * ikx + iky * iky;
     const int64_t o = t.base + (int64_t)y * t.rs;
@@ -311,7 +334,7 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d(cpx<R>* W, 
     // symmetrize2d (symmetrize.f90:17-22) and the 2/3 cut
     if (y == N / 2 || t.kx == g.mx || ik2 == 0 || k2 >= p.kc2) r = mk<R>(0, 0);
     cpx<R> o1 = r, o2 = mk<R>(0, 0);
-    if (mode != 0 && t.ok) {
+    if (mode != 0 && t.ok && !left_out(y)) {
       const R x = -p.rate(k2) * p.dt / (R)2;
       const R em1 = expm1_r(x);
       const cpx<R> wv = wv_c;
