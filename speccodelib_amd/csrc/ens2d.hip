@@ -44,9 +44,9 @@ struct Group {
 };
 
 // Scheme 1 (turb_2d.f90) keeps the previous nonlinear term in F_ACC, the
-// state before the first step in F_S and the unshifted half of the
-// nonlinear term in a seventh field, F_NA.
-enum { F_W = 0, F_WS = 3, F_ACC = 4, F_S = 5, F_NA = 6, NFIELDS = 6, NFIELDS_TURB = 7 };
+// state before the first step in F_S and the shifted half's work fields in
+// three more, F_W2.
+enum { F_W = 0, F_WS = 3, F_ACC = 4, F_S = 5, F_W2 = 6, NFIELDS = 6, NFIELDS_TURB = 9 };
 
 // FP64 plans keep one schedule: E = 8 with 8 columns, 4 at 1024 points
 // (8 would need 163 KB of LDS with the line's twiddles).
@@ -189,25 +189,27 @@ int64_t row_grid_size(const scl_ens2d& e, const Group& gr) {
   return gr.row_grid ? ngroups : std::min<int64_t>(ngroups, (int64_t)resident * e.ncu);
 }
 
+// halves = 2 (here and in row_launch): the shifted half of scheme 1 as well.
 template <class R>
-int32_t yinv_launch(const Group& gr, const cpx<R>* src, int shift, hipStream_t st, Cut<R> cut) {
+int32_t yinv_launch(const Group& gr, const cpx<R>* src, int halves, hipStream_t st, Cut<R> cut) {
   const cpx<R>* tw = reinterpret_cast<const cpx<R>*>(gr.tw);
   return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
     constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
-    hipLaunchKernelGGL((k_yinv2d<R, N, E, CW>), dim3(ycut_grid<CW>(gr.g, cut.nkx)), dim3(Col2D<R, N, E, CW>::BS), 0,
-                       st, src, gr.field<R>(F_W), gr.fs(), gr.g, tw, 1, shift, cut);
+    hipLaunchKernelGGL((k_yinv2d<R, N, E, CW>), dim3(ycut_grid<CW>(gr.g, cut.nkx), halves),
+                       dim3(Col2D<R, N, E, CW>::BS), 0, st, src, gr.field<R>(F_W), gr.fs(), gr.g, tw, 1,
+                       (F_W2 - F_W) * gr.fs(), cut);
     return check_launch("yinv2d");
   });
 }
 
 template <class R>
-int32_t row_launch(const scl_ens2d& e, const Group& gr, hipStream_t st, Cut<R> cut) {
+int32_t row_launch(const scl_ens2d& e, const Group& gr, int halves, hipStream_t st, Cut<R> cut) {
   const cpx<R>* tw = reinterpret_cast<const cpx<R>*>(gr.tw);
   return with_row2d<R>(gr.n / 2, [&](auto MC) -> int32_t {
     constexpr int M = decltype(MC)::value;
     const R scale = (R)1 / (R)((double)gr.n * gr.n);
-    hipLaunchKernelGGL((k_row_adv2d<R, M>), dim3((unsigned)row_grid_size<R, M>(e, gr)), dim3(RowCfg<R, M>::BS), 0,
-                       st, gr.field<R>(F_W), gr.fs(), gr.g, scale, tw, 2, 1, cut.nkx);
+    hipLaunchKernelGGL((k_row_adv2d<R, M>), dim3((unsigned)row_grid_size<R, M>(e, gr), halves), dim3(RowCfg<R, M>::BS),
+                       0, st, gr.field<R>(F_W), gr.fs(), (F_W2 - F_W) * gr.fs(), gr.g, scale, tw, 2, 1, cut.nkx);
     return check_launch("row_adv2d");
   });
 }
@@ -231,8 +233,8 @@ int32_t stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st, boo
   const Rhs2D<R> rp = rhs_params<R>(e, gr.n, trunc);
   const Cut<R> cut = cut2d<R>(e, gr, trunc);
   if (fuse && mode < 1) return set_error("fused 2D stage: mode %d is not a stage 1..4", mode), SCL_EINVAL;
-  if (!primed) SCL_CHECK(yinv_launch<R>(gr, sin, 0, st, cut));
-  SCL_CHECK(row_launch<R>(e, gr, st, cut));
+  if (!primed) SCL_CHECK(yinv_launch<R>(gr, sin, 1, st, cut));
+  SCL_CHECK(row_launch<R>(e, gr, 1, st, cut));
   return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
     constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
     const dim3 grd(ycut_grid<CW>(gr.g, cut.nkx)), blk(Col2D<R, N, E, CW>::BS);
@@ -262,32 +264,34 @@ Turb2DP<R> turb_params(const scl_ens2d& e, int n) {
 }
 
 // One turb_2d.f90 step (mode TURB_STEP0, TURB_STEP1, TURB_AB2) or nonlinear
-// term (TURB_RHS) of a group: the unshifted half, then the shifted half and
-// the update.
+// term (TURB_RHS) of a group, both halves of the products in each pass.
+// primed, fuse: as stage.
 template <class R>
-int32_t turb_stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st) {
+int32_t turb_stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st, bool primed = false,
+                   bool fuse = false) {
   using C = cpx<R>;
   const C* tw = reinterpret_cast<const C*>(gr.tw);
   const Turb2DP<R> tp = turb_params<R>(e, gr.n);
-  for (int half = 0; half < 2; ++half) {
-    const Cut<R> all = cut2d<R>(e, gr, false);
-    SCL_CHECK(yinv_launch<R>(gr, gr.field<R>(F_WS), half, st, all));
-    SCL_CHECK(row_launch<R>(e, gr, st, all));
-    SCL_CHECK(with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
-      constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
-      hipLaunchKernelGGL((k_yfwd2d_turb<R, N, E, CW>), dim3(col_grid<CW, 1>(gr.g)), dim3(Col2D<R, N, E, CW>::BS), 0,
-                         st, gr.field<R>(F_W), gr.fs(), gr.field<R>(F_NA), gr.field<R>(F_WS), gr.field<R>(F_ACC),
-                         gr.field<R>(F_S), half ? mode : (int)TURB_HALF, tp, gr.g, tw, 1);
-      return check_launch("yfwd2d_turb");
-    }));
-  }
-  return SCL_OK;
+  const Cut<R> all = cut2d<R>(e, gr, false);
+  if (!primed) SCL_CHECK(yinv_launch<R>(gr, gr.field<R>(F_WS), 2, st, all));
+  SCL_CHECK(row_launch<R>(e, gr, 2, st, all));
+  return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
+    constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(col_grid<CW, 1>(gr.g)), dim3(Col2D<R, N, E, CW>::BS), 0, st, gr.field<R>(F_W),
+                         gr.fs(), (F_W2 - F_W) * gr.fs(), gr.field<R>(F_WS), gr.field<R>(F_ACC), gr.field<R>(F_S),
+                         mode, tp, gr.g, tw, 1);
+    };
+    if (fuse) go(k_yfwd2d_turb<R, N, E, CW, true>);
+    else go(k_yfwd2d_turb<R, N, E, CW, false>);
+    return check_launch("yfwd2d_turb");
+  });
 }
 
 int turb_mode(int64_t step) { return step == 0 ? TURB_STEP0 : step == 1 ? TURB_STEP1 : TURB_AB2; }
 
-// nsteps steps of a group as one stage chain: the first stage runs its own
-// y-inverse, every later one gets it from the previous stage's fused
+// nsteps steps of a group as one stage chain: the first stage (scheme 1: step)
+// runs its own y-inverse, every later one gets it from the previous one's fused
 // y-forward, and the last stage is not fused (the chain leaves no state in
 // W).  The kx = 0 column is made Hermitian in the same workgroup, so the
 // chain gives the same results as separate stages.  Scheme 0's passes leave
@@ -297,7 +301,8 @@ int turb_mode(int64_t step) { return step == 0 ? TURB_STEP0 : step == 1 ? TURB_S
 template <class R>
 int32_t group_steps(const scl_ens2d& e, const Group& gr, hipStream_t st, int nsteps, int64_t first, bool trunc) {
   if (e.p.scheme == 1) {
-    for (int s = 0; s < nsteps; ++s) SCL_CHECK(turb_stage<R>(e, gr, turb_mode(first + s), st));
+    for (int s = 0; s < nsteps; ++s)
+      SCL_CHECK(turb_stage<R>(e, gr, turb_mode(first + s), st, s > 0, s < nsteps - 1));
     return SCL_OK;
   }
   for (int s = 0; s < nsteps; ++s)
@@ -739,9 +744,9 @@ extern "C" int32_t scl_ens2d_rhs(scl_ens2d* e, int32_t group, int32_t member, co
     e->steps = 0;
     SCL_CHECK(e->prec == SCL_SP ? turb_stage<float>(*e, *gr, TURB_RHS, e->stream)
                                 : turb_stage<double>(*e, *gr, TURB_RHS, e->stream));
-    return take_member(*e, *gr, b, F_NA, rhs);
+  } else {
+    SCL_CHECK(e->prec == SCL_SP ? stage<float>(*e, *gr, 0, e->stream) : stage<double>(*e, *gr, 0, e->stream));
   }
-  SCL_CHECK(e->prec == SCL_SP ? stage<float>(*e, *gr, 0, e->stream) : stage<double>(*e, *gr, 0, e->stream));
   return take_member(*e, *gr, b, F_W, rhs);
 }
 

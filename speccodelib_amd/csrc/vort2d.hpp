@@ -127,16 +127,22 @@ __device__ inline cpx<R> half_cell_phase(int s, int n) {
   return mk<R>(cs, sn);
 }
 
+// The entry v of the mode with kx + ky = s of the field taken at points moved
+// by half a cell along x and y: times exp(-i pi (kx + ky)/n) (the phase shift
+// of turb_2d.f90:369-371, in the normalised coefficients of the real field).
+template <class R>
+__device__ inline cpx<R> shifted(cpx<R> v, int s, int n) {
+  return v * conj(half_cell_phase<R>(s, n));
+}
+
 // YINV.  s: the stage vorticity; w: three work fields (u, v, w) at stride
-// fstride.  shift: the fields are taken at points moved by half a cell along
-// x and y, the spectrum times exp(-i pi (kx + ky)/N) (the phase shift of
-// turb_2d.f90:369-371, in the normalised coefficients of the real field).
+// fstride.  Blocks of blockIdx.y = 1 do the shifted field, into w + hs.
 // cut: modes beyond it are taken as zero, and only its nkx columns stored.
 template <class R, int N, int E, int CW>
 __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yinv2d(const cpx<R>* __restrict__ s,
                                                                    cpx<R>* __restrict__ w, int64_t fstride, Geom g,
                                                                    const cpx<R>* __restrict__ tw, int tws,
-                                                                   int shift, Cut<R> cut) {
+                                                                   int64_t hs, Cut<R> cut) {
   using CC = Col2D<R, N, E, CW>;
   constexpr int T = CC::T;
   __shared__ cpx<R> lds[lds_pad(N) * CW];
@@ -151,21 +157,22 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yinv2d(const cpx<R
     const int j = rt + T * m;
     o[m] = ld_or_zero(s, t.base + (int64_t)j * t.rs, t.base, t.ok && !col_cut<R>(t.kx, kwave(j, N), cut.kc2));
   }
-  if (shift) {
+  if (blockIdx.y) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) o[m] = o[m] * conj(half_cell_phase<R>(t.kx + kwave(rt + T * m, N), N));
+    for (int m = 0; m < E; ++m) o[m] = shifted(o[m], t.kx + kwave(rt + T * m, N), N);
   }
-  yinv2d_store<R, N, E, CW>(o, lds, twl, rt, c, t, w, fstride);
+  yinv2d_store<R, N, E, CW>(o, lds, twl, rt, c, t, w + blockIdx.y * hs, fstride);
 }
 
 // XPASS: per row, c2r of u, v, w; u w and v w times scale; r2c of both
 // into work fields 0 and 1.  Persistent grid over groups of RPW rows.  Entries
 // k >= nkx of the inputs are taken as zero and those of the outputs not
-// stored (the truncation; nx/2 + 1: all of them).
+// stored (the truncation; nx/2 + 1: all of them).  Blocks of blockIdx.y = 1 do
+// the fields at W + hs (the shifted half of scheme 1).
 template <class R, int M>
-__global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int64_t fstride, Geom g, R scale,
-                                                                const cpx<R>* __restrict__ tw, int twsM, int twsN,
-                                                                int nkx) {
+__global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int64_t fstride, int64_t hs, Geom g,
+                                                                R scale, const cpx<R>* __restrict__ tw, int twsM,
+                                                                int twsN, int nkx) {
   using C = RowCfg<R, M>;
   constexpr int T = C::TPR;
   __shared__ cpx<R> lds[C::RPW * lds_pad(M)];
@@ -177,6 +184,7 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int
   __syncthreads();
   const int slot = threadIdx.x / T, rt = threadIdx.x % T;
   cpx<R>* lrow = lds + slot * lds_pad(M);
+  W += blockIdx.y * hs;
   using L = Line<R, M, 8, +1>;
   using LF = Line<R, M, 8, -1>;
   const int64_t ngroups = g.nrow / C::RPW;
@@ -400,25 +408,31 @@ struct Turb2DP {
   int forced;
 };
 
-enum { TURB_HALF = 0, TURB_STEP0 = 1, TURB_STEP1 = 2, TURB_AB2 = 3, TURB_RHS = 4 };
+enum { TURB_STEP0 = 1, TURB_STEP1 = 2, TURB_AB2 = 3, TURB_RHS = 4 };
 
-// YFWD of one half of the phase-shift dealiased nonlinear term
-// (turb_2d.f90:287-421) and the stepper (:430-483).  W: the two product
-// fields; NA: the unshifted half; WS: state w; OWZ: the previous nonlinear
+// YFWD of the phase-shift dealiased nonlinear term (turb_2d.f90:287-421) and
+// the stepper (:430-483).  W: the products of the unshifted (W[0], W[1]) and of
+// the shifted half (hs further on); WS: state w; OWZ: the previous nonlinear
 // term owz; W0: the state before the first step.
-//   TURB_HALF: NA = -(i/2)(kx F + ky G) of the unshifted products;
-//   otherwise N = NA - (i/2) exp(i phi)(kx F + ky G) of the shifted ones,
+//   N = -(i/2) (kx F + ky G) of the unshifted products
+//       - (i/2) exp(i phi) (kx F + ky G) of the shifted ones,
 //   zeroed on k2 >= kc2, ky = -n/2, kx = n/2 and k = 0 (dealiasing and
 //   symmetrize, :428-429), then with f(a) = etak4/conj(a) in the band:
 //   TURB_STEP0: W0 = w; OWZ = N; w = w (1 - L dt/2) + dt/2 (N + f(w))
 //   TURB_STEP1: w = W0 + dt (N + f(w)) - L dt w
 //   TURB_AB2:   w = [w + dt/2 (3 (N + f(w)) - E (owz + f(owz)))] E,
 //               E = exp(-L dt) (1 at k = 0); OWZ = N
-//   TURB_RHS:   NA = N.
+//   TURB_RHS:   W[0] = N.
 // The kx = 0 column of N and of the new w is made Hermitian as in k_yfwd2d.
-template <class R, int N, int E, int CW>
+// FUSED: the new w stays in registers and its y-inverses, unshifted and
+// shifted, go to W[0..2] and W + hs for the next step.
+// Both halves and the next step's y-inverses in one kernel make a step of two
+// launches (with the x-pass), not six, and the unshifted half of N and the
+// state do not go through memory between them (7 members of 128^2 and 3 of
+// 512^2, FP32, 200 steps and read-back: 24.8 -> 16.9 ms).
+template <class R, int N, int E, int CW, bool FUSED = false>
 __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
-    const cpx<R>* W, int64_t fstride, cpx<R>* NA, cpx<R>* WS, cpx<R>* OWZ, cpx<R>* W0, int mode, Turb2DP<R> p, Geom g,
+    cpx<R>* W, int64_t fstride, int64_t hs, cpx<R>* WS, cpx<R>* OWZ, cpx<R>* W0, int mode, Turb2DP<R> p, Geom g,
     const cpx<R>* __restrict__ tw, int tws) {
   using CC = Col2D<R, N, E, CW>;
   constexpr int T = CC::T;
@@ -431,26 +445,37 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
   const bool kx0_tile = wg < xtn * g.nz && wg % xtn == 0;
   const Tile t = col_tile<CW, 1>(g, wg, c);
   using L = Line<R, N, E, -1>;
-  cpx<R> f0[E], f1[E];
-#pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const int64_t o = t.base + (int64_t)(rt + T * m) * t.rs;
-    f0[m] = t.ok ? W[o] : mk<R>(0, 0);
-    f1[m] = t.ok ? W[o + fstride] : mk<R>(0, 0);
-  }
-  L::run(f0, lds, rt, twl, 1, ColIdx<CW>{c});
-  L::run(f1, lds, rt, twl, 1, ColIdx<CW>{c});
-  if (kx0_tile) __syncthreads();  // the transforms' LDS reads are done
   const int ikx = t.kx;
   const R kx = (R)ikx;
+  // -(i/2) (kx F + ky G) of the products at w
+  cpx<R> f0[E], f1[E];
+  auto half_term = [&](const cpx<R>* w, cpx<R>(&r)[E]) {
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const int64_t o = t.base + (int64_t)(rt + T * m) * t.rs;
+      f0[m] = t.ok ? w[o] : mk<R>(0, 0);
+      f1[m] = t.ok ? w[o + fstride] : mk<R>(0, 0);
+    }
+    L::run(f0, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+    L::run(f1, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const cpx<R> d = kx * f0[m] + (R)kwave(L::out_pos(m, rt), N) * f1[m];
+      r[m] = mk<R>((R)0.5 * d.y, (R)-0.5 * d.x);
+    }
+  };
+  cpx<R> na[E], nb[E];
+  half_term(W, na);
+  half_term(W + hs, nb);
+  if (kx0_tile) __syncthreads();  // the transforms' LDS reads are done
   auto force = [&](cpx<R> a) {
     const R den = a.x * a.x + a.y * a.y;
     return mk<R>(p.etak4 * a.x / den, p.etak4 * a.y / den);
   };
   auto put = [&](int y, cpx<R> v1, cpx<R> v2) {
     const int64_t o = t.base + (int64_t)y * t.rs;
-    if (mode == TURB_HALF || mode == TURB_RHS) {
-      NA[o] = v1;
+    if (mode == TURB_RHS) {
+      W[o] = v1;
     } else {
       WS[o] = v1;
       if (mode != TURB_STEP1) OWZ[o] = v2;
@@ -463,37 +488,33 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
     const int ik2 = ikx * ikx + iky * iky;
     const R k2 = ik2 == 0 ? (R)0.5 : (R)ik2;  // wavenumber(): k2(0, 0) = 0.5
     const int64_t o = t.base + (int64_t)y * t.rs;
-    const cpx<R> d = kx * f0[m] + (R)iky * f1[m];
-    cpx<R> r = mk<R>((R)0.5 * d.y, (R)-0.5 * d.x);  // -(i/2) d
+    cpx<R> r = na[m] + nb[m] * half_cell_phase<R>(ikx + iky, N);
+    if (y == N / 2 || ikx == g.mx || ik2 == 0 || k2 >= p.kc2) r = mk<R>(0, 0);
     cpx<R> o1 = r, o2 = mk<R>(0, 0);
-    if (mode != TURB_HALF) {
-      r = (t.ok ? NA[o] : mk<R>(0, 0)) + r * half_cell_phase<R>(ikx + iky, N);
-      if (y == N / 2 || ikx == g.mx || ik2 == 0 || k2 >= p.kc2) r = mk<R>(0, 0);
-      o1 = r;
-      if (mode != TURB_RHS && t.ok) {
-        const cpx<R> w = WS[o];
-        const R k = sqrt(k2);
-        const R ks = k * p.sigma, kn = k / p.nu;
-        const R lam = ipow(ks, 16) + (R)1 / ipow(kn, 4);
-        const bool band = p.forced && k >= p.kf && k <= p.kf + (R)3;
-        const R dth = (R)0.5 * p.dt;
-        const cpx<R> fw = band ? force(w) : mk<R>(0, 0);
-        if (mode == TURB_STEP0) {
-          o1 = ((R)1 - lam * dth) * w + dth * (r + fw);
-          o2 = r;
-          W0[o] = w;
-        } else if (mode == TURB_STEP1) {
-          o1 = W0[o] + p.dt * (r + fw) - (lam * p.dt) * w;
-        } else {
-          const R ef = ik2 == 0 ? (R)1 : exp(-lam * p.dt);
-          const cpx<R> ow = OWZ[o];
-          const cpx<R> fo = band ? force(ow) : mk<R>(0, 0);
-          o1 = ef * (w + dth * ((R)3 * (r + fw) - ef * (ow + fo)));
-          o2 = r;
-        }
+    if (mode != TURB_RHS && t.ok) {
+      const cpx<R> w = WS[o];
+      const R k = sqrt(k2);
+      const R ks = k * p.sigma, kn = k / p.nu;
+      const R lam = ipow(ks, 16) + (R)1 / ipow(kn, 4);
+      const bool band = p.forced && k >= p.kf && k <= p.kf + (R)3;
+      const R dth = (R)0.5 * p.dt;
+      const cpx<R> fw = band ? force(w) : mk<R>(0, 0);
+      if (mode == TURB_STEP0) {
+        o1 = ((R)1 - lam * dth) * w + dth * (r + fw);
+        o2 = r;
+        W0[o] = w;
+      } else if (mode == TURB_STEP1) {
+        o1 = W0[o] + p.dt * (r + fw) - (lam * p.dt) * w;
+      } else {
+        const R ef = ik2 == 0 ? (R)1 : exp(-lam * p.dt);
+        const cpx<R> ow = OWZ[o];
+        const cpx<R> fo = band ? force(ow) : mk<R>(0, 0);
+        o1 = ef * (w + dth * ((R)3 * (r + fw) - ef * (ow + fo)));
+        o2 = r;
       }
     }
     if (t.ok) put(y, o1, o2);
+    if constexpr (FUSED) na[m] = o1;
     if (kx0_tile && c == 0) {
       lds[y] = o1;
       lds[N + y] = o2;
@@ -505,9 +526,20 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
 #pragma unroll
       for (int m = 0; m < E; ++m) {
         const int y = L::out_pos(m, rt);
-        if (y > N / 2) put(y, conj(lds[N - y]), conj(lds[2 * N - y]));
+        if (y > N / 2) {
+          const cpx<R> v1 = conj(lds[N - y]);
+          put(y, v1, conj(lds[2 * N - y]));
+          if constexpr (FUSED) na[m] = v1;
+        }
       }
     }
+  }
+  if constexpr (FUSED) {
+    if (kx0_tile) __syncthreads();  // the staged kx = 0 column is read
+#pragma unroll
+    for (int m = 0; m < E; ++m) nb[m] = shifted(na[m], t.kx + kwave(rt + T * m, N), N);
+    yinv2d_store<R, N, E, CW>(na, lds, twl, rt, c, t, W, fstride);
+    yinv2d_store<R, N, E, CW>(nb, lds, twl, rt, c, t, W + hs, fstride);
   }
 }
 
