@@ -125,9 +125,13 @@ struct scl_ens2d {
   hipGraph_t graph[2] = {nullptr, nullptr};      // one step; a chunk of steps
   hipGraphExec_t exec[2] = {nullptr, nullptr};
   int chunk = 10;  // steps per chunk graph (batched mode; 1 per member)
-  // One stream for all groups: 2.03 vs 2.20 ms/step for a graph branch per
-  // size group (SCL_ENS2D_FORK=1), whose concurrent groups slow each other.
-  bool fork_groups = false;
+  // A branch per size group: a group of few members leaves most of the chip
+  // idle, and a large one its tail rounds.  us per step, one stream / a branch
+  // each (scheme 0; then scheme 1): 7 members of 128^2 and 3 of 512^2 200/128,
+  // 82/55; 20 of 64^2 and 10 of 256^2 174/110, 69/48; 40 of 256^2 and 10 of
+  // 512^2 318/197, 170/136; 192 of 256^2, 48 of 512^2 and 16 of 1024^2
+  // 1424/1413, 1336/1279.  SCL_ENS2D_FORK=0: one stream.
+  bool fork_groups = true;
   double* diag = nullptr;
   void* pin = nullptr;  // pinned host memory of the member copies
   std::mutex pin_use;
