@@ -249,6 +249,10 @@ extern "C" int32_t scl_plan3d_create(int32_t nx, int32_t ny, int32_t nz, int32_t
   // tests of that path against the oracle
   const char* uf = std::getenv("SCL_EXT_UNFUSED");
   p->zfused = nz < 1024 && ny < 1024 && !(uf && uf[0] == '1');
+  // SCL_PLANE=0: the y- and x-passes in launches of their own at any size, to
+  // compare the two
+  const char* pp = std::getenv("SCL_PLANE");
+  p->plane = !(pp && pp[0] == '0');
   (void)hipGetDevice(&p->device);
   {
     int ncu = 0;
@@ -571,7 +575,8 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
   cpx<R>* W = d.W<R>();
   Timer none;
   if (!tm) tm = &none;
-  if (rp.forced) {
+  const bool plane = Ops<R>::plane_fits(*p, 0, 0);
+  if (rp.forced && !plane) {
     tm->mark(SCL_K_FORCE);
     SCL_CHECK(Ops<R>::force_coef(*p, st, fs, fkmax, eps, eta, rp.forced, d.coef));
   }
@@ -579,12 +584,20 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
     tm->mark(SCL_K_ZINV);
     SCL_CHECK(Ops<R>::zinv_vort(*p, st, fs, W, fs));
   }
-  tm->mark(SCL_K_YINV);
-  SCL_CHECK(Ops<R>::yinv_vort(*p, W, fs, kc2_in));
-  tm->mark(SCL_K_XPASS);
-  SCL_CHECK(Ops<R>::row_convec(*p, W, fs, reinterpret_cast<cpx<R>*>(d.phys_out), kc2_in, kc2_out));
-  tm->mark(SCL_K_YFWD);
-  SCL_CHECK(Ops<R>::colfft(*p, W, fs, 3, 1, -1, kc2_out));
+  cpx<R>* const tape = reinterpret_cast<cpx<R>*>(d.phys_out);
+  if (plane) {
+    tm->mark(SCL_K_XPASS);
+    const Geom& g = p->g;
+    SCL_CHECK(Ops<R>::plane(*p, W, fs, 0, 0, (R)1 / (R)((double)g.nx * g.ny * g.nz), (R)0, (R)0, nullptr, tape,
+                            force_args<R>(st, fkmax, eps, eta, rp.forced, d.coef), kc2_in, kc2_out));
+  } else {
+    tm->mark(SCL_K_YINV);
+    SCL_CHECK(Ops<R>::yinv_vort(*p, W, fs, kc2_in));
+    tm->mark(SCL_K_XPASS);
+    SCL_CHECK(Ops<R>::row_convec(*p, W, fs, tape, kc2_in, kc2_out));
+    tm->mark(SCL_K_YFWD);
+    SCL_CHECK(Ops<R>::colfft(*p, W, fs, 3, 1, -1, kc2_out));
+  }
   tm->mark(fuse ? (mode >= 4 ? SCL_K_ZFWD4_ZINV : SCL_K_ZFWD_ZINV) : SCL_K_ZFWD);
   SCL_CHECK(Ops<R>::zfwd_rhs(*p, mode, W, fs, V, DU, S, st, d.coef, rp, fuse));
   // The kx = 0 Hermitian copy (symmetrize.f90:51-61) goes on N (mode 0),
@@ -730,13 +743,11 @@ static int32_t rk_stage_ext(scl_plan3d* p, const DevFields& d, int mode, const s
   ep.grad = (R)prm.grad;
   ep.sign_phi = 1;
   const double delta = prm.delta > 0 ? prm.delta : 2.0 * M_PI / p->g.nx;
-  if (prm.forced) {
-    tm->mark(SCL_K_FORCE);
-    SCL_CHECK(Ops<R>::force_coef(*p, st, fs, prm.fkmax, prm.eps, prm.eta, prm.forced, d.coef));
-  }
-  tm->mark(SCL_K_ZFWD);
+  if (prm.forced) tm->mark(SCL_K_FORCE);
   SCL_CHECK(ExtOps<R>::rhs(*p, mode, L, d.W<R>(), fs, d.V<R>(), d.DU<R>(), d.S<R>(), st, d.coef, ep,
-                           (R)(delta * delta), reinterpret_cast<cpx<R>*>(d.phys_out)));
+                           (R)(delta * delta), reinterpret_cast<cpx<R>*>(d.phys_out),
+                           force_args<R>(st, prm.fkmax, prm.eps, prm.eta, prm.forced, d.coef),
+                           [&] { tm->mark(SCL_K_ZFWD); }));
   // the kx = 0 Hermitian copy: as in rk_stage
   if (mode >= 1 && mode < 4 && !d.s_out) {
     tm->mark(-1);

@@ -867,17 +867,40 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
 // Forcing coefficients from the stage state: a reduction over the box of
 // modes that can satisfy k2 < fk2 (force.f90:16-24, force_heli.f90:15-42),
 // accumulated in FP64 in a fixed order.  coef = {a, b, E_f, Omega_f, uw}.
+// One workgroup of 256 threads or more (the first 256 do the sums) does it;
+// red: 3 x 256 doubles of LDS.  A kernel that runs between the state's last
+// writer and the coefficients' reader can give it a workgroup (k_plane).
 template <class R>
-__global__ __launch_bounds__(256) void k_force_coef(const cpx<R>* __restrict__ st, int64_t fstride, Geom g,
-                                                    R fk2, int fbox, double eps, double eta, int type,
-                                                    double* __restrict__ coef) {
-  __shared__ double red[3][256];
+struct ForceArgs {
+  const cpx<R>* st;
+  R fk2;
+  int fbox;
+  double eps, eta;
+  int type;  // 0: no forcing
+  double* coef;
+};
+
+// The arguments for the modes of st with |k| < fkmax.
+template <class R>
+inline ForceArgs<R> force_args(const cpx<R>* st, double fkmax, double eps, double eta, int type, double* coef) {
+  const R fk = (R)fkmax;
+  const int fbox = (int)fkmax;
+  return ForceArgs<R>{st, fk * fk, fbox < 0 ? 0 : fbox, eps, eta, type, coef};
+}
+
+template <class R>
+__device__ inline void force_coef_block(const ForceArgs<R>& fa, int64_t fstride, const Geom& g, double (*red)[256]) {
+  const cpx<R>* const st = fa.st;
+  const R fk2 = fa.fk2;
+  const int fbox = fa.fbox, type = fa.type;
+  const double eps = fa.eps, eta = fa.eta;
+  double* const coef = fa.coef;
   const int nxb = min(fbox, g.mx) + 1;
   const int nyb = min(2 * fbox + 1, g.ny), nzb = min(2 * fbox + 1, g.nz);
   const int total = nxb * nyb * nzb;
   double e = 0, en = 0, uw = 0;
   const R tiny = std::numeric_limits<R>::min();
-  for (int i = threadIdx.x; i < total; i += 256) {
+  for (int i = threadIdx.x; threadIdx.x < 256 && i < total; i += 256) {
     const int ix = i % nxb, jy = (i / nxb) % nyb, jz = i / (nxb * nyb);
     const int iy = nyb == g.ny ? jy : (jy - fbox + g.ny) % g.ny;
     const int iz = nzb == g.nz ? jz : (jz - fbox + g.nz) % g.nz;
@@ -908,9 +931,11 @@ __global__ __launch_bounds__(256) void k_force_coef(const cpx<R>* __restrict__ s
       }
     }
   }
-  red[0][threadIdx.x] = e;
-  red[1][threadIdx.x] = en;
-  red[2][threadIdx.x] = uw;
+  if (threadIdx.x < 256) {
+    red[0][threadIdx.x] = e;
+    red[1][threadIdx.x] = en;
+    red[2][threadIdx.x] = uw;
+  }
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
     if ((int)threadIdx.x < s) {
@@ -934,6 +959,12 @@ __global__ __launch_bounds__(256) void k_force_coef(const cpx<R>* __restrict__ s
     coef[3] = O;
     coef[4] = U;
   }
+}
+
+template <class R>
+__global__ __launch_bounds__(256) void k_force_coef(ForceArgs<R> fa, int64_t fstride, Geom g) {
+  __shared__ double red[3][256];
+  force_coef_block<R>(fa, fstride, g, red);
 }
 
 // IF-AB2 energy of v for the umax refresh (spectral_dns_dealiased.f90:

@@ -54,6 +54,12 @@ struct Ops {
   // tape (optional): u, w in physical space (k_row_convec TAPE)
   static int32_t row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape = nullptr, R kc2_in = 0,
                             R kc2_out = 0);
+  // the y- and x-passes of a RHS in one launch (k_plane) for the DNS (les =
+  // sc = 0) or the LES / scalar layout, where its planes fit in LDS; fa: the
+  // forcing coefficients it computes on the side (type 0: none)
+  static bool plane_fits(const scl_plan3d& pl, int les, int sc);
+  static int32_t plane(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, R sg,
+                       const double* cs2p, C* tape, const ForceArgs<R>& fa, R kc2_in = 0, R kc2_out = 0);
   static int32_t row_c2r(const scl_plan3d& pl, C* W, int64_t fstride, int nf);
   static int32_t row_r2c(const scl_plan3d& pl, C* W, int64_t fstride, int nf);
   static int32_t ref_to_split(const scl_plan3d& pl, const C* ref, C* f);

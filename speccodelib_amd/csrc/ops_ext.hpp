@@ -29,10 +29,24 @@ struct ExtOps {
 
   // N(st) of the extended RHS into W (MODE 0) or one RK4 stage (MODE 1..4).
   // W holds max(nin, nout) fields.  phys_tape (optional): where the
-  // physical-space u, w, S_ij of this evaluation are kept (k_ext_phys).
+  // physical-space u, w, S_ij of this evaluation are kept (k_ext_phys).  fa:
+  // the forcing coefficients the combine reads (type 0: there already, or not
+  // forced).  begun(): called where the transforms start.
   static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
                      const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape = nullptr) {
+    return rhs(pl, mode, L, W, fs, V, DU, S, st, coef, ep, delta2, phys_tape, ForceArgs<R>{}, [] {});
+  }
+  template <class F>
+  static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
+                     const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape, const ForceArgs<R>& fa,
+                     F&& begun) {
     const Geom& g = pl.g;
+    const bool plane = pl.zfused && Ops<R>::plane_fits(pl, L.les, L.scalar);
+    if (fa.type && !plane) {
+      hipLaunchKernelGGL((k_force_coef<R>), dim3(1), dim3(256), 0, pl.stream, fa, fs, g);
+      SCL_CHECK(check_launch("force_coef"));
+    }
+    begun();
     // 1024-point z- or y-lines keep the separate prep and combine: the
     // fused passes spill there
     const bool fused = pl.zfused;
@@ -47,6 +61,10 @@ struct ExtOps {
     // y-inverse (fused: w and S_ij formed there); the x-pass with the
     // physical products; y-forward
     const R scale = (R)1 / (R)((double)g.nx * g.ny * g.nz);
+    if (plane) {
+      SCL_CHECK(Ops<R>::plane(pl, W, fs, L.les, L.scalar, scale, delta2, (R)(-ep.sign_phi), coef + 5, phys_tape, fa));
+      return Ops<R>::ext_zfwd(pl, mode, W, fs, V, DU, S, st, coef, ep, L);
+    }
     if (fused) SCL_CHECK(Ops<R>::ext_yinv(pl, W, fs, L));
     else SCL_CHECK(Ops<R>::colfft(pl, W, fs, L.nin(), 1, +1));
     SCL_CHECK(Ops<R>::row_ext(pl, W, fs, L, scale, delta2, coef + 5, phys_tape));

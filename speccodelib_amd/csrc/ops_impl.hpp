@@ -5,6 +5,7 @@
 #include "adjoint.hpp"
 #include "les.hpp"
 #include "ops.hpp"
+#include "plane.hpp"
 
 namespace scl {
 
@@ -377,12 +378,8 @@ int32_t Ops<R>::adj_zinv(const scl_plan3d& pl, const C* s, const C* Y, C* W, int
 template <class R>
 int32_t Ops<R>::force_coef(const scl_plan3d& pl, const C* st, int64_t fstride, double fkmax, double eps, double eta,
                            int type, double* coef) {
-  const R fk = (R)fkmax;
-  const R fk2 = fk * fk;
-  int fbox = (int)std::floor(fkmax);
-  if (fbox < 0) fbox = 0;
-  hipLaunchKernelGGL((k_force_coef<R>), dim3(1), dim3(256), 0, pl.stream, st, fstride, pl.g, fk2, fbox, eps, eta, type,
-                     coef);
+  hipLaunchKernelGGL((k_force_coef<R>), dim3(1), dim3(256), 0, pl.stream,
+                     force_args<R>(st, fkmax, eps, eta, type, coef), fstride, pl.g);
   return check_launch("force_coef");
 }
 
@@ -481,6 +478,53 @@ int32_t Ops<R>::row_adj(const scl_plan3d& pl, C* W, int64_t fs, R scale, R c, R 
     if (les) return go(IC<1>{}, k_row_adj<R, M, 1>);
     return go(IC<0>{}, k_row_adj<R, M, 0>);
   });
+}
+
+// f(kernel config, kernel) for the plan's plane size and layout if its planes
+// fit in LDS; false: they don't.
+template <class R, class F>
+static bool with_plane(const scl_plan3d& pl, int les, int sc, F&& f) {
+  const Geom& g = pl.g;
+  if (!pl.plane || g.mx > 128 || g.ny > 256) return false;
+  bool fits = false;
+  (void)with_half<R>(g.mx, [&](auto MC) -> int32_t {
+    return with_line<R>(g.ny, [&](auto NC) -> int32_t {
+      constexpr int M = decltype(MC)::value, NY = decltype(NC)::value;
+      auto pick = [&](auto LC, auto SC) {
+        constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
+        if constexpr (M <= 128 && NY <= 256) {
+          using PC = PlaneCfg<R, M, NY, LES, S>;
+          if constexpr (PC::fits) {
+            fits = true;
+            f(PC{}, k_plane<R, M, NY, LES, S>);
+          }
+        }
+      };
+      if (les && sc) pick(IC<1>{}, IC<1>{});
+      else if (les) pick(IC<1>{}, IC<0>{});
+      else if (sc) pick(IC<0>{}, IC<1>{});
+      else pick(IC<0>{}, IC<0>{});
+      return SCL_OK;
+    });
+  });
+  return fits;
+}
+
+template <class R>
+bool Ops<R>::plane_fits(const scl_plan3d& pl, int les, int sc) {
+  return with_plane<R>(pl, les, sc, [](auto, auto) {});
+}
+
+template <class R>
+int32_t Ops<R>::plane(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, R sg,
+                      const double* cs2p, C* tape, const ForceArgs<R>& fa, R kc2_in, R kc2_out) {
+  const Geom& g = pl.g;
+  const bool fits = with_plane<R>(pl, les, sc, [&](auto cfg, auto kern) {
+    hipLaunchKernelGGL(kern, dim3(g.nz + (fa.type ? 1 : 0)), dim3(decltype(cfg)::BS), 0, pl.stream, W, fs, g, scale,
+                       d2, sg, cs2p, twp<R>(pl), pl.L, cut_of<R>(g, kc2_in), cut_of<R>(g, kc2_out), tape, fa);
+  });
+  if (!fits) return set_error("plane pass: (%d, %d) planes do not fit", g.nx, g.ny), SCL_EINVAL;
+  return check_launch("plane");
 }
 
 template <class R>

@@ -23,6 +23,9 @@ struct scl_plan3d {
   // combine fused into the z- and y-passes (off for 1024-point z- or
   // y-lines, where those kernels spill)
   bool zfused = true;
+  // the y- and x-passes of a RHS in one launch where the planes fit in LDS
+  // (Ops::plane_fits); SCL_PLANE=0 at plan creation: the separate passes
+  bool plane = true;
   hipStream_t stream = nullptr;
   bool own_stream = false;
   void* tw = nullptr;  // twiddle table exp(-2 pi i j/L), j < L, in the plan's precision

@@ -1,0 +1,413 @@
+// The y- and x-passes of a RHS in one launch, for planes that fit in LDS.
+//
+// Between the two z-passes everything happens within a z-plane, so where the
+// (kx, ky) planes of all its fields fit in the 160 KB of one CU's LDS, one
+// workgroup takes a plane through the y-inverse, the c2r along x, the
+// physical products, the r2c and the y-forward: of the 26 F that the separate
+// passes of a DNS RHS move (F: one field), 8 F are left, and of its four
+// launches (with the forcing coefficients', which a workgroup of their own
+// does on the side) one.  Small grids are bound by launches and by chains of
+// dependent passes: there each line transform belongs to one wavefront, which
+// needs no workgroup barrier inside it, and all fields' lines of a phase are
+// spread over the workgroup's 4 to 16 wavefronts.
+//
+// LDS holds NP planes [y][x], x in [0, M] (M = nx/2); the transforms exchange
+// in the line they transform.
+#pragma once
+
+#include "les.hpp"
+
+namespace scl {
+
+// NP planes: the largest number live at once.
+//   DNS          u(3) w(3)
+//   scalar       u(3) w(3) phi, then N(3) F(3)
+//   LES          u(3) w(3), then N(3) S(6)
+//   LES, scalar  u(3) w(3) phi, then N(3) F(3) S(6)
+template <class R, int M, int NY, int LES, int SC>
+struct PlaneCfg {
+  static constexpr int X1 = M + 1;                  // entries of a row
+  // LDS pitch of a row: with M/8 more (M >= 32) the 8 M/64 rows that a
+  // wavefront's x-lines read at once fall on banks side by side; M + 1 does
+  // the same for the short rows
+  static constexpr int P = M < 32 ? X1 : M + M / 8;
+  static constexpr int PL = P * NY;                 // entries of a plane
+  static constexpr int NP = LES ? (SC ? 12 : 9) : (SC ? 7 : 6);
+  static constexpr int TY = NY / 8, CW = 64 / TY;   // y-lines: threads per line, lines per wavefront
+  static constexpr int TX = M / 8, RW = 64 / TX;    // x-lines
+  // one line tile of 512 entries per wavefront and phase, at least 4
+  // wavefronts (the forcing sum takes 256 threads)
+  static constexpr int TASKS = NP * X1 * NY / 512;
+  static constexpr int NW = TASKS > 8 ? 16 : TASKS > 4 ? 8 : 4;
+  static constexpr int BS = 64 * NW;
+  // the planes, 512 entries where the idle lanes of a list's last tile
+  // exchange (what they hold is never used), the twiddles of both line lengths
+  // and of the real-FFT packing
+  static constexpr int LDS = NP * PL + 512 + NY + 2 * M;
+  // Where it is the faster one.  us per step, separate passes / this: DNS FP32
+  // 32^3 134/73, 64^3 169/117, 64x64x1024 641/548, 16x256x512 421/292, FP64 32^3
+  // 160/96, 16x128x512 353/251; LES 32^3 280/138, 64x16x512 473/289, FP64
+  // 16x64x256 437/283; scalar 64x64x256 386/285.  With a scalar or the
+  // Smagorinsky term and y-lines of 128 points and more, planes of many entries
+  // are slower: 15232 (scalar, 32x128x64) 256/257, 13824 (both, 16x128x512)
+  // 654/845, 19584 (LES, 32x128x64) 373/428, where 10368 (LES, 16x128x512) are
+  // not: 527/411.
+  static constexpr bool fits = TY <= 32 && TX >= 1 && TX <= 16 && (size_t)LDS * sizeof(cpx<R>) <= 160 * 1024 &&
+                               !((LES || SC) && NY >= 128 && NP * X1 * NY > 12000);
+};
+
+// What the y-inverse of output field f transforms: (i (ax kx + ay ky) + a0) A +
+// (i (bx kx + by ky) + b0) B, halved where half, from the z-pass's fields
+// W[qa], W[qb].  Tables of small digits: 4 bits a field number, 2 bits a
+// coefficient plus one.
+struct PlaneForm {
+  uint64_t qa, qb;
+  uint32_t ax, ay, a0, bx, by, b0;
+  uint32_t half;
+  __host__ __device__ constexpr void set(int f, int a, int cax, int cay, int ca0, int b, int cbx, int cby, int cb0,
+                                         bool h) {
+    qa |= (uint64_t)a << (4 * f);
+    qb |= (uint64_t)b << (4 * f);
+    ax |= (uint32_t)(cax + 1) << (2 * f);
+    ay |= (uint32_t)(cay + 1) << (2 * f);
+    a0 |= (uint32_t)(ca0 + 1) << (2 * f);
+    bx |= (uint32_t)(cbx + 1) << (2 * f);
+    by |= (uint32_t)(cby + 1) << (2 * f);
+    b0 |= (uint32_t)(cb0 + 1) << (2 * f);
+    half |= (uint32_t)h << f;
+  }
+};
+
+// DNS: u, w_x, w_y from zinv_store, w_z formed here.  Scalar: all from
+// k_ext_zinv.  LES: u, i kz u_x, i kz u_y, i kz u_z (= S_33) from k_ext_zinv,
+// w and the other S_ij formed here, as k_yinv_les does.
+template <int LES, int SC>
+__host__ __device__ constexpr PlaneForm plane_form() {
+  PlaneForm t{};
+  for (int f = 0; f < 3; ++f) t.set(f, f, 0, 0, 1, f, 0, 0, 0, false);
+  if (LES) {
+    t.set(3, 2, 0, 1, 0, 4, 0, 0, -1, false);   // w_x = i ky u_z - i kz u_y
+    t.set(4, 2, -1, 0, 0, 3, 0, 0, 1, false);   // w_y = i kz u_x - i kx u_z
+  } else {
+    t.set(3, 3, 0, 0, 1, 3, 0, 0, 0, false);
+    t.set(4, 4, 0, 0, 1, 4, 0, 0, 0, false);
+  }
+  if (LES || !SC) t.set(5, 1, 1, 0, 0, 0, 0, -1, 0, false);  // w_z = i kx u_y - i ky u_x
+  else t.set(5, 5, 0, 0, 1, 5, 0, 0, 0, false);
+  if (LES) {
+    t.set(6, 0, 1, 0, 0, 0, 0, 0, 0, false);    // S_11
+    t.set(7, 1, 1, 0, 0, 0, 0, 1, 0, true);     // S_12
+    t.set(8, 2, 1, 0, 0, 3, 0, 0, 1, true);     // S_13
+    t.set(9, 1, 0, 1, 0, 1, 0, 0, 0, false);    // S_22
+    t.set(10, 2, 0, 1, 0, 4, 0, 0, 1, true);    // S_23
+    t.set(11, 11, 0, 0, 1, 11, 0, 0, 0, false); // S_33
+  }
+  const int ph = 6 + 6 * LES;
+  if (SC) t.set(ph, ph, 0, 0, 1, ph, 0, 0, 0, false);
+  return t;
+}
+
+// One workgroup per z-plane, and, with forcing, one more for its coefficients.
+// in, out: the truncation of the inputs (columns outside hold nothing) and of
+// the outputs (not wanted outside).  tape: u, w [, S_ij] in physical space, as
+// k_row_convec and k_row_ext leave them.  The workgroup reads all it needs of
+// its plane of W before it writes any of it.
+template <class R, int M, int NY, int LES, int SC>
+__global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
+    cpx<R>* W, int64_t fs, Geom g, R scale, R d2, R sg, const double* __restrict__ cs2p, const cpx<R>* __restrict__ tw,
+    int L, Cut<R> in, Cut<R> out, cpx<R>* __restrict__ tape, ForceArgs<R> fa) {
+  using C = PlaneCfg<R, M, NY, LES, SC>;
+  constexpr int X1 = C::X1, P = C::P, PL = C::PL, NW = C::NW, CW = C::CW, TY = C::TY, TX = C::TX, RW = C::RW;
+  constexpr ExtLayout X{LES, SC};
+  constexpr PlaneForm F = plane_form<LES, SC>();
+  __shared__ cpx<R> sh[C::LDS];
+  if ((int)blockIdx.x == g.nz) {
+    force_coef_block<R>(fa, fs, g, reinterpret_cast<double(*)[256]>(sh));
+    return;
+  }
+  constexpr int IDLE = C::NP * PL;
+  cpx<R>* const twY = sh + IDLE + 512;
+  cpx<R>* const twM = twY + NY;
+  cpx<R>* const twN = twM + M;
+  for (int i = threadIdx.x; i < NY; i += C::BS) twY[i] = tw[i * (L / NY)];
+  for (int i = threadIdx.x; i < M; i += C::BS) {
+    twM[i] = tw[i * (L / M)];
+    twN[i] = tw[i * (L / g.nx)];
+  }
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int z = blockIdx.x;
+  __syncthreads();
+
+  // y-lines: the columns x of all fields in one list, CW of them a tile
+  const int yc = lane % CW, yr = lane / CW;
+  auto y_index = [&](int q, int x, bool ok) {
+    return [=](int pos) { return ok ? q * PL + pos * P + x : IDLE + pos * CW + yc; };
+  };
+  // column x of this plane in a field: entry j at o + j st (a field of planes
+  // this small has far fewer than 2^31 entries)
+  struct Col {
+    uint32_t o, st;
+    __device__ uint32_t at(int j) const { return o + (uint32_t)j * st; }
+  };
+  const uint32_t row0 = (uint32_t)g.row(0, z);
+  auto column = [&](int x) {
+    return x < M ? Col{row0 * (uint32_t)M + (uint32_t)x, (uint32_t)M << g.zs}
+                 : Col{(uint32_t)g.nmain + row0, 1u << g.zs};
+  };
+  // y-inverse of the fields first .. first + n - 1 into the planes from to on
+  auto y_inverse = [&](int first, int n, int to, int w0) {
+    using Ln = Line<R, NY, 8, +1, true>;
+    const int cols = n * X1;
+    for (int task = w0; task * CW < cols; task += NW) {
+      const int col = task * CW + yc;
+      const bool ok = col < cols;
+      const int q = ok ? col / X1 : 0, x = ok ? col % X1 : 0, f = first + q;
+      const Col cl = column(x);
+      // no truncation: one branch for the wavefront, not one per entry
+      auto load = [&](cpx<R>(&a)[8], const cpx<R>* A) {
+        if (in.nkx > M) {
+#pragma unroll
+          for (int m = 0; m < 8; ++m) a[m] = A[cl.at(yr + TY * m)];
+        } else {
+#pragma unroll
+          for (int m = 0; m < 8; ++m) {
+            const int j = yr + TY * m;
+            a[m] = ld_or_zero(A, cl.at(j), cl.o, x < in.nkx && !col_cut<R>(x, kwave(j, NY), in.kc2));
+          }
+        }
+      };
+      cpx<R> v[8];
+      load(v, W + (int)((F.qa >> (4 * f)) & 15u) * fs);
+      // a tile of fields that the z-pass has left ready takes them as they are
+      const bool formed = LES ? true : !SC && (task * CW + CW - 1) / X1 + first >= 5;
+      if (formed) {
+        auto digit = [&](uint32_t t) { return (R)((int)((t >> (2 * f)) & 3u) - 1); };
+        const R a0 = digit(F.a0), b0 = digit(F.b0), ay = digit(F.ay), by = digit(F.by);
+        const R akx = digit(F.ax) * (R)x, bkx = digit(F.bx) * (R)x;
+        const R h = ((F.half >> f) & 1u) ? (R)0.5 : (R)1;
+        cpx<R> b[8];
+        load(b, W + (int)((F.qb >> (4 * f)) & 15u) * fs);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+          const R ky = (R)kwave(yr + TY * m, NY);
+          const R ka = akx + ay * ky, kb = bkx + by * ky;
+          v[m] = mk<R>(h * (a0 * v[m].x - ka * v[m].y + (b0 * b[m].x - kb * b[m].y)),
+                       h * (a0 * v[m].y + ka * v[m].x + (b0 * b[m].y + kb * b[m].x)));
+        }
+      }
+      const auto at = y_index(to + q, x, ok);
+      Ln::run(v, sh, yr, twY, 1, at);
+#pragma unroll
+      for (int m = 0; m < 8; ++m) sh[at(Ln::out_pos(m, yr))] = v[m];
+    }
+  };
+
+  // x-lines: the rows of n planes in one list, RW of them a tile
+  const int xs = lane / TX, xr = lane % TX;
+  // c2r of the planes from to on, in place; the physical rows also to the
+  // tape's fields from tf on (tf < 0: not)
+  auto c2r = [&](int to, int n, int tf) {
+    using Ln = Line<R, M, 8, +1, true>;
+    const int rows = n * NY;
+    for (int task = wave; task * RW < rows; task += NW) {
+      const int r = task * RW + xs;
+      const bool ok = r < rows;
+      const int q = ok ? r / NY : 0, y = ok ? r % NY : 0;
+      const int base = (to + q) * PL + y * P;
+      auto at = [=](int pos) { return ok ? base + pos : IDLE + xs * M + pos; };
+      cpx<R> raw[8], a[8];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) raw[m] = sh[base + xr + TX * m];
+      const cpx<R> xm = sh[base + M];
+      row_c2r_prep<R, M>(a, raw, xm, xr, twN, 1);
+      wave_sync();
+      Ln::run(a, sh, xr, twM, 1, at);
+#pragma unroll
+      for (int m = 0; m < 8; ++m) sh[at(Ln::out_pos(m, xr))] = a[m];
+      if (tape && tf >= 0 && ok) {
+        cpx<R>* const tb = tape + (tf + q) * fs + g.row(y, z) * M;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) tb[Ln::out_pos(m, xr)] = a[m];
+      }
+    }
+  };
+  auto r2c = [&](int to, int n) {
+    using Ln = Line<R, M, 8, -1, true>;
+    const int rows = n * NY;
+    for (int task = wave; task * RW < rows; task += NW) {
+      const int r = task * RW + xs;
+      const bool ok = r < rows;
+      const int q = ok ? r / NY : 0, y = ok ? r % NY : 0;
+      const int base = (to + q) * PL + y * P;
+      auto at = [=](int pos) { return ok ? base + pos : IDLE + xs * M + pos; };
+      cpx<R> p[8];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) p[m] = sh[base + xr + TX * m];
+      wave_sync();
+      Ln::run(p, sh, xr, twM, 1, at);
+      row_r2c_post<R, M>(p, sh + (ok ? base : IDLE + xs * M), sh + (ok ? base + M : IDLE), xr, twN, 1);
+    }
+  };
+
+  constexpr int N0 = 0, F0 = 3, S0 = SC ? 6 : 3;  // planes of N, the fluxes and S_ij, tau_ij
+  y_inverse(0, 6, 0, wave);
+  if constexpr (SC != 0) y_inverse(X.phi_in(), 1, 6, wave);
+  __syncthreads();
+  c2r(0, 6, 0);
+  if constexpr (SC != 0) c2r(6, 1, -1);
+  __syncthreads();
+  // u x w and u_j phi on the packed reals, in place (convec_dns.f90:30-42,
+  // convecphi_dns.f90:23,33,42)
+  for (int i = threadIdx.x; i < M * NY; i += C::BS) {
+    const int o = (i / M) * P + i % M;
+    cpx<R> u[3], w[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      u[q] = sh[q * PL + o];
+      w[q] = sh[(3 + q) * PL + o];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int q1 = (q + 1) % 3, q2 = (q + 2) % 3;
+      sh[(N0 + q) * PL + o] = mk<R>((u[q1].x * w[q2].x - u[q2].x * w[q1].x) * scale,
+                                    (u[q1].y * w[q2].y - u[q2].y * w[q1].y) * scale);
+    }
+    if constexpr (SC != 0) {
+      const cpx<R> ph = sh[6 * PL + o];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) sh[(F0 + q) * PL + o] = mk<R>(u[q].x * ph.x * scale, u[q].y * ph.y * scale);
+    }
+  }
+  __syncthreads();
+  r2c(N0, 3 + 3 * SC);
+  if constexpr (LES != 0) {
+    // the S_ij planes are free of w and phi here; the tiles go on from the
+    // wavefront after the last of the r2c's
+    y_inverse(X.s_in(), 6, S0, (wave + NW - ((3 + 3 * SC) * NY / RW) % NW) % NW);
+    __syncthreads();
+    c2r(S0, 6, 6);
+    __syncthreads();
+    // tau_ij = -2 cs2 D^2 |S| S_ij (dynsmag.f90:206-225)
+    const R c = (R)(-2.0 * cs2p[0]) * d2 * scale;
+    for (int i = threadIdx.x; i < M * NY; i += C::BS) {
+      const int o = (i / M) * P + i % M;
+      R sx[6], sy[6];
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        const cpx<R> s = sh[(S0 + q) * PL + o];
+        sx[q] = s.x;
+        sy[q] = s.y;
+      }
+      const R ax = c * abs_strain<R>(sx), ay = c * abs_strain<R>(sy);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) sh[(S0 + q) * PL + o] = mk<R>(ax * sx[q], ay * sy[q]);
+    }
+    __syncthreads();
+    r2c(S0, 6);
+  }
+  __syncthreads();
+
+  // y-forward and the fields the z-pass takes.  The terms with kx are formed
+  // before the transform, those with ky after it, so tau_12, tau_22, F_y only
+  // pass through registers (k_yfwd_ext writes the same fields).  A tile of the
+  // list does everything that touches one field's column group: transforms
+  // exchange in the first one's line, whose other readers are none.
+  using Lf = Line<R, NY, 8, -1, true>;
+  auto load_col = [&](cpx<R>(&v)[8], int q, int x) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) v[m] = sh[q * PL + (yr + TY * m) * P + x];
+  };
+  auto store = [&](const cpx<R>(&v)[8], int q, int x, bool ok) {
+    const Col cl = column(x);
+    cpx<R>* const w = W + q * fs;
+    if (out.nkx > M) {
+      if (!ok) return;
+#pragma unroll
+      for (int m = 0; m < 8; ++m) w[cl.at(Lf::out_pos(m, yr))] = v[m];
+    } else if (ok && x < out.nkx) {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        const int j = Lf::out_pos(m, yr);
+        if (!col_cut<R>(x, kwave(j, NY), out.kc2)) w[cl.at(j)] = v[m];
+      }
+    }
+  };
+  auto ky = [&](int m) { return (R)kwave(Lf::out_pos(m, yr), NY); };
+  if constexpr (LES == 0 && SC == 0) {
+    for (int task = wave; task * CW < 3 * X1; task += NW) {
+      const int col = task * CW + yc;
+      const bool ok = col < 3 * X1;
+      const int q = ok ? col / X1 : 0, x = ok ? col % X1 : 0;
+      cpx<R> v[8];
+      load_col(v, q, x);
+      wave_sync();
+      Lf::run(v, sh, yr, twY, 1, y_index(q, x, ok));
+      store(v, q, x, ok);
+    }
+  } else {
+    constexpr int XT = (X1 + CW - 1) / CW;  // tiles of a field
+    constexpr int KINDS = 3 + LES + 2 * SC;
+    constexpr int t0 = X.tau_out(), f0 = X.flux_out();
+    for (int task = wave; task < KINDS * XT; task += NW) {
+      const int kind = task / XT, x = (task % XT) * CW + yc;
+      const bool ok = x < X1;
+      const int xx = ok ? x : 0;
+      const R kx = (R)xx;
+      cpx<R> a[8], b[8], d[8];
+      if (LES != 0 && kind < 3) {
+        // N_i - i kx tau_i1 - i ky tau_i2: i = 3 first, the longest
+        constexpr int T1[3] = {2, 0, 1}, T2[3] = {4, 1, 3};
+        const int i = kind == 0 ? 2 : kind - 1;
+        const int p1 = kind == 0 ? T1[0] : kind == 1 ? T1[1] : T1[2];
+        const int p2 = kind == 0 ? T2[0] : kind == 1 ? T2[1] : T2[2];
+        load_col(a, N0 + i, xx);
+        load_col(d, S0 + p1, xx);
+        load_col(b, S0 + p2, xx);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) a[m] = a[m] - mul_i(kx * d[m]);
+        const auto at = y_index(N0 + i, xx, ok);
+        wave_sync();
+        Lf::run(a, sh, yr, twY, 1, at);
+        Lf::run(b, sh, yr, twY, 1, at);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) a[m] = a[m] - mul_i(ky(m) * b[m]);
+        store(a, i, xx, ok);
+        if (kind == 0) {
+          store(b, t0 + 4, xx, ok);  // tau_23
+          Lf::run(d, sh, yr, twY, 1, at);
+          store(d, t0 + 2, xx, ok);  // tau_13
+        }
+      } else if (LES == 0 && kind < 3) {
+        load_col(a, N0 + kind, xx);
+        wave_sync();
+        Lf::run(a, sh, yr, twY, 1, y_index(N0 + kind, xx, ok));
+        store(a, kind, xx, ok);
+      } else if (LES != 0 && kind == 3) {
+        load_col(a, S0 + 5, xx);
+        wave_sync();
+        Lf::run(a, sh, yr, twY, 1, y_index(S0 + 5, xx, ok));
+        store(a, t0 + 5, xx, ok);  // tau_33
+      } else if (kind == KINDS - 2) {
+        // sg (i kx F_x + i ky F_y)
+        load_col(a, F0, xx);
+        load_col(b, F0 + 1, xx);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) a[m] = sg * mul_i(kx * a[m]);
+        const auto at = y_index(F0, xx, ok);
+        wave_sync();
+        Lf::run(a, sh, yr, twY, 1, at);
+        Lf::run(b, sh, yr, twY, 1, at);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) a[m] = a[m] + sg * mul_i(ky(m) * b[m]);
+        store(a, f0, xx, ok);
+      } else {
+        load_col(a, F0 + 2, xx);
+        wave_sync();
+        Lf::run(a, sh, yr, twY, 1, y_index(F0 + 2, xx, ok));
+        store(a, f0 + 2, xx, ok);  // F_z
+      }
+    }
+  }
+}
+
+}  // namespace scl

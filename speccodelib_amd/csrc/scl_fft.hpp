@@ -167,12 +167,24 @@ __device__ inline int pass_out_pos(int m, int rt) {
   return (j / NS) * NS * RAD + (j & (NS - 1)) + r * NS;
 }
 
-template <class R, int N, int E, int DIR, int NS, class L>
+// Between a wavefront's own LDS writes and reads: the LDS serves one
+// wavefront's accesses in order, so only the compiler has to keep theirs.
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <class R, int N, int E, int DIR, int NS, class L, bool WAVE>
 struct Passes;
 
-template <class R, int N, int E, int DIR, int NS, int RAD, int... REST>
-struct Passes<R, N, E, DIR, NS, RList<RAD, REST...>> {
-  using Next = Passes<R, N, E, DIR, NS * RAD, RList<REST...>>;
+template <class R, int N, int E, int DIR, int NS, int RAD, int... REST, bool WAVE>
+struct Passes<R, N, E, DIR, NS, RList<RAD, REST...>, WAVE> {
+  using Next = Passes<R, N, E, DIR, NS * RAD, RList<REST...>, WAVE>;
+  __device__ static inline void sync() {
+    if constexpr (WAVE) wave_sync();
+    else __syncthreads();
+  }
   template <class IDX>
   __device__ static inline void run(cpx<R> (&v)[E], cpx<R>* lds, int rt, const cpx<R>* tw, int tws,
                                     const IDX& idx) {
@@ -181,10 +193,10 @@ struct Passes<R, N, E, DIR, NS, RList<RAD, REST...>> {
       constexpr int T = N / E;
 #pragma unroll
       for (int m = 0; m < E; ++m) lds[idx(pass_out_pos<N, E, NS, RAD>(m, rt))] = v[m];
-      __syncthreads();
+      sync();
 #pragma unroll
       for (int m = 0; m < E; ++m) v[m] = lds[idx(rt + T * m)];
-      __syncthreads();
+      sync();
       Next::run(v, lds, rt, tw, tws, idx);
     }
   }
@@ -196,10 +208,11 @@ struct Passes<R, N, E, DIR, NS, RList<RAD, REST...>> {
 
 // Full line transform.  LDS must hold N points addressed through idx; all
 // threads of the block must call it (it synchronises the block).  On return
-// the LDS region is free for reuse.
-template <class R, int N, int E, int DIR>
+// the LDS region is free for reuse.  WAVE: every line is inside one wavefront
+// and only that wavefront uses its LDS region; no workgroup barrier is needed.
+template <class R, int N, int E, int DIR, bool WAVE = false>
 struct Line {
-  using P = Passes<R, N, E, DIR, 1, typename PlanOf<N, E>::L>;
+  using P = Passes<R, N, E, DIR, 1, typename PlanOf<N, E>::L, WAVE>;
   template <class IDX>
   __device__ static inline void run(cpx<R> (&v)[E], cpx<R>* lds, int rt, const cpx<R>* tw, int tws,
                                     const IDX& idx) {
