@@ -220,6 +220,9 @@ template <class R>
 struct Cut {
   R kc2;
   int nkx;
+  // nothing is left out (nkx alone does not say so: a radius above nx/2 keeps
+  // every kx and still leaves out columns)
+  __device__ bool all() const { return kc2 == std::numeric_limits<R>::infinity(); }
 };
 
 // Tile order of a z-pass that leaves tiles out: the left-out tiles are those

@@ -165,7 +165,7 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
       const Col cl = column(x);
       // no truncation: one branch for the wavefront, not one per entry
       auto load = [&](cpx<R>(&a)[8], const cpx<R>* A) {
-        if (in.nkx > M) {
+        if (in.all()) {
 #pragma unroll
           for (int m = 0; m < 8; ++m) a[m] = A[cl.at(yr + TY * m)];
         } else {
@@ -320,7 +320,7 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
   auto store = [&](const cpx<R>(&v)[8], int q, int x, bool ok) {
     const Col cl = column(x);
     cpx<R>* const w = W + q * fs;
-    if (out.nkx > M) {
+    if (out.all()) {
       if (!ok) return;
 #pragma unroll
       for (int m = 0; m < 8; ++m) w[cl.at(Lf::out_pos(m, yr))] = v[m];

@@ -72,6 +72,11 @@ def test_truncated_and_ab2_steps(monkeypatch, kw):
     compare(monkeypatch, (64, 64, 128), scl.SP, steps=5, forced=1, **kw)
 
 
+def test_radius_above_half_nx(monkeypatch):
+    """Every kx is kept, and still not every column."""
+    compare(monkeypatch, (32, 64, 512), scl.SP, steps=5, forced=1, kcut=20.5)
+
+
 @pytest.mark.parametrize("sgs", [0, 1])
 def test_blocked_row_order(monkeypatch, sgs):
     compare(monkeypatch, (32, 32, 32), scl.DP, zblock=8, forced=1, sgs=sgs, cs2=0.03 if sgs else 0.0)
