@@ -95,6 +95,11 @@ int32_t set_cs2(scl_adjoint* a, double cs2) {
 
 DevFields dev(const scl_adjoint* a) {
   DevFields d{a->fields, a->plan->fstride(), 3, a->coef};
+  // dL/dc_s^2 comes back in FP64, also from an FP32 plan, and moves in its
+  // eighth digit with the rounding of the forward passes (6e-8 at 64^3): the LES
+  // keeps theirs, though the passes with a wavefront per field would take 14.3
+  // ms for 17.4 there.
+  d.separate = a->L.les;
   return d;
 }
 

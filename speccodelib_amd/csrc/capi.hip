@@ -249,8 +249,8 @@ extern "C" int32_t scl_plan3d_create(int32_t nx, int32_t ny, int32_t nz, int32_t
   // tests of that path against the oracle
   const char* uf = std::getenv("SCL_EXT_UNFUSED");
   p->zfused = nz < 1024 && ny < 1024 && !(uf && uf[0] == '1');
-  // SCL_PLANE=0: the y- and x-passes in launches of their own at any size, to
-  // compare the two
+  // SCL_PLANE=0: the y- and x-passes in launches of their own, all fields of a
+  // line in one wavefront, at any size, to compare the two
   const char* pp = std::getenv("SCL_PLANE");
   p->plane = !(pp && pp[0] == '0');
   (void)hipGetDevice(&p->device);
@@ -576,7 +576,8 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
   Timer none;
   if (!tm) tm = &none;
   const bool plane = Ops<R>::plane_fits(*p, 0, 0);
-  if (rp.forced && !plane) {
+  const bool sy = !plane && Ops<R>::split_y(*p, 0, 0);
+  if (rp.forced && !plane && !sy) {
     tm->mark(SCL_K_FORCE);
     SCL_CHECK(Ops<R>::force_coef(*p, st, fs, fkmax, eps, eta, rp.forced, d.coef));
   }
@@ -592,9 +593,16 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
                             force_args<R>(st, fkmax, eps, eta, rp.forced, d.coef), kc2_in, kc2_out));
   } else {
     tm->mark(SCL_K_YINV);
-    SCL_CHECK(Ops<R>::yinv_vort(*p, W, fs, kc2_in));
+    if (sy)
+      SCL_CHECK(Ops<R>::yinv_split(*p, W, fs, 0, 0, force_args<R>(st, fkmax, eps, eta, rp.forced, d.coef), kc2_in));
+    else
+      SCL_CHECK(Ops<R>::yinv_vort(*p, W, fs, kc2_in));
     tm->mark(SCL_K_XPASS);
-    SCL_CHECK(Ops<R>::row_convec(*p, W, fs, tape, kc2_in, kc2_out));
+    if (Ops<R>::split_x(*p, 0, 0))
+      SCL_CHECK(Ops<R>::row_split(*p, W, fs, 0, 0, (R)1 / (R)((double)p->g.nx * p->g.ny * p->g.nz), (R)0, nullptr, tape,
+                                  kc2_in, kc2_out));
+    else
+      SCL_CHECK(Ops<R>::row_convec(*p, W, fs, tape, kc2_in, kc2_out));
     tm->mark(SCL_K_YFWD);
     SCL_CHECK(Ops<R>::colfft(*p, W, fs, 3, 1, -1, kc2_out));
   }
@@ -747,7 +755,7 @@ static int32_t rk_stage_ext(scl_plan3d* p, const DevFields& d, int mode, const s
   SCL_CHECK(ExtOps<R>::rhs(*p, mode, L, d.W<R>(), fs, d.V<R>(), d.DU<R>(), d.S<R>(), st, d.coef, ep,
                            (R)(delta * delta), reinterpret_cast<cpx<R>*>(d.phys_out),
                            force_args<R>(st, prm.fkmax, prm.eps, prm.eta, prm.forced, d.coef),
-                           [&] { tm->mark(SCL_K_ZFWD); }));
+                           [&] { tm->mark(SCL_K_ZFWD); }, d.separate));
   // the kx = 0 Hermitian copy: as in rk_stage
   if (mode >= 1 && mode < 4 && !d.s_out) {
     tm->mark(-1);

@@ -60,6 +60,15 @@ struct Ops {
   static bool plane_fits(const scl_plan3d& pl, int les, int sc);
   static int32_t plane(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, R sg,
                        const double* cs2p, C* tape, const ForceArgs<R>& fa, R kc2_in = 0, R kc2_out = 0);
+  // the y- and x-passes of the DNS / LES / scalar RHS with a wavefront per
+  // field (k_yinv_split, k_row_split, k_yfwd_split)
+  static bool split_y(const scl_plan3d& pl, int les, int sc);
+  static bool split_x(const scl_plan3d& pl, int les, int sc);
+  static int32_t yinv_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, const ForceArgs<R>& fa,
+                            R kc2 = 0);
+  static int32_t row_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, const double* cs2p,
+                           C* tape, R kc2_in = 0, R kc2_out = 0);
+  static int32_t yfwd_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R sg);
   static int32_t row_c2r(const scl_plan3d& pl, C* W, int64_t fstride, int nf);
   static int32_t row_r2c(const scl_plan3d& pl, C* W, int64_t fstride, int nf);
   static int32_t ref_to_split(const scl_plan3d& pl, const C* ref, C* f);

@@ -31,7 +31,8 @@ struct ExtOps {
   // W holds max(nin, nout) fields.  phys_tape (optional): where the
   // physical-space u, w, S_ij of this evaluation are kept (k_ext_phys).  fa:
   // the forcing coefficients the combine reads (type 0: there already, or not
-  // forced).  begun(): called where the transforms start.
+  // forced).  begun(): called where the transforms start.  separate: as
+  // DevFields.
   static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
                      const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape = nullptr) {
     return rhs(pl, mode, L, W, fs, V, DU, S, st, coef, ep, delta2, phys_tape, ForceArgs<R>{}, [] {});
@@ -39,10 +40,11 @@ struct ExtOps {
   template <class F>
   static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
                      const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape, const ForceArgs<R>& fa,
-                     F&& begun) {
+                     F&& begun, bool separate = false) {
     const Geom& g = pl.g;
-    const bool plane = pl.zfused && Ops<R>::plane_fits(pl, L.les, L.scalar);
-    if (fa.type && !plane) {
+    const bool plane = !separate && pl.zfused && Ops<R>::plane_fits(pl, L.les, L.scalar);
+    const bool sy = !separate && pl.zfused && !plane && Ops<R>::split_y(pl, L.les, L.scalar);
+    if (fa.type && !plane && !sy) {
       hipLaunchKernelGGL((k_force_coef<R>), dim3(1), dim3(256), 0, pl.stream, fa, fs, g);
       SCL_CHECK(check_launch("force_coef"));
     }
@@ -65,9 +67,17 @@ struct ExtOps {
       SCL_CHECK(Ops<R>::plane(pl, W, fs, L.les, L.scalar, scale, delta2, (R)(-ep.sign_phi), coef + 5, phys_tape, fa));
       return Ops<R>::ext_zfwd(pl, mode, W, fs, V, DU, S, st, coef, ep, L);
     }
-    if (fused) SCL_CHECK(Ops<R>::ext_yinv(pl, W, fs, L));
+    if (sy) SCL_CHECK(Ops<R>::yinv_split(pl, W, fs, L.les, L.scalar, fa));
+    else if (fused) SCL_CHECK(Ops<R>::ext_yinv(pl, W, fs, L));
     else SCL_CHECK(Ops<R>::colfft(pl, W, fs, L.nin(), 1, +1));
-    SCL_CHECK(Ops<R>::row_ext(pl, W, fs, L, scale, delta2, coef + 5, phys_tape));
+    if (!separate && Ops<R>::split_x(pl, L.les, L.scalar))
+      SCL_CHECK(Ops<R>::row_split(pl, W, fs, L.les, L.scalar, scale, delta2, coef + 5, phys_tape));
+    else
+      SCL_CHECK(Ops<R>::row_ext(pl, W, fs, L, scale, delta2, coef + 5, phys_tape));
+    if (sy) {
+      SCL_CHECK(Ops<R>::yfwd_split(pl, W, fs, L.les, L.scalar, (R)(-ep.sign_phi)));
+      return Ops<R>::ext_zfwd(pl, mode, W, fs, V, DU, S, st, coef, ep, L);
+    }
     // fused: the y-forward folds the kx, ky terms and the z-forward the kz
     // terms and the combine; else plain passes and the combine kernel
     if (fused) {

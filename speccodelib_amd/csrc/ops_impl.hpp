@@ -495,6 +495,7 @@ static bool with_plane(const scl_plan3d& pl, int les, int sc, F&& f) {
         if constexpr (M <= 128 && NY <= 256) {
           using PC = PlaneCfg<R, M, NY, LES, S>;
           if constexpr (PC::fits) {
+            if (g.nz > PC::max_nz) return;
             fits = true;
             f(PC{}, k_plane<R, M, NY, LES, S>);
           }
@@ -525,6 +526,115 @@ int32_t Ops<R>::plane(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R
   });
   if (!fits) return set_error("plane pass: (%d, %d) planes do not fit", g.nx, g.ny), SCL_EINVAL;
   return check_launch("plane");
+}
+
+// f(les, sc) with both as compile-time constants.
+template <class F>
+static int32_t with_layout(int les, int sc, F&& f) {
+  if (les && sc) return f(IC<1>{}, IC<1>{});
+  if (les) return f(IC<1>{}, IC<0>{});
+  if (sc) return f(IC<0>{}, IC<1>{});
+  return f(IC<0>{}, IC<0>{});
+}
+
+// Whether the y-passes run with a wavefront per field.  A wavefront holds
+// 512/ny columns, so the longer the lines the shorter the row segments that it
+// reads, and the smaller a field must be for the caches to serve the rest of
+// each 128-byte line.  The FP64 LES kernels that it replaces run at two waves
+// per SIMD, which it beats at larger sizes too.  us per step with three solvers
+// running side by side, separate / this: DNS FP32 128x64x64 93/85, 256x64x256
+// (16 MB a field, segments of 64 bytes) 505/498, 128x128x32 (2 MB, 32) 95/89,
+// 128^3 (8 MB, 32) 218/232, 32x256x64 (2 MB, 16) 94/96; LES FP32 64^3 128/107,
+// 512x64x64 (8 MB, 64) 602/603, 1024x64x64 1284/1309, 128^3 584/648; FP64 LES
+// 128^3 (16 MB, 64) 1309/1252, 256x64x256 (32 MB) 2693/2407, 32x256x64 (4 MB,
+// 32) 384/311; with split_x too, DNS FP64 64^3 92/76, 128x64x128 (8 MB) 216/233.
+template <class R>
+bool Ops<R>::split_y(const scl_plan3d& pl, int les, int sc) {
+  const Geom& g = pl.g;
+  if (!pl.plane || g.ny > 256 || g.mx % (512 / g.ny)) return false;
+  const int seg = 512 / g.ny * (int)sizeof(C);  // bytes
+  int64_t mb = 0;                               // the largest field
+  if (sizeof(R) == 4) mb = seg >= 64 ? (les ? 8 : 16) : seg == 32 ? 2 : 0;
+  else if (les) mb = seg >= 64 ? 32 : 4;
+  else mb = seg >= 64 ? 4 : 0;
+  return g.nmain * (int64_t)sizeof(C) <= mb << 20;
+}
+
+// Whether the x-pass runs with a wavefront per field: where a grid has few
+// lines, and at any size where the kernel it replaces has too many registers
+// for the wavefronts it needs in flight (FP64 DNS, the scalar).  Rows of 8
+// entries have no use for it.  us per step as above: DNS FP32 512x16x64 105/99,
+// 128^3 (8 MB a field) 218/211, 256x64x256 505/525; LES FP32, with split_y,
+// 64^3 107/98, 128x64x64 (2 MB) 145/141, 256x32x64 150/155, 128x64x128 262/261;
+// LES FP64, with split_y, 128x64x64 (4 MB) 275/261, 64x64x256 574/593; DNS
+// FP64 64x64x256 209/195, 256x64x256 991/943; scalar FP32 512x256x64 2148/2076,
+// FP64 256x64x256 1977/1848.
+template <class R>
+bool Ops<R>::split_x(const scl_plan3d& pl, int les, int sc) {
+  const Geom& g = pl.g;
+  if (!pl.plane || g.mx < 16) return false;
+  const int64_t bytes = g.nmain * (int64_t)sizeof(C);
+  if (les) return sizeof(R) == 4 ? bytes <= 2 << 20 && g.mx <= 64 : bytes <= 4 << 20;
+  return sc || sizeof(R) == 8 || bytes <= 8 << 20;
+}
+
+template <class R>
+int32_t Ops<R>::yinv_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, const ForceArgs<R>& fa, R kc2) {
+  const Geom& g = pl.g;
+  const Cut<R> in = cut_of<R>(g, kc2);
+  return with_line<R>(g.ny, [&](auto NC) -> int32_t {
+    constexpr int N = decltype(NC)::value;
+    if constexpr (N <= 512) {
+      return with_layout(les, sc, [&](auto LC, auto SC) -> int32_t {
+        constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
+        using C2 = SplitY<R, N, LES, S>;
+        if (g.mx % C2::CW) return set_error("y-lines of %d: %d columns", g.ny, g.mx), SCL_EINVAL;
+        hipLaunchKernelGGL((k_yinv_split<R, N, LES, S>), dim3(ycut_grid<C2::CW>(g, in.nkx) + (fa.type ? 1 : 0)),
+                           dim3(64 * C2::NF), 0, pl.stream, W, fs, g, twp<R>(pl), pl.L / N, in, fa);
+        return check_launch("yinv_split");
+      });
+    } else {
+      return set_error("y-lines of %d points: no wavefront holds one", g.ny), SCL_EINVAL;
+    }
+  });
+}
+
+template <class R>
+int32_t Ops<R>::yfwd_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R sg) {
+  const Geom& g = pl.g;
+  return with_line<R>(g.ny, [&](auto NC) -> int32_t {
+    constexpr int N = decltype(NC)::value;
+    if constexpr (N <= 512) {
+      return with_layout(les, sc, [&](auto LC, auto SC) -> int32_t {
+        constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
+        using C2 = SplitY<R, N, LES, S>;
+        if (g.mx % C2::CW) return set_error("y-lines of %d: %d columns", g.ny, g.mx), SCL_EINVAL;
+        hipLaunchKernelGGL((k_yfwd_split<R, N, LES, S>), dim3(col_grid<C2::CW, 1>(g)), dim3(64 * C2::KINDS), 0,
+                           pl.stream, W, fs, g, sg, twp<R>(pl), pl.L / N);
+        return check_launch("yfwd_split");
+      });
+    } else {
+      return set_error("y-lines of %d points: no wavefront holds one", g.ny), SCL_EINVAL;
+    }
+  });
+}
+
+template <class R>
+int32_t Ops<R>::row_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, const double* cs2p,
+                          C* tape, R kc2_in, R kc2_out) {
+  const Geom& g = pl.g;
+  const int kin = cut_of<R>(g, kc2_in).nkx, kout = cut_of<R>(g, kc2_out).nkx;
+  return with_half<R>(g.mx, [&](auto MC) -> int32_t {
+    constexpr int M = decltype(MC)::value;
+    return with_layout(les, sc, [&](auto LC, auto SC) -> int32_t {
+      constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
+      using C2 = SplitX<R, M, LES, S>;
+      if (g.nrow % C2::RW) return set_error("%lld rows: not whole groups of %d", (long long)g.nrow, C2::RW), SCL_EINVAL;
+      hipLaunchKernelGGL((k_row_split<R, M, LES, S>), dim3((unsigned)(g.nrow / C2::RW)), dim3(64 * C2::NF), 0,
+                         pl.stream, W, fs, g, scale, d2, cs2p, tape, twp<R>(pl), pl.L / M, pl.L / g.nx, kin, kout);
+      return check_launch("row_split");
+    });
+  });
 }
 
 template <class R>

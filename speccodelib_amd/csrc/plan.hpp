@@ -24,7 +24,8 @@ struct scl_plan3d {
   // y-lines, where those kernels spill)
   bool zfused = true;
   // the y- and x-passes of a RHS in one launch where the planes fit in LDS
-  // (Ops::plane_fits); SCL_PLANE=0 at plan creation: the separate passes
+  // (Ops::plane_fits), with a wavefront per field where that is faster
+  // (Ops::split_y, split_x); SCL_PLANE=0 at plan creation: neither
   bool plane = true;
   hipStream_t stream = nullptr;
   bool own_stream = false;

@@ -19,6 +19,9 @@
 
 namespace scl {
 
+// The wavefront's number in its workgroup, known to the compiler as uniform.
+__device__ inline int wave_index() { return __builtin_amdgcn_readfirstlane(threadIdx.x / 64); }
+
 // NP planes: the largest number live at once.
 //   DNS          u(3) w(3)
 //   scalar       u(3) w(3) phi, then N(3) F(3)
@@ -54,6 +57,11 @@ struct PlaneCfg {
   // not: 527/411.
   static constexpr bool fits = TY <= 32 && TX >= 1 && TX <= 16 && (size_t)LDS * sizeof(cpx<R>) <= 160 * 1024 &&
                                !((LES || SC) && NY >= 128 && NP * X1 * NY > 12000);
+  // FP32 with a scalar or the Smagorinsky term: where one workgroup fills a CU's
+  // LDS and there are as many as CUs, solvers running side by side are faster
+  // with the separate passes (64x64 planes, scalar: 128 of them 133/123, 256
+  // 214/247; 64x32, LES and scalar: 64 of them 137/92, 256 205/251).
+  static constexpr int max_nz = sizeof(R) == 4 && (LES || SC) && LDS * 8 > 100 * 1024 ? 128 : 1024;
 };
 
 // What the y-inverse of output field f transforms: (i (ax kx + ay ky) + a0) A +
@@ -134,7 +142,7 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
     twM[i] = tw[i * (L / M)];
     twN[i] = tw[i * (L / g.nx)];
   }
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int wave = wave_index(), lane = threadIdx.x % 64;
   const int z = blockIdx.x;
   __syncthreads();
 
@@ -408,6 +416,245 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
       }
     }
   }
+}
+
+// --------------------------------------------------------------------------
+// The same passes one axis at a time, a wavefront per field.  Where a grid has
+// few lines, a pass whose wavefronts take all fields' transforms one after the
+// other leaves most of the chip's wavefront slots empty and takes as long as
+// its chain of transforms: at 64^3 the LES x-pass was 256 wavefronts with 21
+// transforms each, 25 us.  Here a workgroup has a wavefront per field, all
+// fields' transforms run side by side, and the products pass through LDS.
+// --------------------------------------------------------------------------
+
+// YINV of all the fields of a RHS (plane_form), in place: all wavefronts of
+// the workgroup have read their columns before any writes.  One workgroup more
+// than there are tiles computes the forcing coefficients (fa.type).  in: as
+// k_colfft's.
+template <class R, int NY, int LES, int SC>
+struct SplitY {
+  static constexpr int TY = NY / 8, CW = 64 / TY;
+  static constexpr int NF = 6 + 6 * LES + SC;     // y-inverse: fields
+  static constexpr int KINDS = 3 + LES + 2 * SC;  // y-forward: tasks of a tile
+  static constexpr int LINE = lds_pad(NY) * CW;   // LDS entries of a wavefront
+};
+
+template <class R, int NY, int LES, int SC>
+__global__ __launch_bounds__((64 * SplitY<R, NY, LES, SC>::NF)) void k_yinv_split(cpx<R>* W, int64_t fs, Geom g,
+                                                                               const cpx<R>* __restrict__ tw, int tws,
+                                                                               Cut<R> in, ForceArgs<R> fa) {
+  using C = SplitY<R, NY, LES, SC>;
+  constexpr int CW = C::CW, TY = C::TY;
+  constexpr PlaneForm F = plane_form<LES, SC>();
+  __shared__ cpx<R> sh[C::NF * C::LINE];
+  __shared__ cpx<R> twl[NY];
+  if (fa.type && blockIdx.x + 1 == gridDim.x) {
+    force_coef_block<R>(fa, fs, g, reinterpret_cast<double(*)[256]>(sh));
+    return;
+  }
+  for (int i = threadIdx.x; i < NY; i += 64 * C::NF) twl[i] = tw[i * tws];
+  const int f = wave_index(), lane = threadIdx.x % 64;
+  const int c = lane % CW, yr = lane / CW;
+  const int tiles = gridDim.x - (fa.type ? 1 : 0);
+  Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, tiles), c, ycut_tiles<CW>(g, in.nkx));
+  if (t.kx >= in.nkx) t.ok = false;
+  const R kx = (R)t.kx;
+  auto digit = [&](uint32_t d) { return (R)((int)((d >> (2 * f)) & 3u) - 1); };
+  const R a0 = digit(F.a0), b0 = digit(F.b0), ay = digit(F.ay), by = digit(F.by);
+  const R akx = digit(F.ax) * kx, bkx = digit(F.bx) * kx;
+  const R h = ((F.half >> f) & 1u) ? (R)0.5 : (R)1;
+  const cpx<R>* const A = W + (int)((F.qa >> (4 * f)) & 15u) * fs;
+  const cpx<R>* const B = W + (int)((F.qb >> (4 * f)) & 15u) * fs;
+  auto load = [&](cpx<R>(&a)[8], const cpx<R>* w) {
+    if (in.all()) {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) a[m] = t.ok ? w[t.off(yr + TY * m)] : mk<R>(0, 0);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        const int j = yr + TY * m;
+        a[m] = ld_or_zero(w, t.off(j), t.base, t.ok && !col_cut<R>(t.kx, kwave(j, NY), in.kc2));
+      }
+    }
+  };
+  cpx<R> v[8];
+  load(v, A);
+  if (LES ? (f >= 3 && f < 11) : (!SC && f == 5)) {  // the others are taken as they are
+    cpx<R> b[8];
+    load(b, B);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const R ky = (R)kwave(yr + TY * m, NY);
+      const R ka = akx + ay * ky, kb = bkx + by * ky;
+      v[m] = mk<R>(h * (a0 * v[m].x - ka * v[m].y + (b0 * b[m].x - kb * b[m].y)),
+                   h * (a0 * v[m].y + ka * v[m].x + (b0 * b[m].y + kb * b[m].x)));
+    }
+  }
+  __syncthreads();
+  using Ln = Line<R, NY, 8, +1, true>;
+  Ln::run(v, sh + f * C::LINE, yr, twl, 1, ColIdx<CW>{c});
+  if (!t.ok) return;
+  cpx<R>* const O = W + f * fs;
+#pragma unroll
+  for (int m = 0; m < 8; ++m) O[t.off(Ln::out_pos(m, yr))] = v[m];
+}
+
+// YFWD of the outputs of the LES / scalar x-pass with the kx, ky terms folded:
+// the fields and slots of k_yfwd_ext, the tasks of k_plane's y-forward, one a
+// wavefront.
+template <class R, int NY, int LES, int SC>
+__global__ __launch_bounds__((64 * SplitY<R, NY, LES, SC>::KINDS)) void k_yfwd_split(cpx<R>* W, int64_t fs, Geom g,
+                                                                                  R sg,
+                                                                                  const cpx<R>* __restrict__ tw,
+                                                                                  int tws) {
+  using C = SplitY<R, NY, LES, SC>;
+  constexpr int CW = C::CW, TY = C::TY;
+  constexpr ExtLayout X{LES, SC};
+  constexpr int t0 = X.tau_out(), f0 = X.flux_out();
+  __shared__ cpx<R> sh[C::KINDS * C::LINE];
+  __shared__ cpx<R> twl[NY];
+  for (int i = threadIdx.x; i < NY; i += 64 * C::KINDS) twl[i] = tw[i * tws];
+  const int kind = wave_index(), lane = threadIdx.x % 64;
+  const int c = lane % CW, yr = lane / CW;
+  const Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, gridDim.x), c);
+  const R kx = (R)t.kx;
+  using Lf = Line<R, NY, 8, -1, true>;
+  cpx<R>* const ex = sh + kind * C::LINE;
+  auto load = [&](cpx<R>(&v)[8], int q) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) v[m] = t.ok ? (W + q * fs)[t.off(yr + TY * m)] : mk<R>(0, 0);
+  };
+  auto run = [&](cpx<R>(&v)[8]) { Lf::run(v, ex, yr, twl, 1, ColIdx<CW>{c}); };
+  auto store = [&](const cpx<R>(&v)[8], int q) {
+    if (!t.ok) return;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) (W + q * fs)[t.off(Lf::out_pos(m, yr))] = v[m];
+  };
+  auto ky = [&](int m) { return (R)kwave(Lf::out_pos(m, yr), NY); };
+  // inputs: N_i or F_x in a, the field of the ky term in b, of the kx term in d
+  const bool les = LES != 0 && kind < 3, flux = SC != 0 && kind == C::KINDS - 2;
+  const int i = les ? (kind + 2) % 3 : kind;  // i = 3 first, the longest
+  const int qa = kind < 3 ? i : LES != 0 && kind == 3 ? t0 + 5 : flux ? f0 : f0 + 2;
+  // tau_i1, tau_i2: 11 12, 12 22, 13 23
+  const int qd = t0 + (i == 0 ? 0 : i == 1 ? 1 : 2), qb = les ? t0 + (i == 0 ? 1 : i == 1 ? 3 : 4) : f0 + 1;
+  cpx<R> a[8], b[8], d[8];
+  load(a, qa);
+  if (les || flux) load(b, qb);
+  if (les) load(d, qd);
+  __syncthreads();
+  if (les) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) a[m] = a[m] - mul_i(kx * d[m]);
+  } else if (flux) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) a[m] = sg * mul_i(kx * a[m]);
+  }
+  run(a);
+  if (les || flux) {
+    run(b);
+    const R s = les ? (R)-1 : sg;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) a[m] = a[m] + s * mul_i(ky(m) * b[m]);
+  }
+  store(a, qa);
+  if (les && i == 2) {
+    store(b, qb);  // tau_23
+    run(d);
+    store(d, qd);  // tau_13
+  }
+}
+
+// XPASS with the products of k_row_convec / k_row_ext, a wavefront per field.
+// A wavefront holds 512/M rows of its field, every wavefront's lane the same
+// points, so the physical values pass through LDS as [field][slot][lane].
+// kin, kout, tape: as k_row_convec (k_row_ext: all).
+template <class R, int M, int LES, int SC>
+struct SplitX {
+  static constexpr int TX = M / 8, RW = 64 / TX;
+  static constexpr int NF = 6 + 6 * LES + SC;
+  static constexpr int LINE = lds_pad(M) * RW;
+};
+
+template <class R, int M, int LES, int SC>
+__global__ __launch_bounds__((64 * SplitX<R, M, LES, SC>::NF)) void k_row_split(
+    cpx<R>* W, int64_t fs, Geom g, R scale, R d2, const double* __restrict__ cs2p, cpx<R>* __restrict__ tape,
+    const cpx<R>* __restrict__ tw, int twsM, int twsN, int kin, int kout) {
+  using C = SplitX<R, M, LES, SC>;
+  constexpr int TX = C::TX, RW = C::RW, LINE = C::LINE;
+  constexpr ExtLayout X{LES, SC};
+  __shared__ cpx<R> sh[C::NF * LINE];
+  __shared__ cpx<R> twM[M], twN[M];
+  for (int i = threadIdx.x; i < M; i += 64 * C::NF) {
+    twM[i] = tw[i * twsM];
+    twN[i] = tw[i * twsN];
+  }
+  const int f = wave_index(), lane = threadIdx.x % 64;
+  const int slot = lane / TX, rt = lane % TX;
+  const int64_t row = (int64_t)blockIdx.x * RW + slot;
+  cpx<R>* const own = sh + f * LINE;
+  cpx<R>* const ex = own + slot * lds_pad(M);
+  cpx<R> v[8], raw[8];
+  {
+    const cpx<R>* const base = W + f * fs;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int k = rt + TX * m;
+      raw[m] = ld_or_zero(base, row * M + k, row * M, k < kin);
+    }
+    const cpx<R> xm = rt == 0 && M < kin ? base[g.nmain + row] : mk<R>(0, 0);
+    __syncthreads();  // the twiddles
+    row_c2r_prep<R, M>(v, raw, xm, rt, twN, 1);
+  }
+  using Li = Line<R, M, 8, +1, true>;
+  Li::run(v, ex, rt, twM, 1, LinIdx{});
+  if (tape && f < 6 + 6 * LES) {
+    cpx<R>* const tb = tape + f * fs + row * M;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) tb[Li::out_pos(m, rt)] = v[m];
+  }
+#pragma unroll
+  for (int m = 0; m < 8; ++m) own[m * 64 + lane] = v[m];
+  __syncthreads();
+  // the products: N by the wavefronts of u, the fluxes by those of w, tau_ij
+  // by those of S_ij
+  auto at = [&](int q, int m) { return sh[q * LINE + m * 64 + lane]; };
+  int q = -1;  // the output field
+  if (f < 3) {
+    const int j1 = (f + 1) % 3, j2 = (f + 2) % 3;
+    q = f;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const cpx<R> u1 = at(j1, m), u2 = at(j2, m), w1 = at(3 + j1, m), w2 = at(3 + j2, m);
+      v[m] = mk<R>((u1.x * w2.x - u2.x * w1.x) * scale, (u1.y * w2.y - u2.y * w1.y) * scale);
+    }
+  } else if (SC != 0 && f < 6) {
+    q = X.flux_out() + f - 3;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const cpx<R> u = at(f - 3, m), ph = at(X.phi_in(), m);
+      v[m] = mk<R>(u.x * ph.x * scale, u.y * ph.y * scale);
+    }
+  } else if (LES != 0 && f >= 6 && f < 12) {
+    q = X.tau_out() + f - 6;
+    const R cs = (R)(-2.0 * cs2p[0]) * d2 * scale;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      R sx[6], sy[6];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        const cpx<R> s = at(6 + k, m);
+        sx[k] = s.x;
+        sy[k] = s.y;
+      }
+      v[m] = mk<R>(cs * abs_strain<R>(sx) * v[m].x, cs * abs_strain<R>(sy) * v[m].y);
+    }
+  }
+  __syncthreads();  // all products are read
+  if (q < 0) return;
+  using Lf = Line<R, M, 8, -1, true>;
+  Lf::run(v, ex, rt, twM, 1, LinIdx{});
+  cpx<R>* const o = W + q * fs;
+  row_r2c_post<R, M, true>(v, o + row * M, o + g.nmain + row, rt, twN, 1, kout);
 }
 
 }  // namespace scl

@@ -18,6 +18,9 @@ struct DevFields {
   double* coef = nullptr;
   void* s_out = nullptr;
   void* phys_out = nullptr;  // the x-pass keeps u, w [, S_ij] in physical space here (adjoint tape)
+  // the y- and x-passes in their separate form at every size, to the bit what
+  // they give there (plan.hpp's plane off)
+  bool separate = false;
   unsigned* nonfinite = nullptr;  // sticky flag: stage 4 found a non-finite v (null: not checked)
   template <class R>
   cpx<R>* f(int i) const {

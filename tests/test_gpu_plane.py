@@ -1,5 +1,6 @@
-"""The y- and x-passes of a RHS in one launch (planes that fit in LDS) against
-the separate passes, over plane shapes, precisions and solver options.
+"""The y- and x-passes of a RHS in one launch (planes that fit in LDS) and with
+a wavefront per field (larger ones) against the separate passes, over plane
+shapes, precisions and solver options.
 
 The two differ in rounding only: the bars are those the steps have against the
 oracle elsewhere (FP64 1e-11, FP32 1e-5 of the largest entry)."""
@@ -67,6 +68,26 @@ def test_les_and_scalar_planes(monkeypatch, plane, prec, sgs, scalar):
             grad=1.0 if scalar else 0.0, schmidt=0.7)
 
 
+LINES = [(64, 128, 16), (32, 256, 16), (16, 512, 16), (32, 512, 16), (128, 64, 16), (512, 16, 16), (1024, 16, 16),
+         (128, 128, 32)]
+
+
+@pytest.mark.parametrize("prec", [scl.SP, scl.DP])
+@pytest.mark.parametrize("shape", LINES)
+@pytest.mark.parametrize("sgs,scalar", [(0, False), (1, False), (0, True), (1, True)])
+def test_wavefront_per_field(monkeypatch, shape, prec, sgs, scalar):
+    compare(monkeypatch, shape, prec, forced=2 if not (sgs or scalar) else 1, sgs=sgs, cs2=0.03 if sgs else 0.0,
+            scalar=scalar, grad=1.0 if scalar else 0.0, schmidt=0.7)
+
+
+# (32, 64, 512) and (32, 512, 64) with a radius above nx/2: every kx is kept, not every column
+@pytest.mark.parametrize("shape", [(64, 128, 16), (64, 128, 128), (256, 64, 64), (32, 64, 512), (32, 512, 64)])
+@pytest.mark.parametrize("prec", [scl.SP, scl.DP])
+@pytest.mark.parametrize("kw", [dict(), dict(dealias_rhs=True), dict(stepper=1, kcut=31.0), dict(kcut=20.5)])
+def test_truncated_lines(monkeypatch, shape, prec, kw):
+    compare(monkeypatch, shape, prec, steps=5, forced=1, **kw)
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(dealias_rhs=True), dict(stepper=1, kcut=31.0), dict(stepper=2)])
 def test_truncated_and_ab2_steps(monkeypatch, kw):
     compare(monkeypatch, (64, 64, 128), scl.SP, steps=5, forced=1, **kw)
@@ -78,8 +99,9 @@ def test_radius_above_half_nx(monkeypatch):
 
 
 @pytest.mark.parametrize("sgs", [0, 1])
-def test_blocked_row_order(monkeypatch, sgs):
-    compare(monkeypatch, (32, 32, 32), scl.DP, zblock=8, forced=1, sgs=sgs, cs2=0.03 if sgs else 0.0)
+@pytest.mark.parametrize("shape", [(32, 32, 32), (64, 128, 16)])
+def test_blocked_row_order(monkeypatch, shape, sgs):
+    compare(monkeypatch, shape, scl.DP, zblock=8, forced=1, sgs=sgs, cs2=0.03 if sgs else 0.0)
 
 
 @pytest.mark.parametrize("prec", [scl.SP, scl.DP])
@@ -97,14 +119,15 @@ def test_rates_of_host_arrays(monkeypatch, prec):
 
 
 @pytest.mark.parametrize("sgs", [0, 1])
-def test_adjoint_tape(monkeypatch, sgs):
+@pytest.mark.parametrize("shape", [(32, 32, 16), (64, 128, 16)])
+def test_adjoint_tape(monkeypatch, shape, sgs):
     """Gradients with the physical tape written by either kernel (FP64)."""
-    v = state(32, 32, 16, 3)
-    g = state(32, 32, 16, 3, seed=2)
+    v = state(*shape, 3)
+    g = state(*shape, 3, seed=2)
     out = []
     for plane in ("0", "1"):
         monkeypatch.setenv("SCL_PLANE", plane)
-        p = scl.Plan3D(32, 32, 16, scl.DP)
+        p = scl.Plan3D(*shape, scl.DP)
         a = scl.Adjoint(p, 4, 2, nu=0.02, dt=1e-3, sgs=sgs)
         a.forward(v, 0.03 if sgs else 0.0)
         out.append(a.backward(g))
