@@ -733,11 +733,15 @@ static int32_t ab2_step_dev(scl_plan3d* p, const DevFields& d, const scl_dns_par
   return ab_end(p, ab);
 }
 
+// Whether LES / scalar steps leave out the modes beyond the truncation.
+static bool ext_trunc(const scl_plan3d* p) { return trunc_pays(p) && p->zfused; }
+
 // The LES and/or scalar RHS (multi-pass) for stage `mode` (IF-RK4 1..4,
-// IF-AB2 5..7 with the weights in ab).
+// IF-AB2 5..7 with the weights in ab).  vcut: v is zero beyond the truncation
+// (a step has left it so).
 template <class R>
 static int32_t rk_stage_ext(scl_plan3d* p, const DevFields& d, int mode, const scl_dns_params& prm, const cpx<R>* st,
-                            Timer* tm, const double* ab = nullptr) {
+                            Timer* tm, const double* ab = nullptr, bool vcut = false) {
   const int64_t fs = d.fs;
   Timer none;
   if (!tm) tm = &none;
@@ -747,6 +751,10 @@ static int32_t rk_stage_ext(scl_plan3d* p, const DevFields& d, int mode, const s
   apply_kcut<R>(ep.r, prm);
   ep.r.nonfinite = d.nonfinite;
   ep.r.ab = ab;
+  ep.r.trunc = mode > 0 && ext_trunc(p) && !d.separate;
+  ep.r.vcut = ep.r.trunc && vcut;
+  // only stage 1 and the AB2 steps read the state itself
+  const R kc2_in = !ep.r.trunc || (mode > 1 && mode < 5) ? (R)0 : ep.r.vcut ? ep.r.kc2 : std::numeric_limits<R>::infinity();
   ep.nu_phi = (R)(prm.nu / (prm.schmidt > 0 ? prm.schmidt : 1.0));
   ep.grad = (R)prm.grad;
   ep.sign_phi = 1;
@@ -755,7 +763,7 @@ static int32_t rk_stage_ext(scl_plan3d* p, const DevFields& d, int mode, const s
   SCL_CHECK(ExtOps<R>::rhs(*p, mode, L, d.W<R>(), fs, d.V<R>(), d.DU<R>(), d.S<R>(), st, d.coef, ep,
                            (R)(delta * delta), reinterpret_cast<cpx<R>*>(d.phys_out),
                            force_args<R>(st, prm.fkmax, prm.eps, prm.eta, prm.forced, d.coef),
-                           [&] { tm->mark(SCL_K_ZFWD); }, d.separate));
+                           [&] { tm->mark(SCL_K_ZFWD); }, d.separate, kc2_in));
   // the kx = 0 Hermitian copy: as in rk_stage
   if (mode >= 1 && mode < 4 && !d.s_out) {
     tm->mark(-1);
@@ -1013,7 +1021,7 @@ extern "C" int32_t scl_dns_set_velocity(scl_dns* d, const void* vx, const void* 
   if (!d) return set_error("null solver"), SCL_EINVAL;
   const void* vi[3] = {vx, vy, vz};
   SCL_CHECK(clear_nonfinite(d));
-  d->chained = false;
+  d->chained = d->truncated = false;
   SCL_CHECK(ab_reset(d));
   return dns_io(d, 0, 3, vi, nullptr);
 }
@@ -1028,6 +1036,7 @@ extern "C" int32_t scl_dns_set_scalar(scl_dns* d, const void* phi) {
   if (!d || d->nc < 4) return set_error("solver has no scalar"), SCL_EINVAL;
   const void* vi[1] = {phi};
   SCL_CHECK(clear_nonfinite(d));
+  d->truncated = false;
   SCL_CHECK(ab_reset(d));
   return dns_io(d, 3, 1, vi, nullptr);
 }
@@ -1079,6 +1088,8 @@ static int32_t dns_step_once(scl_dns* d, Timer* tm) {
     return SCL_OK;
   }
   const scl_dns_params& prm = d->p;
+  const bool vcut = d->truncated;
+  d->truncated = false;  // until the step is queued whole
   if (prm.sgs == 2 && d->steps % (prm.iupdate > 0 ? prm.iupdate : 1) == 0) {
     const double delta = prm.delta > 0 ? prm.delta : 2.0 * M_PI / p->g.nx;
     const double dtest = prm.delta_test > 0 ? prm.delta_test : 2.0 * delta;
@@ -1090,15 +1101,17 @@ static int32_t dns_step_once(scl_dns* d, Timer* tm) {
     // LES / scalar passes with the AB2 combine
     SCL_CHECK(ab_begin<R>(p, f, prm, d->ab, d->ab_part));
     const int mode = d->ab_steps == 0 ? 5 : d->ab_steps == 1 ? 6 : 7;
-    SCL_CHECK(rk_stage_ext<R>(p, f, mode, prm, f.V<R>(), tm, d->ab));
+    SCL_CHECK(rk_stage_ext<R>(p, f, mode, prm, f.V<R>(), tm, d->ab, vcut));
     SCL_CHECK(ab_end(p, d->ab));
     d->ab_steps += 1;
+    d->truncated = true;
     return SCL_OK;
   }
   for (int stage = 1; stage <= 4; ++stage) {
     const cpx<R>* st = stage == 1 ? f.V<R>() : f.S<R>();
-    SCL_CHECK(rk_stage_ext<R>(p, f, stage, prm, st, tm));
+    SCL_CHECK(rk_stage_ext<R>(p, f, stage, prm, st, tm, nullptr, vcut));
   }
+  d->truncated = true;
   return SCL_OK;
 }
 
@@ -1111,7 +1124,8 @@ static int32_t dns_launch_steps(scl_dns* d, int nsteps, Timer* tm) {
     // chain and takes v as it was given, not truncated; the captured step is
     // the chained one.  IF-AB2: so do the two bootstrap steps; the captured
     // step is the Adams-Bashforth one
-    while (nsteps > 0 && ((d->p.stepper && d->ab_steps < 2) || (!d->ext && !d->chained))) {
+    while (nsteps > 0 && ((d->p.stepper && d->ab_steps < 2) || (!d->ext && !d->chained) ||
+                          (d->ext && ext_trunc(p) && !d->truncated))) {
       SCL_CHECK(dns_step_once<R>(d, nullptr));
       d->steps += 1;
       --nsteps;
@@ -1126,7 +1140,7 @@ static int32_t dns_launch_steps(scl_dns* d, int nsteps, Timer* tm) {
       int32_t st = dns_step_once<R>(d, nullptr);
       d->steps = keep;
       d->ab_steps = keep_ab;
-      if (st != SCL_OK) d->chained = false;
+      if (st != SCL_OK) d->chained = d->truncated = false;
       hipGraph_t gr = nullptr;
       hipError_t e = hipStreamEndCapture(p->stream, &gr);
       if (st != SCL_OK) {

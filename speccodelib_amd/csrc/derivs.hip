@@ -163,7 +163,7 @@ extern "C" int32_t scl_dns_state(scl_dns* d, void** state, int64_t* n) {
   if (!d || !state || !n) return set_error("null argument"), SCL_EINVAL;
   *state = d->fields;
   *n = (int64_t)d->nc * d->plan->fstride();
-  d->chained = false;  // the caller may change the state through the pointer
+  d->chained = d->truncated = false;  // the caller may change the state through the pointer
   return SCL_OK;
 }
 

@@ -32,15 +32,16 @@ struct ExtOps {
   // physical-space u, w, S_ij of this evaluation are kept (k_ext_phys).  fa:
   // the forcing coefficients the combine reads (type 0: there already, or not
   // forced).  begun(): called where the transforms start.  separate: as
-  // DevFields.
+  // DevFields.  kc2_in: the truncation st is known to have (infinite: it may
+  // have one in another step; 0: none); ep.r.trunc: as RhsParams.
   static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
                      const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape = nullptr) {
-    return rhs(pl, mode, L, W, fs, V, DU, S, st, coef, ep, delta2, phys_tape, ForceArgs<R>{}, [] {});
+    return rhs(pl, mode, L, W, fs, V, DU, S, st, coef, ep, delta2, phys_tape, ForceArgs<R>{}, [] {}, false, (R)0);
   }
   template <class F>
   static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
                      const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape, const ForceArgs<R>& fa,
-                     F&& begun, bool separate = false) {
+                     F&& begun, bool separate, R kc2_in) {
     const Geom& g = pl.g;
     const bool plane = !separate && pl.zfused && Ops<R>::plane_fits(pl, L.les, L.scalar);
     const bool sy = !separate && pl.zfused && !plane && Ops<R>::split_y(pl, L.les, L.scalar);
@@ -49,12 +50,13 @@ struct ExtOps {
       SCL_CHECK(check_launch("force_coef"));
     }
     begun();
+    const R kc2_out = ep.r.trunc && (mode >= 4 || ep.r.dealias) ? ep.r.kc2 : (R)0;
     // 1024-point z- or y-lines keep the separate prep and combine: the
     // fused passes spill there
     const bool fused = pl.zfused;
     if (fused) {
       // prep fused into the z-inverse
-      SCL_CHECK(Ops<R>::ext_zinv(pl, st, W, fs, L));
+      SCL_CHECK(Ops<R>::ext_zinv(pl, st, W, fs, L, kc2_in));
     } else {
       hipLaunchKernelGGL((k_ext_prep<R>), grid_all(g), dim3(256), 0, pl.stream, st, W, fs, g, L);
       SCL_CHECK(check_launch("ext_prep"));
@@ -64,16 +66,18 @@ struct ExtOps {
     // physical products; y-forward
     const R scale = (R)1 / (R)((double)g.nx * g.ny * g.nz);
     if (plane) {
-      SCL_CHECK(Ops<R>::plane(pl, W, fs, L.les, L.scalar, scale, delta2, (R)(-ep.sign_phi), coef + 5, phys_tape, fa));
+      SCL_CHECK(Ops<R>::plane(pl, W, fs, L.les, L.scalar, scale, delta2, (R)(-ep.sign_phi), coef + 5, phys_tape, fa, kc2_in,
+                              kc2_out));
       return Ops<R>::ext_zfwd(pl, mode, W, fs, V, DU, S, st, coef, ep, L);
     }
-    if (sy) SCL_CHECK(Ops<R>::yinv_split(pl, W, fs, L.les, L.scalar, fa));
-    else if (fused) SCL_CHECK(Ops<R>::ext_yinv(pl, W, fs, L));
+    if (sy) SCL_CHECK(Ops<R>::yinv_split(pl, W, fs, L.les, L.scalar, fa, kc2_in));
+    else if (fused) SCL_CHECK(Ops<R>::ext_yinv(pl, W, fs, L, kc2_in));
     else SCL_CHECK(Ops<R>::colfft(pl, W, fs, L.nin(), 1, +1));
     if (!separate && Ops<R>::split_x(pl, L.les, L.scalar))
-      SCL_CHECK(Ops<R>::row_split(pl, W, fs, L.les, L.scalar, scale, delta2, coef + 5, phys_tape));
+      SCL_CHECK(Ops<R>::row_split(pl, W, fs, L.les, L.scalar, scale, delta2, coef + 5, phys_tape, kc2_in,
+                                  sy ? (R)0 : kc2_out));
     else
-      SCL_CHECK(Ops<R>::row_ext(pl, W, fs, L, scale, delta2, coef + 5, phys_tape));
+      SCL_CHECK(Ops<R>::row_ext(pl, W, fs, L, scale, delta2, coef + 5, phys_tape, kc2_in, sy ? (R)0 : kc2_out));
     if (sy) {
       SCL_CHECK(Ops<R>::yfwd_split(pl, W, fs, L.les, L.scalar, (R)(-ep.sign_phi)));
       return Ops<R>::ext_zfwd(pl, mode, W, fs, V, DU, S, st, coef, ep, L);
@@ -81,7 +85,7 @@ struct ExtOps {
     // fused: the y-forward folds the kx, ky terms and the z-forward the kz
     // terms and the combine; else plain passes and the combine kernel
     if (fused) {
-      SCL_CHECK(Ops<R>::ext_yfwd(pl, W, fs, L, (R)(-ep.sign_phi)));
+      SCL_CHECK(Ops<R>::ext_yfwd(pl, W, fs, L, (R)(-ep.sign_phi), kc2_out));
       return Ops<R>::ext_zfwd(pl, mode, W, fs, V, DU, S, st, coef, ep, L);
     }
     SCL_CHECK(Ops<R>::colfft(pl, W, fs, L.nout(), 1, -1));

@@ -262,7 +262,7 @@ int32_t Ops<R>::zfwd_rhs(const scl_plan3d& pl, int mode, C* W, int64_t fstride, 
 }
 
 template <class R>
-int32_t Ops<R>::ext_zinv(const scl_plan3d& pl, const C* st, C* W, int64_t fs, const ExtLayout& L) {
+int32_t Ops<R>::ext_zinv(const scl_plan3d& pl, const C* st, C* W, int64_t fs, const ExtLayout& L, R kc2) {
   const Geom& g = pl.g;
   return with_line<R>(g.nz, [&](auto NC) -> int32_t {
     constexpr int N = decltype(NC)::value;
@@ -271,55 +271,61 @@ int32_t Ops<R>::ext_zinv(const scl_plan3d& pl, const C* st, C* W, int64_t fs, co
     if constexpr (N >= 1024) {
       return set_error("fused LES z-pass: 1024-point lines take the unfused path"), SCL_EINVAL;
     } else {
-      hipLaunchKernelGGL((k_ext_zinv<R, N>), dim3(col_grid<CC::CW, 2>(g)), dim3(CC::BS), 0, pl.stream, st, W, fs, g, L,
-                         twp<R>(pl), pl.L / N);
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(col_grid<CC::CW, 2>(g)), dim3(CC::BS), 0, pl.stream, st, W, fs, g, L, twp<R>(pl),
+                           pl.L / N, kc2);
+      };
+      if (kc2 > 0) go(k_ext_zinv<R, N, true>);
+      else go(k_ext_zinv<R, N>);
       return check_launch("ext_zinv");
     }
   });
 }
 
 template <class R>
-int32_t Ops<R>::ext_yinv(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout& L) {
+int32_t Ops<R>::ext_yinv(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout& L, R kc2) {
   const Geom& g = pl.g;
-  if (!L.les) return colfft(pl, W, fs, L.nin(), 1, +1);
+  if (!L.les) return colfft(pl, W, fs, L.nin(), 1, +1, kc2);
   return with_line<R>(g.ny, [&](auto NC) -> int32_t {
     constexpr int N = decltype(NC)::value;
     using CC = ColCfg<R, N>;
     SCL_CHECK((check_cols<R, N>(g)));
-    const dim3 grd(col_grid<CC::CW, 1>(g)), blk(CC::BS);
-    hipLaunchKernelGGL((k_yinv_les<R, N, 0>), grd, blk, 0, pl.stream, W, fs, g, twp<R>(pl), pl.L / N);
-    SCL_CHECK(check_launch("yinv_les"));
-    hipLaunchKernelGGL((k_yinv_les<R, N, 1>), grd, blk, 0, pl.stream, W, fs, g, twp<R>(pl), pl.L / N);
-    SCL_CHECK(check_launch("yinv_les"));
+    const Cut<R> cut = cut_of<R>(g, kc2);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(ycut_grid<CC::CW>(g, cut.nkx)), dim3(CC::BS), 0, pl.stream, W, fs, g, twp<R>(pl),
+                         pl.L / N, cut);
+      return check_launch("yinv_les");
+    };
+    SCL_CHECK(kc2 > 0 ? go(k_yinv_les<R, N, 0, true>) : go(k_yinv_les<R, N, 0>));
+    SCL_CHECK(kc2 > 0 ? go(k_yinv_les<R, N, 1, true>) : go(k_yinv_les<R, N, 1>));
     // S_33 (= i kz u_z after the z-pass) and phi: a plain y-inverse
-    return colfft(pl, W + (L.s_in() + 5) * fs, fs, 1 + L.scalar, 1, +1);
+    return colfft(pl, W + (L.s_in() + 5) * fs, fs, 1 + L.scalar, 1, +1, kc2);
   });
 }
 
 template <class R>
-int32_t Ops<R>::ext_yfwd(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout& L, R sg) {
+int32_t Ops<R>::ext_yfwd(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout& L, R sg, R kc2) {
   const Geom& g = pl.g;
   return with_line<R>(g.ny, [&](auto NC) -> int32_t {
     constexpr int N = decltype(NC)::value;
     using CC = ColCfg<R, N>;
     SCL_CHECK((check_cols<R, N>(g)));
-    const dim3 grd(col_grid<CC::CW, 1>(g)), blk(CC::BS);
-    const cpx<R>* tw = twp<R>(pl);
-    const int tws = pl.L / N;
+    const Cut<R> cut = cut_of<R>(g, kc2);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(ycut_grid<CC::CW>(g, cut.nkx)), dim3(CC::BS), 0, pl.stream, W, fs, g, sg,
+                         twp<R>(pl), pl.L / N, cut);
+      return check_launch("yfwd_ext");
+    };
     if (!L.les && !L.scalar) return set_error("ext_yfwd: neither a Smagorinsky term nor a scalar"), SCL_EINVAL;
     if (L.les) {
-      if (L.scalar)
-        hipLaunchKernelGGL((k_yfwd_ext<R, N, 0, 1>), grd, blk, 0, pl.stream, W, fs, g, sg, tw, tws);
-      else
-        hipLaunchKernelGGL((k_yfwd_ext<R, N, 0, 0>), grd, blk, 0, pl.stream, W, fs, g, sg, tw, tws);
-      SCL_CHECK(check_launch("yfwd_ext"));
+      if (L.scalar) SCL_CHECK(kc2 > 0 ? go(k_yfwd_ext<R, N, 0, 1, true>) : go(k_yfwd_ext<R, N, 0, 1>));
+      else SCL_CHECK(kc2 > 0 ? go(k_yfwd_ext<R, N, 0, 0, true>) : go(k_yfwd_ext<R, N, 0, 0>));
     } else {
-      SCL_CHECK(colfft(pl, W, fs, 3, 1, -1));  // N alone
+      SCL_CHECK(colfft(pl, W, fs, 3, 1, -1, kc2));  // N alone
     }
     if (!L.scalar) return SCL_OK;
     // the flux slots are W[3..5] with or without the Smagorinsky term
-    hipLaunchKernelGGL((k_yfwd_ext<R, N, 1, 1>), grd, blk, 0, pl.stream, W, fs, g, sg, tw, tws);
-    return check_launch("yfwd_ext");
+    return kc2 > 0 ? go(k_yfwd_ext<R, N, 1, 1, true>) : go(k_yfwd_ext<R, N, 1, 1>);
   });
 }
 
@@ -337,15 +343,19 @@ int32_t Ops<R>::ext_zfwd(const scl_plan3d& pl, int mode, C* W, int64_t fs, C* V,
       const dim3 grd(col_grid<CC::CW, 2>(g)), blk(CC::BS);
       const cpx<R>* tw = twp<R>(pl);
       const int tws = pl.L / N;
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws);
+      };
+      const bool tr = ep.r.trunc;
       switch (mode) {
-        case 0: hipLaunchKernelGGL((k_ext_zfwd<R, N, 0>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
-        case 1: hipLaunchKernelGGL((k_ext_zfwd<R, N, 1>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
-        case 2: hipLaunchKernelGGL((k_ext_zfwd<R, N, 2>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
-        case 3: hipLaunchKernelGGL((k_ext_zfwd<R, N, 3>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
-        case 4: hipLaunchKernelGGL((k_ext_zfwd<R, N, 4>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
-        case 5: hipLaunchKernelGGL((k_ext_zfwd<R, N, 5>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
-        case 6: hipLaunchKernelGGL((k_ext_zfwd<R, N, 6>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
-        case 7: hipLaunchKernelGGL((k_ext_zfwd<R, N, 7>), grd, blk, 0, pl.stream, W, fs, V, DU, S, st, coef, ep, g, L, tw, tws); break;
+        case 0: go(k_ext_zfwd<R, N, 0>); break;
+        case 1: tr ? go(k_ext_zfwd<R, N, 1, true>) : go(k_ext_zfwd<R, N, 1>); break;
+        case 2: tr ? go(k_ext_zfwd<R, N, 2, true>) : go(k_ext_zfwd<R, N, 2>); break;
+        case 3: tr ? go(k_ext_zfwd<R, N, 3, true>) : go(k_ext_zfwd<R, N, 3>); break;
+        case 4: tr ? go(k_ext_zfwd<R, N, 4, true>) : go(k_ext_zfwd<R, N, 4>); break;
+        case 5: tr ? go(k_ext_zfwd<R, N, 5, true>) : go(k_ext_zfwd<R, N, 5>); break;
+        case 6: tr ? go(k_ext_zfwd<R, N, 6, true>) : go(k_ext_zfwd<R, N, 6>); break;
+        case 7: tr ? go(k_ext_zfwd<R, N, 7, true>) : go(k_ext_zfwd<R, N, 7>); break;
         default: set_error("bad mode %d", mode); return SCL_EINVAL;
       }
       return check_launch("ext_zfwd");
@@ -424,8 +434,9 @@ int32_t Ops<R>::row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape,
 
 template <class R>
 int32_t Ops<R>::row_ext(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout& L, R scale, R d2,
-                        const double* cs2p, C* tape) {
+                        const double* cs2p, C* tape, R kc2_in, R kc2_out) {
   const Geom& g = pl.g;
+  const int kin = cut_of<R>(g, kc2_in).nkx, kout = cut_of<R>(g, kc2_out).nkx;
   if (!L.les && !L.scalar) return set_error("row_ext: neither a Smagorinsky term nor a scalar"), SCL_EINVAL;
   return with_half<R>(g.mx, [&](auto MC) -> int32_t {
     constexpr int M = decltype(MC)::value;
@@ -441,13 +452,18 @@ int32_t Ops<R>::row_ext(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout&
       const int64_t groups = g.nrow / RC::RPW;
       const int64_t grid = std::min<int64_t>(groups, (int64_t)per_cu * pl.ncu);
       hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(RC::BS), 0, pl.stream, W, fs, g, scale, d2, cs2p, tape,
-                         twp<R>(pl), pl.L / M, pl.L / g.nx);
+                         twp<R>(pl), pl.L / M, pl.L / g.nx, kin, kout);
       return check_launch("row_ext");
     };
     if (tape) {
       if (L.les && L.scalar) return go(IC<0>{}, k_row_ext<R, M, 1, 1, true>);
       if (L.les) return go(IC<1>{}, k_row_ext<R, M, 1, 0, true>);
       return set_error("row_ext: the tape needs the Smagorinsky term"), SCL_EINVAL;
+    }
+    if (kc2_in > 0 || kc2_out > 0) {
+      if (L.les && L.scalar) return go(IC<5>{}, k_row_ext<R, M, 1, 1, false, true>);
+      if (L.les) return go(IC<6>{}, k_row_ext<R, M, 1, 0, false, true>);
+      return go(IC<7>{}, k_row_ext<R, M, 0, 1, false, true>);
     }
     if (L.les && L.scalar) return go(IC<2>{}, k_row_ext<R, M, 1, 1, false>);
     if (L.les) return go(IC<3>{}, k_row_ext<R, M, 1, 0, false>);

@@ -68,6 +68,9 @@ struct scl_dns {
   // by the last step's fused stage 4): the next step's stage 1 needs no
   // z-inverse pass.  Cleared whenever v or W change outside a step.
   bool chained = false;
+  // LES / scalar: the state is zero beyond the truncation (a step has left it
+  // so); cleared with chained
+  bool truncated = false;
   // IF-AB2 (p.stepper 1, 2): device state (AB_* slots), energy partials, and
   // the steps taken since the state was set (selects the bootstrap modes)
   double* ab = nullptr;
