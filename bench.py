@@ -35,31 +35,34 @@ def field_bytes(n):
 
 
 # Algorithmic HBM bytes per launch of these kernels, in units of F (one read
-# or write of a field counts F).  The forced-mode coefficient kernel and the
-# kx=0-plane Hermitian copy move O(N^2) bytes and count 0.
+# or write of a field counts F), averaged over a step's launches of the kind:
+# at the 2/3 radius 2/3 of the kx, 0.35 of the (kx, ky) columns and 0.155 of
+# the modes are kept, and du, v, stage 1's inputs and stage 4's outputs move
+# those only.  The forced-mode coefficient kernel and the kx=0-plane Hermitian
+# copy move O(N^2) bytes and count 0.
 KIND_BYTES_F = {
     "force_coef": 0.0,
     "zinv_vort": 8.0,    # read u (3), write u, w_x, w_y (5)
-    "y_inverse": 11.0,   # read 5, write 6 (w_z formed in the pass)
-    "x_pass": 9.0,       # read 6, write 3
-    "y_forward": 6.0,    # 3 fields read + written
+    "y_inverse": 9.7,    # read 5, write 6 (w_z formed in the pass); stage 1: 1.75 + 4
+    "x_pass": 8.25,      # read 6, write 3; stage 1: 4 + 3, stage 4: 6 + 2
+    "y_forward": 5.25,   # 3 fields read + written; stage 4: 2 + 1.05
     "zfwd_rk": 12.75,    # stages 1..4: 12, 15, 15, 9 (W, v, du in; du, S or v out)
     "herm_fix": 0.0,
     # z-forward + stage + z-inverse of the next stage state (stage chain):
-    # stages 1..3: 14, 17, 17 (W, v, du in; du and W[0..4] out)
-    "zfwd_zinv": 16.0,
-    # stage 4 + z-inverse of the new v for the next step: W and du in (3 + 3),
-    # v and W[0..4] out (3 + 5)
-    "zfwd4_zinv": 14.0,
+    # stages 1..3: 8.9, 9.4, 9.4 (W 3, v, du in; du and W[0..4] out)
+    "zfwd_zinv": 9.25,
+    # stage 4 + z-inverse of the new v for the next step: W and du in, v and
+    # W[0..4] out
+    "zfwd4_zinv": 3.7,
 }
 # The step model that the roofline fraction is priced against: one read +
 # write per axis pass (z-inverse 9, y-inverse 12, x-pass 9, y-forward 6;
 # z-forward + stage 12, 15, 15, 12).
 STEP_BYTES_F = 198.0
-# What these kernels move per step: 4 x (11 + 9 + 6) for the y-inverse,
+# What these kernels move per step: 4 x (9.7 + 8.25 + 5.25) for the y-inverse,
 # x-pass and y-forward, and the four z-forwards, each fused with the next
-# z-inverse (14 + 17 + 17, and 14 for stage 4 with the next step's): 166 F.
-IMPL_STEP_BYTES_F = 166.0
+# z-inverse (3 x 9.25, and 3.7 for stage 4 with the next step's): 124 F.
+IMPL_STEP_BYTES_F = 124.0
 
 
 def kind_bytes_f(kinds):
@@ -67,7 +70,6 @@ def kind_bytes_f(kinds):
     chaining the unfused z-forward is stage 4 only."""
     out = dict(KIND_BYTES_F)
     if kinds.get("zfwd_zinv", (0.0, 0))[1]:
-        out["zfwd_zinv"] = 16.0  # (14 + 17 + 17) / 3
         out["zfwd_rk"] = 9.0
     return out
 

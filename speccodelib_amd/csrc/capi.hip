@@ -577,7 +577,9 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
   if (!tm) tm = &none;
   const bool plane = Ops<R>::plane_fits(*p, 0, 0);
   const bool sy = !plane && Ops<R>::split_y(*p, 0, 0);
-  if (rp.forced && !plane && !sy) {
+  const bool sx = !plane && Ops<R>::split_x(*p, 0, 0);
+  const ForceArgs<R> fa = force_args<R>(st, fkmax, eps, eta, rp.forced, d.coef);
+  if (rp.forced && !plane && !sy && !sx) {
     tm->mark(SCL_K_FORCE);
     SCL_CHECK(Ops<R>::force_coef(*p, st, fs, fkmax, eps, eta, rp.forced, d.coef));
   }
@@ -590,17 +592,17 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
     tm->mark(SCL_K_XPASS);
     const Geom& g = p->g;
     SCL_CHECK(Ops<R>::plane(*p, W, fs, 0, 0, (R)1 / (R)((double)g.nx * g.ny * g.nz), (R)0, (R)0, nullptr, tape,
-                            force_args<R>(st, fkmax, eps, eta, rp.forced, d.coef), kc2_in, kc2_out));
+                            fa, kc2_in, kc2_out));
   } else {
     tm->mark(SCL_K_YINV);
     if (sy)
-      SCL_CHECK(Ops<R>::yinv_split(*p, W, fs, 0, 0, force_args<R>(st, fkmax, eps, eta, rp.forced, d.coef), kc2_in));
+      SCL_CHECK(Ops<R>::yinv_split(*p, W, fs, 0, 0, fa, kc2_in));
     else
       SCL_CHECK(Ops<R>::yinv_vort(*p, W, fs, kc2_in));
     tm->mark(SCL_K_XPASS);
-    if (Ops<R>::split_x(*p, 0, 0))
+    if (sx)
       SCL_CHECK(Ops<R>::row_split(*p, W, fs, 0, 0, (R)1 / (R)((double)p->g.nx * p->g.ny * p->g.nz), (R)0, nullptr, tape,
-                                  kc2_in, kc2_out));
+                                  kc2_in, kc2_out, sy ? ForceArgs<R>{} : fa));
     else
       SCL_CHECK(Ops<R>::row_convec(*p, W, fs, tape, kc2_in, kc2_out));
     tm->mark(SCL_K_YFWD);

@@ -67,7 +67,7 @@ struct Ops {
   static int32_t yinv_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, const ForceArgs<R>& fa,
                             R kc2 = 0);
   static int32_t row_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, const double* cs2p,
-                           C* tape, R kc2_in = 0, R kc2_out = 0);
+                           C* tape, R kc2_in = 0, R kc2_out = 0, const ForceArgs<R>& fa = ForceArgs<R>{});
   static int32_t yfwd_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R sg);
   static int32_t row_c2r(const scl_plan3d& pl, C* W, int64_t fstride, int nf);
   static int32_t row_r2c(const scl_plan3d& pl, C* W, int64_t fstride, int nf);

@@ -199,6 +199,9 @@ int32_t Ops<R>::zinv_vort(const scl_plan3d& pl, const C* s, int64_t sstride, C* 
   });
 }
 
+// The fused z-forward takes as long to compile as all the rest: it has
+// translation units of its own (SCL_OPS_ZFWD), and the others leave it out.
+#ifdef SCL_OPS_ZFWD
 template <class R>
 int32_t Ops<R>::zfwd_rhs(const scl_plan3d& pl, int mode, C* W, int64_t fstride, C* V, C* DU, C* S, const C* st,
                          const double* coef, const RhsParams<R>& p, bool fused) {
@@ -260,6 +263,8 @@ int32_t Ops<R>::zfwd_rhs(const scl_plan3d& pl, int mode, C* W, int64_t fstride, 
     return go(IC<ColCfg<R, N>::CW>{});
   });
 }
+
+#endif
 
 template <class R>
 int32_t Ops<R>::ext_zinv(const scl_plan3d& pl, const C* st, C* W, int64_t fs, const ExtLayout& L, R kc2) {
@@ -637,7 +642,7 @@ int32_t Ops<R>::yfwd_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int 
 
 template <class R>
 int32_t Ops<R>::row_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, const double* cs2p,
-                          C* tape, R kc2_in, R kc2_out) {
+                          C* tape, R kc2_in, R kc2_out, const ForceArgs<R>& fa) {
   const Geom& g = pl.g;
   const int kin = cut_of<R>(g, kc2_in).nkx, kout = cut_of<R>(g, kc2_out).nkx;
   return with_half<R>(g.mx, [&](auto MC) -> int32_t {
@@ -646,8 +651,9 @@ int32_t Ops<R>::row_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int s
       constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
       using C2 = SplitX<R, M, LES, S>;
       if (g.nrow % C2::RW) return set_error("%lld rows: not whole groups of %d", (long long)g.nrow, C2::RW), SCL_EINVAL;
-      hipLaunchKernelGGL((k_row_split<R, M, LES, S>), dim3((unsigned)(g.nrow / C2::RW)), dim3(64 * C2::NF), 0,
-                         pl.stream, W, fs, g, scale, d2, cs2p, tape, twp<R>(pl), pl.L / M, pl.L / g.nx, kin, kout);
+      hipLaunchKernelGGL((k_row_split<R, M, LES, S>), dim3((unsigned)(g.nrow / C2::RW) + (fa.type ? 1 : 0)),
+                         dim3(64 * C2::NF), 0, pl.stream, W, fs, g, scale, d2, cs2p, tape, twp<R>(pl), pl.L / M,
+                         pl.L / g.nx, kin, kout, fa);
       return check_launch("row_split");
     });
   });

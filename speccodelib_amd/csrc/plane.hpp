@@ -567,7 +567,8 @@ __global__ __launch_bounds__((64 * SplitY<R, NY, LES, SC>::KINDS)) void k_yfwd_s
 // XPASS with the products of k_row_convec / k_row_ext, a wavefront per field.
 // A wavefront holds 512/M rows of its field, every wavefront's lane the same
 // points, so the physical values pass through LDS as [field][slot][lane].
-// kin, kout, tape: as k_row_convec (k_row_ext: all).
+// kin, kout, tape: as k_row_convec (k_row_ext: all).  One workgroup more than
+// there are row groups computes the forcing coefficients (fa.type).
 template <class R, int M, int LES, int SC>
 struct SplitX {
   static constexpr int TX = M / 8, RW = 64 / TX;
@@ -578,12 +579,16 @@ struct SplitX {
 template <class R, int M, int LES, int SC>
 __global__ __launch_bounds__((64 * SplitX<R, M, LES, SC>::NF)) void k_row_split(
     cpx<R>* W, int64_t fs, Geom g, R scale, R d2, const double* __restrict__ cs2p, cpx<R>* __restrict__ tape,
-    const cpx<R>* __restrict__ tw, int twsM, int twsN, int kin, int kout) {
+    const cpx<R>* __restrict__ tw, int twsM, int twsN, int kin, int kout, ForceArgs<R> fa) {
   using C = SplitX<R, M, LES, SC>;
   constexpr int TX = C::TX, RW = C::RW, LINE = C::LINE;
   constexpr ExtLayout X{LES, SC};
   __shared__ cpx<R> sh[C::NF * LINE];
   __shared__ cpx<R> twM[M], twN[M];
+  if (fa.type && blockIdx.x + 1 == gridDim.x) {
+    force_coef_block<R>(fa, fs, g, reinterpret_cast<double(*)[256]>(sh));
+    return;
+  }
   for (int i = threadIdx.x; i < M; i += 64 * C::NF) {
     twM[i] = tw[i * twsM];
     twN[i] = tw[i * twsN];
