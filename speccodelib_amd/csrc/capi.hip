@@ -575,9 +575,10 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
   cpx<R>* W = d.W<R>();
   Timer none;
   if (!tm) tm = &none;
-  const bool plane = Ops<R>::plane_fits(*p, 0, 0);
-  const bool sy = !plane && Ops<R>::split_y(*p, 0, 0);
-  const bool sx = !plane && Ops<R>::split_x(*p, 0, 0);
+  const bool ab2 = mode >= 5;  // in the separate passes, over all modes (k_zfwd_ab2)
+  const bool plane = !ab2 && Ops<R>::plane_fits(*p, 0, 0);
+  const bool sy = !ab2 && !plane && Ops<R>::split_y(*p, 0, 0);
+  const bool sx = !ab2 && !plane && Ops<R>::split_x(*p, 0, 0);
   const ForceArgs<R> fa = force_args<R>(st, fkmax, eps, eta, rp.forced, d.coef);
   if (rp.forced && !plane && !sy && !sx) {
     tm->mark(SCL_K_FORCE);
@@ -585,7 +586,7 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
   }
   if (!primed) {
     tm->mark(SCL_K_ZINV);
-    SCL_CHECK(Ops<R>::zinv_vort(*p, st, fs, W, fs));
+    SCL_CHECK(Ops<R>::zinv_vort(*p, st, fs, W, fs, ab2));
   }
   cpx<R>* const tape = reinterpret_cast<cpx<R>*>(d.phys_out);
   if (plane) {
@@ -725,13 +726,13 @@ static int32_t ab2_step_dev(scl_plan3d* p, const DevFields& d, const scl_dns_par
   apply_kcut<R>(rp, prm);
   rp.nonfinite = d.nonfinite;
   rp.ab = ab;
-  rp.vcut = rp.trunc && primed;
+  rp.trunc = 0;
   Timer none;
   if (!tm) tm = &none;
   tm->mark(-1);
   SCL_CHECK(ab_begin<R>(p, d, prm, ab, ab_part));
   const int mode = istep == 0 ? 5 : istep == 1 ? 6 : 7;
-  SCL_CHECK(rk_stage<R>(p, d, mode, rp, prm.eps, prm.eta, prm.fkmax, d.V<R>(), tm, primed, true, rp.vcut));
+  SCL_CHECK(rk_stage<R>(p, d, mode, rp, prm.eps, prm.eta, prm.fkmax, d.V<R>(), tm, primed, true));
   return ab_end(p, ab);
 }
 

@@ -867,6 +867,230 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
   }
 }
 
+// The z-passes of the IF-AB2 steps (MODE 5..7; ab_apply), over all modes.  An
+// AB2 run of a field with energy up to its truncation multiplies any rounding
+// difference (8e-8 after 20 steps becomes 1e-5 and more within the next 20), so
+// these keep to the bit what the steps have always given; the passes that leave
+// modes out (k_zfwd_rhs<5..7>) made a 256^3 step 692 -> 622 us and moved such
+// runs by up to 3.5e-5.
+template <class R, int N, int E, int CW, bool PARK, int ZS>
+__device__ inline void zinv_store_all(cpx<R> (&ux)[E], cpx<R> (&uy)[E], cpx<R> (&uz)[E], cpx<R>* lds, cpx<R>* park,
+                                  const cpx<R>* twl, int rt, int c, R kx, R ky, int nz, ZOff<ZS> zo,
+                                  cpx<R>* __restrict__ w, int64_t ws) {
+  constexpr int T = N / E, BS = CW * T;
+  using L = Line<R, N, E, +1>;
+  // An empty asm that "changes" the base offset: the store addresses below
+  // are then recomputed here rather than kept live (and spilled) from the
+  // caller's loads of the same columns.
+  asm volatile("" : "+v"(zo.ob));
+  auto off = [&](int m) { return zo.at(rt + T * m); };
+  auto kz = [&](int m) { return (R)kwave(rt + T * m, nz); };
+  const int slot = rt * CW + c;
+  cpx<R> d[E];
+  L::run(uz, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    (w + 2 * ws)[off(m)] = uz[m];
+    if constexpr (PARK) park[m * BS + slot] = uz[m];
+  }
+  auto Uz = [&](int m) { return PARK ? park[m * BS + slot] : uz[m]; };
+#pragma unroll
+  for (int m = 0; m < E; ++m) d[m] = kz(m) * uy[m];
+  L::run(d, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+#pragma unroll
+  for (int m = 0; m < E; ++m) (w + 3 * ws)[off(m)] = mul_i(ky * Uz(m) - d[m]);
+  L::run(uy, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+#pragma unroll
+  for (int m = 0; m < E; ++m) (w + ws)[off(m)] = uy[m];
+#pragma unroll
+  for (int m = 0; m < E; ++m) d[m] = kz(m) * ux[m];
+  L::run(d, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+#pragma unroll
+  for (int m = 0; m < E; ++m) (w + 4 * ws)[off(m)] = mul_i(d[m] - kx * Uz(m));
+  L::run(ux, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+#pragma unroll
+  for (int m = 0; m < E; ++m) w[off(m)] = ux[m];
+}
+
+template <class R, int N, int CWZ, int EZ = 0, int ZS = 0>
+__global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zinv_all(const cpx<R>* __restrict__ s,
+                                                                     int64_t sstride, cpx<R>* __restrict__ w,
+                                                                     int64_t wstride, Geom g,
+                                                                     const cpx<R>* __restrict__ tw, int tws) {
+  using CC = ColCfg<R, N, CWZ, EZ>;
+  constexpr int CW = CC::CW, E = CC::E, T = CC::T;
+  constexpr bool PARK = CC::BS >= 1024 || (N >= 1024 && sizeof(R) == 4);
+  __shared__ cpx<R> lds[lds_pad(N) * CW];
+  __shared__ cpx<R> twl[N];  // this line length's twiddles; first read after a barrier
+  __shared__ cpx<R> park[PARK ? E * CC::BS : 1];
+  for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
+  const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
+  const Tile t = col_tile<CW, 2>(g, xcd_swizzle(blockIdx.x, gridDim.x), c);
+  const ZOff<ZS> zo = zoff<ZS>(t);
+  cpx<R> ux[E], uy[E], uz[E];
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const uint32_t o = zo.at(rt + T * m);
+    uz[m] = ld_once<R, (CW >= 16)>(s + o + 2 * sstride);
+    uy[m] = ld_once<R, (CW >= 16)>(s + o + sstride);
+    ux[m] = ld_once<R, (CW >= 16)>(s + o);
+  }
+  zinv_store_all<R, N, E, CW, PARK, ZS>(ux, uy, uz, lds, park, twl, rt, c, (R)t.kx, (R)kwave(t.oth, g.ny), g.nz, zo, w,
+                                    wstride);
+}
+
+template <class R, int N, int MODE, int CWZ, int EZ = 0, bool FUSED = false, int ZS = 0>
+__global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_ab2(cpx<R>* W, int64_t fstride, cpx<R>* V,
+                                                                    cpx<R>* DU, cpx<R>* S, const cpx<R>* st,
+                                                                    const double* __restrict__ coef, RhsParams<R> p,
+                                                                    Geom g, const cpx<R>* __restrict__ tw, int tws) {
+  using CC = ColCfg<R, N, CWZ, EZ>;
+  constexpr int CW = CC::CW, E = CC::E, T = CC::T;
+  __shared__ cpx<R> lds[lds_pad(N) * CW];
+  __shared__ cpx<R> twl[N];  // this line length's twiddles; first read after a barrier
+  for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
+  const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
+  const Tile t = col_tile<CW, 2>(g, xcd_swizzle(blockIdx.x, gridDim.x), c);
+  // 32-bit in-field offsets: the three components go through their own
+  // base pointers, so a thread keeps one 32-bit offset per slot instead of
+  // 64-bit ones (which spilled).
+  const ZOff<ZS> zo = zoff<ZS>(t);
+  cpx<R>* const W1 = W + fstride;
+  cpx<R>* const W2 = W + 2 * fstride;
+  // 1024-thread workgroups (and 1024-point lines) run one per CU, which
+  // leaves LDS to spare: the transformed x component waits there (each
+  // thread reads back only its own entries) instead of holding 2E registers
+  // through the other two transforms, and z is loaded after x is parked.
+  constexpr bool PARK = CC::BS >= 1024 || (N >= 1024 && sizeof(R) == 4);
+  __shared__ cpx<R> park[PARK ? E * CC::BS : 1];
+  cpx<R> nx_[E], ny_[E], nz_[E];
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const uint32_t o = zo.at(rt + T * m);
+    nx_[m] = ld_once<R, (CW >= 16)>(W + o);
+    ny_[m] = ld_once<R, (CW >= 16)>(W1 + o);
+    if constexpr (!PARK) nz_[m] = ld_once<R, (CW >= 16)>(W2 + o);
+  }
+  using L = Line<R, N, E, -1>;
+  L::run(nx_, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+  if constexpr (PARK) {
+    // offsets recomputed, not kept live through the transform above
+    ZOff<ZS> zn = zo;
+    asm volatile("" : "+v"(zn.ob));
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      park[m * CC::BS + threadIdx.x] = nx_[m];
+      nz_[m] = ld_once<R, (CW >= 16)>(W2 + zn.at(rt + T * m));
+    }
+  }
+  L::run(ny_, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+  // The stage update's loads (v, du or the AB2 history) of all three
+  // components of slot m are issued together, before any of the slot's
+  // stores: V, DU and S may alias as far as the compiler knows, so it would
+  // otherwise wait out one load round trip per component.
+  constexpr bool NT = CW >= 16;
+  auto stage_in = [&](int m, const ZOff<ZS>& zz, StageIn<R> (&dst)[3]) {
+    const int z = L::out_pos(m, rt);
+    const int iy = kwave(t.oth, g.ny), iz = kwave(z, g.nz);
+    const int ik2 = t.kx * t.kx + iy * iy + iz * iz;
+    // MODE 4 reads du only inside the cut
+    const bool cut = (ik2 == 0 ? std::numeric_limits<R>::min() : (R)ik2) >= p.kc2;
+    const uint32_t o = zz.at(z);
+    dst[0] = stage_load<MODE, R, uint32_t, NT>(o, V, DU, S, cut);
+    dst[1] = stage_load<MODE, R, uint32_t, NT>(o, V + fstride, DU + fstride, S + fstride, cut);
+    dst[2] = stage_load<MODE, R, uint32_t, NT>(o, V + 2 * fstride, DU + 2 * fstride, S + 2 * fstride, cut);
+  };
+  L::run(nz_, lds, opaque(rt), twl, 1, ColIdx<CW>{c});
+  // the epilogue recomputes its offsets (not kept live from the loads)
+  ZOff<ZS> ze = zo;
+  asm volatile("" : "+v"(ze.ob));
+
+  const int ikx = t.kx, iky = kwave(t.oth, g.ny);
+  const R kx = (R)ikx, ky = (R)iky;
+  const R tiny = std::numeric_limits<R>::min();
+  const bool plane_zero = (t.oth == g.ny / 2) || (t.kx == g.mx);
+  R fa = 0, fb = 0;
+  if (p.forced) {
+    fa = (R)coef[0];
+    fb = (R)coef[1];
+  }
+  R ab_dt = 0, ab_dto = 0, ab_s = 0, ab_ek = 0, ab_del = 0;
+  if constexpr (MODE >= 5) {
+    ab_dt = (R)p.ab[AB_DT];
+    ab_dto = (R)p.ab[AB_DTO];
+    ab_s = (R)p.ab[AB_S];
+    ab_ek = (R)p.ab[AB_EK];
+    ab_del = (R)p.ab[AB_DELTA];
+  }
+  // With the park, the new x stage state goes back to its park slot (just
+  // read) until the z-inverse, which keeps 2E registers free here.
+  auto keep_x = [&](int m, cpx<R> v) {
+    if constexpr (PARK && FUSED) park[m * CC::BS + threadIdx.x] = v;
+    else nx_[m] = v;
+  };
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    StageIn<R> in[3];
+    if constexpr (MODE > 0) stage_in(m, ze, in);
+    const int z = L::out_pos(m, rt);
+    const int ikz = kwave(z, g.nz);
+    const R kz = (R)ikz;
+    const int ik2 = ikx * ikx + iky * iky + ikz * ikz;
+    const R k2 = ik2 == 0 ? tiny : (R)ik2;
+    const uint32_t o = ze.at(z);
+    cpx<R> a = PARK ? park[m * CC::BS + threadIdx.x] : nx_[m], b = ny_[m], d = nz_[m];
+    // forcing (force.f90:25-29 / force_heli.f90:44-52)
+    if (p.forced && k2 < p.fk2) {
+      const cpx<R> sx = st[o], sy = st[fstride + o], sz = st[2 * fstride + o];
+      a = a + fa * sx;
+      b = b + fa * sy;
+      d = d + fa * sz;
+      if (p.forced == 2) {
+        a = a + fb * mul_i(ky * sz - kz * sy);
+        b = b + fb * mul_i(kz * sx - kx * sz);
+        d = d + fb * mul_i(kx * sy - ky * sx);
+      }
+    }
+    // symmetrize.f90:41-48: ky=-ny/2, kz=-nz/2, kx=nx/2 planes and the mean
+    if (plane_zero || z == g.nz / 2 || ik2 == 0) {
+      a = mk<R>(0, 0);
+      b = a;
+      d = a;
+    }
+    // projection.f90:16-30
+    {
+      const R den = kx * kx + ky * ky + kz * kz + tiny;
+      const cpx<R> q = mk<R>((kx * a.x + ky * b.x + kz * d.x) / den, (kx * a.y + ky * b.y + kz * d.y) / den);
+      a = a - kx * q;
+      b = b - ky * q;
+      d = d - kz * q;
+    }
+    if (p.dealias && k2 >= p.kc2) {
+      a = mk<R>(0, 0);
+      b = a;
+      d = a;
+    }
+    {
+      const R xk = -p.nu * k2;
+      const R e1 = expm1_r(xk * ab_dt);
+      const R e2 = MODE == 5 ? (R)0 : expm1_r(xk * ab_dto);
+      const bool cut = k2 >= p.kc2 || ik2 == 0;
+      keep_x(m, ab_apply<MODE, R>(in[0], a, o, V, DU, S, ab_dt, ab_s, ab_ek, ab_del, e1, e2, cut, p.nonfinite));
+      ny_[m] = ab_apply<MODE, R>(in[1], b, o, V + fstride, DU + fstride, S + fstride, ab_dt, ab_s, ab_ek, ab_del, e1,
+                                 e2, cut, p.nonfinite);
+      nz_[m] = ab_apply<MODE, R>(in[2], d, o, V + 2 * fstride, DU + 2 * fstride, S + 2 * fstride, ab_dt, ab_s, ab_ek,
+                                 ab_del, e1, e2, cut, p.nonfinite);
+    }
+  }
+  if constexpr (FUSED && MODE > 0) {
+    if constexpr (PARK) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) nx_[m] = park[m * CC::BS + threadIdx.x];
+    }
+    zinv_store_all<R, N, E, CW, PARK, ZS>(nx_, ny_, nz_, lds, park, twl, rt, c, kx, ky, g.nz, zo, W, fstride);
+  }
+}
+
 // Forcing coefficients from the stage state: a reduction over the box of
 // modes that can satisfy k2 < fk2 (force.f90:16-24, force_heli.f90:15-42),
 // accumulated in FP64 in a fixed order.  coef = {a, b, E_f, Omega_f, uw}.

@@ -20,7 +20,8 @@ struct Ops {
   // truncation k^2 < kc2 are there (inverse) or wanted (forward); infinite:
   // all of them, by the same kernels as with a truncation
   static int32_t colfft(const scl_plan3d& pl, C* f0, int64_t fstride, int nf, int axis, int dir, R kc2 = 0);
-  static int32_t zinv_vort(const scl_plan3d& pl, const C* s, int64_t sstride, C* w, int64_t wstride);
+  // ab2: as the IF-AB2 steps' z-passes have it (k_zinv_all)
+  static int32_t zinv_vort(const scl_plan3d& pl, const C* s, int64_t sstride, C* w, int64_t wstride, bool ab2 = false);
   static int32_t yinv_vort(const scl_plan3d& pl, C* W, int64_t fstride, R kc2 = 0);
   // fused (mode 1..4): also z-inverse the new stage state (mode 4: the new
   // v) into W[0..4] for the next RHS (k_zfwd_rhs FUSED)

@@ -174,7 +174,7 @@ inline int32_t check_zs(const Geom& g) {
 }
 
 template <class R>
-int32_t Ops<R>::zinv_vort(const scl_plan3d& pl, const C* s, int64_t sstride, C* w, int64_t wstride) {
+int32_t Ops<R>::zinv_vort(const scl_plan3d& pl, const C* s, int64_t sstride, C* w, int64_t wstride, bool ab2) {
   const Geom& g = pl.g;
   return with_line<R>(g.nz, [&](auto NC) -> int32_t {
     constexpr int N = decltype(NC)::value;
@@ -184,12 +184,14 @@ int32_t Ops<R>::zinv_vort(const scl_plan3d& pl, const C* s, int64_t sstride, C* 
       using CC = ColCfg<R, N, CW, EZ>;
       SCL_CHECK((check_cols<R, N, CW>(g)));
       SCL_CHECK(check_zs(g));
-      if (g.zs == 3)
-        hipLaunchKernelGGL((k_zinv_vort<R, N, CW, EZ, 3>), dim3(col_grid<CW, 2>(g)), dim3(CC::BS), 0, pl.stream, s,
-                           sstride, w, wstride, g, twp<R>(pl), pl.L / N);
-      else
-        hipLaunchKernelGGL((k_zinv_vort<R, N, CW, EZ, 0>), dim3(col_grid<CW, 2>(g)), dim3(CC::BS), 0, pl.stream, s,
-                           sstride, w, wstride, g, twp<R>(pl), pl.L / N);
+      auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(col_grid<CW, 2>(g)), dim3(CC::BS), 0, pl.stream, s, sstride, w, wstride, g,
+                           twp<R>(pl), pl.L / N);
+      };
+      if (ab2 && g.zs == 3) launch(k_zinv_all<R, N, CW, EZ, 3>);
+      else if (ab2) launch(k_zinv_all<R, N, CW, EZ, 0>);
+      else if (g.zs == 3) launch(k_zinv_vort<R, N, CW, EZ, 3>);
+      else launch(k_zinv_vort<R, N, CW, EZ, 0>);
       return check_launch("zinv_vort");
     };
     if constexpr (sizeof(R) == 4 && N <= 512) {
@@ -225,10 +227,14 @@ int32_t Ops<R>::zfwd_rhs(const scl_plan3d& pl, int mode, C* W, int64_t fstride, 
         };
         // short lines come in both variants: their grids can be so small
         // that the instructions of the unused one are felt (Cut)
-        if constexpr (N <= 64) {
-          if (!p.trunc) return go(k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS, false>);
+        if constexpr (MODE >= 5) {
+          go(k_zfwd_ab2<R, N, MODE, CW, EZ, FUSED, ZS>);
+        } else {
+          if constexpr (N <= 64) {
+            if (!p.trunc) return go(k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS, false>);
+          }
+          go(k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS>);
         }
-        go(k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS>);
       };
       auto by_zs = [&](auto MC, auto FC) {
         if (g.zs == 3) launch(MC, FC, IC<3>{});
