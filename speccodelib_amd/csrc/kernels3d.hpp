@@ -494,12 +494,8 @@ __device__ inline void stage_load3(StageIn<R> (&in)[3], uint32_t o, int64_t fs, 
     for (int q = 0; q < 3; ++q) in[q].v = ld_once<R, NT>(V + q * fs + o);
   }
   if (MODE > 1 && !cut) {
-    const cpx<R>* const H = MODE == 7 ? S : DU;
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      if constexpr (MODE >= 5) in[q].v = ld_once<R, NT>(V + q * fs + o);
-      if constexpr (MODE != 5) in[q].h = ld_once<R, NT>(H + q * fs + o);
-    }
+    for (int q = 0; q < 3; ++q) in[q].h = ld_once<R, NT>(DU + q * fs + o);
   }
 }
 
@@ -629,29 +625,6 @@ __device__ inline cpx<R> ab_math(const StageIn<R>& in, cpx<R> a, const AbWeights
   else y = v + w.cS * a + w.cek * (in.h + e2 * in.h);
   return cut ? mk<R>(0, 0) : y + e1 * y;
 }
-// ab_math of the three components of a mode with its stores.  over: k2 >=
-// kcut^2, where the history is never used and not kept; vcut: as stage_apply3.
-template <int MODE, class R>
-__device__ inline void ab_apply3(const StageIn<R> (&in)[3], const cpx<R> (&a)[3], cpx<R> (&out)[3], uint32_t o,
-                                 int64_t fs, cpx<R>* V, cpx<R>* DU, cpx<R>* S, const AbWeights<R>& w, R e1, R e2,
-                                 bool cut, unsigned* nf, bool over, bool vcut) {
-#pragma unroll
-  for (int q = 0; q < 3; ++q) out[q] = ab_math<MODE, R>(in[q], a[q], w, e1, e2, cut);
-  if (!over) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      if constexpr (MODE == 5) (DU + q * fs)[o] = in[q].v;
-      if constexpr (MODE != 6) (S + q * fs)[o] = a[q];
-    }
-  }
-  if (!(over && vcut)) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) (V + q * fs)[o] = out[q];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) flag_nonfinite(nf, out[q]);
-  }
-}
-
 // ZFWD: z-forward of the three transformed products + forcing + the
 // pointwise part of symmetrize + projection (+ optional RHS truncation),
 // then, for MODE 1..4, the IF-RK4 stage update; MODE 0 writes N(u) back
@@ -686,7 +659,7 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
   __shared__ cpx<R> twl[N];  // this line length's twiddles; first read after a barrier
   for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
   const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
-  // MODE 4 and up end a step, so only the modes inside the truncation count:
+  // MODE 4 ends a step, so only the modes inside the truncation count:
   // columns without any (col_cut) are neither read nor transformed, and their
   // z-inverse is not stored (the next y-inverse leaves them out).  With
   // scut (RHS truncated as well) the same holds for every stage.
@@ -772,12 +745,6 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
     fa = (R)coef[0];
     fb = (R)coef[1];
   }
-  R ab_dto = 0;
-  AbWeights<R> ab{};
-  if constexpr (MODE >= 5) {
-    ab_dto = (R)p.ab[AB_DTO];
-    ab = {(R)p.ab[AB_DT], (R)p.ab[AB_S], (R)p.ab[AB_EK], (R)p.ab[AB_DELTA]};
-  }
   // With the park, the new x stage state goes back to its park slot (just
   // read) until the z-inverse, which keeps 2E registers free here.
   auto keep_x = [&](int m, cpx<R> v) {
@@ -830,17 +797,6 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
       W[o] = a;
       W1[o] = b;
       W2[o] = d;
-    } else if constexpr (MODE >= 5) {
-      const R xk = -p.nu * k2;
-      const R e1 = expm1_r(xk * ab.dt);
-      const R e2 = MODE == 5 ? (R)0 : expm1_r(xk * ab_dto);
-      const bool cut = k2 >= p.kc2 || ik2 == 0, over = trunc && k2 >= p.kc2;
-      const cpx<R> n[3] = {a, b, d};
-      cpx<R> out[3];
-      ab_apply3<MODE, R>(in, n, out, o, fstride, V, DU, S, ab, e1, e2, cut, p.nonfinite, over, vcut);
-      keep_x(m, out[0]);
-      ny_[m] = out[1];
-      nz_[m] = out[2];
     } else {
       // E = exp(x), x = -nu k2 dt/2.  E is within 1e-3 of 1 for most modes,
       // where FP32 spacing (6e-8) makes a rounded E or E*E a biased factor
