@@ -161,9 +161,18 @@ extern "C" int32_t scl_dns_rhs(scl_dns* d, double t, const void* const* y, void*
 
 extern "C" int32_t scl_dns_state(scl_dns* d, void** state, int64_t* n) {
   if (!d || !state || !n) return set_error("null argument"), SCL_EINVAL;
+  if (d->ext && !d->state_out && d->exec) {
+    // the captured step takes the state to be truncated
+    SCL_HIP(hipStreamSynchronize(d->plan->stream));
+    (void)hipGraphExecDestroy(d->exec);
+    (void)hipGraphDestroy(d->graph);
+    d->exec = nullptr;
+    d->graph = nullptr;
+  }
   *state = d->fields;
   *n = (int64_t)d->nc * d->plan->fstride();
   d->chained = d->truncated = false;  // the caller may change the state through the pointer
+  d->state_out = true;
   return SCL_OK;
 }
 

@@ -71,6 +71,10 @@ struct scl_dns {
   // LES / scalar: the state is zero beyond the truncation (a step has left it
   // so); cleared with chained
   bool truncated = false;
+  // scl_dns_state has given the state's address out: the caller may write to
+  // it at any time, so LES / scalar steps take it as it is (truncated stays
+  // false)
+  bool state_out = false;
   // IF-AB2 (p.stepper 1, 2): device state (AB_* slots), energy partials, and
   // the steps taken since the state was set (selects the bootstrap modes)
   double* ab = nullptr;
