@@ -34,6 +34,7 @@ struct Group {
   const void* tw = nullptr;  // exp(-2 pi i j/n), j < n (owned by the ensemble)
   void* base = nullptr;
   int e = 8, cw = 8, row_grid = 0;
+  bool split = false;  // scheme 1: the halves of a step one after the other (turb_split)
   hipStream_t stream = nullptr;  // branch stream (batched mode)
   hipEvent_t done = nullptr;
   int64_t fs() const { return g.ntot + SCL_FIELD_PAD; }  // padded as the 3D fields
@@ -45,8 +46,47 @@ struct Group {
 
 // Scheme 1 (turb_2d.f90) keeps the previous nonlinear term in F_ACC, the
 // state before the first step in F_S and the shifted half's work fields in
-// three more, F_W2.
-enum { F_W = 0, F_WS = 3, F_ACC = 4, F_S = 5, F_W2 = 6, NFIELDS = 6, NFIELDS_TURB = 9 };
+// three more, F_W2; where the halves go one after the other, the unshifted half
+// of the nonlinear term in one more.
+enum { F_W = 0, F_WS = 3, F_ACC = 4, F_S = 5, F_W2 = 6, NFIELDS = 6, NFIELDS_TURB = 9, NFIELDS_TURB_SPLIT = 7 };
+
+int fields_of(const scl_ens2d_params& p, const Group& gr) {
+  return p.scheme != 1 ? NFIELDS : gr.split ? NFIELDS_TURB_SPLIT : NFIELDS_TURB;
+}
+
+// Whether a batch of scheme 1 runs the two halves of a step one after the other
+// (six launches and seven fields, k_yfwd2d_turb SPLIT) or both in each pass (two
+// launches and nine fields).  Both halves at once hold twice the columns in
+// registers, so fewer workgroups are in flight: that is the faster one while a
+// batch leaves the chip room, and where lines are so short that many workgroups
+// fit anyway.  us per step, both at once / one after the other, by members:
+//   FP32 1024^2: 3 120/124, 4 203/186, 16 664/518, 32 1233/1010
+//        512^2: 12 103/113, 16 139/136, 64 475/416, 128 921/881
+//        256^2: 128 182/192, 256 401/398, 512 845/912
+//        128^2: 512 181/178, 1024 407/411, 2048 819/913
+//        64^2: 1536 136/137, 2048 198/182, 4096 439/422, 6144 658/685
+//        32^2: 6144 163/177, 8192 245/226
+//   (between 2^23 and 2^24 points seven fields stay largely in the 256 MB of the
+//   last cache and nine do not; far above, neither)
+//   FP64 1024^2: 4 305/310, 32 2016/2208
+//        512^2: 6 94/110, 8 159/152, 16 271/238, 128 1757/1586
+//        256^2: 24 99/106, 32 132/121, 512 1710/1548
+//        128^2: 96 86/96, 128 115/109, 2048 1597/1506
+//        64^2: 384 75/88, 512 100/103, 768 141/137, 8192 1541/1525
+//        32^2: 768 65/81, 1024 88/85, 4096 283/203
+// SCL_TURB2D_SPLIT = 1 or 0 when the ensemble is made: always or never, to
+// compare the two.
+bool turb_split(int prec, int n, int nb) {
+  if (const char* s = std::getenv("SCL_TURB2D_SPLIT")) return s[0] == '1';
+  const int64_t points = (int64_t)nb * n * n, m = (int64_t)1 << 20;
+  if (prec == SCL_SP) {
+    if (n >= 1024) return points >= 4 * m;
+    if (n >= 512) return points >= 4 * m;
+    return n <= 64 && points >= 8 * m && points <= 16 * m;
+  }
+  if (n >= 1024) return false;
+  return n >= 64 ? points >= 2 * m : points >= m;
+}
 
 // FP64 plans keep one schedule: E = 8 with 8 columns, 4 at 1024 points
 // (8 would need 163 KB of LDS with the line's twiddles).
@@ -178,13 +218,13 @@ Cut<R> cut2d(const scl_ens2d& e, const Group& gr, bool trunc) {
 
 // Workgroups of the x-pass: persistent (as many as can be resident) or one
 // per row group.
-template <class R, int M>
+template <class R, int M, bool CUT>
 int64_t row_grid_size(const scl_ens2d& e, const Group& gr) {
   using RC = RowCfg<R, M>;
   static int resident = 0;
   if (!resident) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_row_adv2d<R, M>, RC::BS, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_row_adv2d<R, M, CUT>, RC::BS, 0) != hipSuccess ||
         per_cu < 1)
       per_cu = 1;
     resident = per_cu;
@@ -193,15 +233,20 @@ int64_t row_grid_size(const scl_ens2d& e, const Group& gr) {
   return gr.row_grid ? ngroups : std::min<int64_t>(ngroups, (int64_t)resident * e.ncu);
 }
 
-// halves = 2 (here and in row_launch): the shifted half of scheme 1 as well.
+// halves = 2 (here and in row_launch): the shifted half of scheme 1 as well;
+// first = 1 (halves = 1): that half alone.
 template <class R>
-int32_t yinv_launch(const Group& gr, const cpx<R>* src, int halves, hipStream_t st, Cut<R> cut) {
+int32_t yinv_launch(const scl_ens2d& e, const Group& gr, const cpx<R>* src, int halves, hipStream_t st, Cut<R> cut,
+                    int first = 0) {
   const cpx<R>* tw = reinterpret_cast<const cpx<R>*>(gr.tw);
   return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
     constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
-    hipLaunchKernelGGL((k_yinv2d<R, N, E, CW>), dim3(ycut_grid<CW>(gr.g, cut.nkx), halves),
-                       dim3(Col2D<R, N, E, CW>::BS), 0, st, src, gr.field<R>(F_W), gr.fs(), gr.g, tw, 1,
-                       (F_W2 - F_W) * gr.fs(), cut);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(ycut_grid<CW>(gr.g, cut.nkx), halves), dim3(Col2D<R, N, E, CW>::BS), 0, st, src,
+                         gr.field<R>(F_W), gr.fs(), gr.g, tw, 1, (F_W2 - F_W) * gr.fs(), first, cut);
+    };
+    if (e.p.scheme == 1) go(k_yinv2d<R, N, E, CW, false>);
+    else go(k_yinv2d<R, N, E, CW, true>);
     return check_launch("yinv2d");
   });
 }
@@ -212,8 +257,12 @@ int32_t row_launch(const scl_ens2d& e, const Group& gr, int halves, hipStream_t 
   return with_row2d<R>(gr.n / 2, [&](auto MC) -> int32_t {
     constexpr int M = decltype(MC)::value;
     const R scale = (R)1 / (R)((double)gr.n * gr.n);
-    hipLaunchKernelGGL((k_row_adv2d<R, M>), dim3((unsigned)row_grid_size<R, M>(e, gr), halves), dim3(RowCfg<R, M>::BS),
-                       0, st, gr.field<R>(F_W), gr.fs(), (F_W2 - F_W) * gr.fs(), gr.g, scale, tw, 2, 1, cut.nkx);
+    auto go = [&](auto kern, int64_t grid) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)grid, halves), dim3(RowCfg<R, M>::BS), 0, st, gr.field<R>(F_W), gr.fs(),
+                         (F_W2 - F_W) * gr.fs(), gr.g, scale, tw, 2, 1, cut.nkx);
+    };
+    if (e.p.scheme == 1) go(k_row_adv2d<R, M, false>, row_grid_size<R, M, false>(e, gr));
+    else go(k_row_adv2d<R, M, true>, row_grid_size<R, M, true>(e, gr));
     return check_launch("row_adv2d");
   });
 }
@@ -237,7 +286,7 @@ int32_t stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st, boo
   const Rhs2D<R> rp = rhs_params<R>(e, gr.n, trunc);
   const Cut<R> cut = cut2d<R>(e, gr, trunc);
   if (fuse && mode < 1) return set_error("fused 2D stage: mode %d is not a stage 1..4", mode), SCL_EINVAL;
-  if (!primed) SCL_CHECK(yinv_launch<R>(gr, sin, 1, st, cut));
+  if (!primed) SCL_CHECK(yinv_launch<R>(e, gr, sin, 1, st, cut));
   SCL_CHECK(row_launch<R>(e, gr, 1, st, cut));
   return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
     constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
@@ -268,8 +317,8 @@ Turb2DP<R> turb_params(const scl_ens2d& e, int n) {
 }
 
 // One turb_2d.f90 step (mode TURB_STEP0, TURB_STEP1, TURB_AB2) or nonlinear
-// term (TURB_RHS) of a group, both halves of the products in each pass.
-// primed, fuse: as stage.
+// term (TURB_RHS) of a group, both halves of the products in each pass (or,
+// gr.split, one after the other).  primed, fuse: as stage, not with gr.split.
 template <class R>
 int32_t turb_stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st, bool primed = false,
                    bool fuse = false) {
@@ -277,19 +326,31 @@ int32_t turb_stage(const scl_ens2d& e, const Group& gr, int mode, hipStream_t st
   const C* tw = reinterpret_cast<const C*>(gr.tw);
   const Turb2DP<R> tp = turb_params<R>(e, gr.n);
   const Cut<R> all = cut2d<R>(e, gr, false);
-  if (!primed) SCL_CHECK(yinv_launch<R>(gr, gr.field<R>(F_WS), 2, st, all));
+  auto yfwd = [&](int m) -> int32_t {
+    return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
+      constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(col_grid<CW, 1>(gr.g)), dim3(Col2D<R, N, E, CW>::BS), 0, st, gr.field<R>(F_W),
+                           gr.fs(), (F_W2 - F_W) * gr.fs(), gr.field<R>(F_WS), gr.field<R>(F_ACC), gr.field<R>(F_S),
+                           m, tp, gr.g, tw, 1);
+      };
+      if (gr.split) go(k_yfwd2d_turb<R, N, E, CW, false, true>);
+      else if (fuse) go(k_yfwd2d_turb<R, N, E, CW, true>);
+      else go(k_yfwd2d_turb<R, N, E, CW, false>);
+      return check_launch("yfwd2d_turb");
+    });
+  };
+  if (gr.split) {
+    for (int half = 0; half < 2; ++half) {
+      SCL_CHECK(yinv_launch<R>(e, gr, gr.field<R>(F_WS), 1, st, all, half));
+      SCL_CHECK(row_launch<R>(e, gr, 1, st, all));
+      SCL_CHECK(yfwd(half ? mode : (int)TURB_HALF));
+    }
+    return SCL_OK;
+  }
+  if (!primed) SCL_CHECK(yinv_launch<R>(e, gr, gr.field<R>(F_WS), 2, st, all));
   SCL_CHECK(row_launch<R>(e, gr, 2, st, all));
-  return with_col2d<R>(gr.n, gr.e, gr.cw, [&](auto NC, auto EC, auto CC) -> int32_t {
-    constexpr int N = decltype(NC)::value, E = decltype(EC)::value, CW = decltype(CC)::value;
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(col_grid<CW, 1>(gr.g)), dim3(Col2D<R, N, E, CW>::BS), 0, st, gr.field<R>(F_W),
-                         gr.fs(), (F_W2 - F_W) * gr.fs(), gr.field<R>(F_WS), gr.field<R>(F_ACC), gr.field<R>(F_S),
-                         mode, tp, gr.g, tw, 1);
-    };
-    if (fuse) go(k_yfwd2d_turb<R, N, E, CW, true>);
-    else go(k_yfwd2d_turb<R, N, E, CW, false>);
-    return check_launch("yfwd2d_turb");
-  });
+  return yfwd(mode);
 }
 
 int turb_mode(int64_t step) { return step == 0 ? TURB_STEP0 : step == 1 ? TURB_STEP1 : TURB_AB2; }
@@ -655,7 +716,8 @@ extern "C" int32_t scl_ens2d_create(int32_t prec, int32_t ngroups, const int32_t
       gr.tw = tw;
       gr.e = 8;  // at 1024 points: one 1024-thread workgroup per CU, 4 waves per SIMD
       gr.cw = prec == SCL_DP && n >= 1024 ? 4 : 8;  // FP64 1024: 4 columns (LDS)
-      const size_t bytes = (size_t)(params->scheme == 1 ? NFIELDS_TURB : NFIELDS) * gr.fs() * es;
+      gr.split = params->scheme == 1 && turb_split(prec, n, nb);
+      const size_t bytes = (size_t)fields_of(*params, gr) * gr.fs() * es;
       if (hipMalloc(&gr.base, bytes) != hipSuccess) {
         (void)hipGetLastError();
         e->groups.push_back(gr);

@@ -136,28 +136,33 @@ __device__ inline cpx<R> shifted(cpx<R> v, int s, int n) {
 }
 
 // YINV.  s: the stage vorticity; w: three work fields (u, v, w) at stride
-// fstride.  Blocks of blockIdx.y = 1 do the shifted field, into w + hs.
-// cut: modes beyond it are taken as zero, and only its nkx columns stored.
-template <class R, int N, int E, int CW>
+// fstride.  Blocks of blockIdx.y = 0 do half `first`, the others half 1, the
+// shifted field, into w + hs.
+// CUT: modes beyond cut are taken as zero, and only its nkx columns stored; in
+// scheme 0 steps of untruncated states too (cut infinite), scheme 1 goes without
+// it (16 members of 1024^2, FP32: 102 us with it, 81 without).
+template <class R, int N, int E, int CW, bool CUT>
 __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yinv2d(const cpx<R>* __restrict__ s,
                                                                    cpx<R>* __restrict__ w, int64_t fstride, Geom g,
                                                                    const cpx<R>* __restrict__ tw, int tws,
-                                                                   int64_t hs, Cut<R> cut) {
+                                                                   int64_t hs, int first, Cut<R> cut) {
   using CC = Col2D<R, N, E, CW>;
   constexpr int T = CC::T;
   __shared__ cpx<R> lds[lds_pad(N) * CW];
   __shared__ cpx<R> twl[N];  // first read after a barrier inside the transform
   for (int i = threadIdx.x; i < N; i += CC::BS) twl[i] = tw[i * tws];
   const int c = threadIdx.x % CW, rt = threadIdx.x / CW;
-  Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, gridDim.x), c, ycut_tiles<CW>(g, cut.nkx));
-  if (t.kx >= cut.nkx) t.ok = false;
+  Tile t = col_tile<CW, 1>(g, xcd_swizzle(blockIdx.x, gridDim.x), c, CUT ? ycut_tiles<CW>(g, cut.nkx) : g.mx / CW);
+  if (CUT && t.kx >= cut.nkx) t.ok = false;
   cpx<R> o[E];
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     const int j = rt + T * m;
-    o[m] = ld_or_zero(s, t.base + (int64_t)j * t.rs, t.base, t.ok && !col_cut<R>(t.kx, kwave(j, N), cut.kc2));
+    const int64_t at = t.base + (int64_t)j * t.rs;
+    if constexpr (CUT) o[m] = ld_or_zero(s, at, t.base, t.ok && !col_cut<R>(t.kx, kwave(j, N), cut.kc2));
+    else o[m] = t.ok ? s[at] : mk<R>(0, 0);
   }
-  if (blockIdx.y) {
+  if (first + blockIdx.y) {
 #pragma unroll
     for (int m = 0; m < E; ++m) o[m] = shifted(o[m], t.kx + kwave(rt + T * m, N), N);
   }
@@ -165,11 +170,12 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yinv2d(const cpx<R
 }
 
 // XPASS: per row, c2r of u, v, w; u w and v w times scale; r2c of both
-// into work fields 0 and 1.  Persistent grid over groups of RPW rows.  Entries
-// k >= nkx of the inputs are taken as zero and those of the outputs not
-// stored (the truncation; nx/2 + 1: all of them).  Blocks of blockIdx.y = 1 do
-// the fields at W + hs (the shifted half of scheme 1).
-template <class R, int M>
+// into work fields 0 and 1.  Persistent grid over groups of RPW rows.  CUT:
+// entries k >= nkx of the inputs are taken as zero and those of the outputs not
+// stored (the truncation; nx/2 + 1: all of them); scheme 1 goes without it (1024
+// members of 64^2, FP64: 34.2 us with it, 31.6 without).  Blocks of blockIdx.y =
+// 1 do the fields at W + hs (the shifted half of scheme 1).
+template <class R, int M, bool CUT>
 __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int64_t fstride, int64_t hs, Geom g,
                                                                 R scale, const cpx<R>* __restrict__ tw, int twsM,
                                                                 int twsN, int nkx) {
@@ -197,9 +203,9 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int
 #pragma unroll
       for (int m = 0; m < 8; ++m) {
         const int k = rt + T * m;
-        raw[f][m] = ld_or_zero(base, row * M + k, row * M, k < nkx);
+        raw[f][m] = CUT ? ld_or_zero(base, row * M + k, row * M, k < nkx) : base[row * M + k];
       }
-      xm[f] = rt == 0 && M < nkx ? base[g.nmain + row] : mk<R>(0, 0);
+      xm[f] = rt == 0 && (!CUT || M < nkx) ? base[g.nmain + row] : mk<R>(0, 0);
     }
     cpx<R> a[3][8];
 #pragma unroll
@@ -220,7 +226,7 @@ __global__ __launch_bounds__((RowCfg<R, M>::BS)) void k_row_adv2d(cpx<R>* W, int
     for (int f = 0; f < 2; ++f) {
       cpx<R>* base = W + f * fstride;
       LF::run(p[f], lrow, rt, twM, 1, LinIdx{});
-      row_r2c_post<R, M, true>(p[f], base + row * M, base + g.nmain + row, rt, twN, 1, nkx);
+      row_r2c_post<R, M, CUT>(p[f], base + row * M, base + g.nmain + row, rt, twN, 1, nkx);
     }
   }
 }
@@ -408,7 +414,7 @@ struct Turb2DP {
   int forced;
 };
 
-enum { TURB_STEP0 = 1, TURB_STEP1 = 2, TURB_AB2 = 3, TURB_RHS = 4 };
+enum { TURB_HALF = 0, TURB_STEP0 = 1, TURB_STEP1 = 2, TURB_AB2 = 3, TURB_RHS = 4 };
 
 // YFWD of the phase-shift dealiased nonlinear term (turb_2d.f90:287-421) and
 // the stepper (:430-483).  W: the products of the unshifted (W[0], W[1]) and of
@@ -430,7 +436,11 @@ enum { TURB_STEP0 = 1, TURB_STEP1 = 2, TURB_AB2 = 3, TURB_RHS = 4 };
 // launches (with the x-pass), not six, and the unshifted half of N and the
 // state do not go through memory between them (7 members of 128^2 and 3 of
 // 512^2, FP32, 200 steps and read-back: 24.8 -> 16.9 ms).
-template <class R, int N, int E, int CW, bool FUSED = false>
+// SPLIT: the halves one after the other in W, a launch each (TURB_HALF leaves
+// the unshifted half of N in W + hs, the other modes take it from there): the
+// kernel then holds one half's columns, and a batch two fields less (16 members
+// of 1024^2, FP32, a step: 664 us both at once, 518 split).
+template <class R, int N, int E, int CW, bool FUSED = false, bool SPLIT = false>
 __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
     cpx<R>* W, int64_t fstride, int64_t hs, cpx<R>* WS, cpx<R>* OWZ, cpx<R>* W0, int mode, Turb2DP<R> p, Geom g,
     const cpx<R>* __restrict__ tw, int tws) {
@@ -466,7 +476,14 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
   };
   cpx<R> na[E], nb[E];
   half_term(W, na);
-  half_term(W + hs, nb);
+  if constexpr (!SPLIT) {
+    half_term(W + hs, nb);
+  } else if (mode == TURB_HALF) {
+    if (!t.ok) return;
+#pragma unroll
+    for (int m = 0; m < E; ++m) W[hs + t.base + (int64_t)L::out_pos(m, rt) * t.rs] = na[m];
+    return;
+  }
   if (kx0_tile) __syncthreads();  // the transforms' LDS reads are done
   auto force = [&](cpx<R> a) {
     const R den = a.x * a.x + a.y * a.y;
@@ -488,7 +505,9 @@ __global__ __launch_bounds__((Col2D<R, N, E, CW>::BS)) void k_yfwd2d_turb(
     const int ik2 = ikx * ikx + iky * iky;
     const R k2 = ik2 == 0 ? (R)0.5 : (R)ik2;  // wavenumber(): k2(0, 0) = 0.5
     const int64_t o = t.base + (int64_t)y * t.rs;
-    cpx<R> r = na[m] + nb[m] * half_cell_phase<R>(ikx + iky, N);
+    cpx<R> r;
+    if constexpr (SPLIT) r = (t.ok ? W[hs + o] : mk<R>(0, 0)) + na[m] * half_cell_phase<R>(ikx + iky, N);
+    else r = na[m] + nb[m] * half_cell_phase<R>(ikx + iky, N);
     if (y == N / 2 || ikx == g.mx || ik2 == 0 || k2 >= p.kc2) r = mk<R>(0, 0);
     cpx<R> o1 = r, o2 = mk<R>(0, 0);
     if (mode != TURB_RHS && t.ok) {
