@@ -357,6 +357,9 @@ void scl_derivs_(const double *x, const double *y, double *dydx, const int32_t *
  * launches per group, the groups on parallel branches of one hipGraph per
  * step).  per_member = 1: every member is its own solver with its own
  * launches, for comparison.
+ *
+ * Device memory: six fields of (n/2 + 1) n entries per member; scheme 1 nine,
+ * or seven where a batch fills the chip or nine do not fit.
  * ------------------------------------------------------------------- */
 typedef struct scl_ens2d scl_ens2d;
 typedef struct scl_ens2d_params {

@@ -632,6 +632,35 @@ void destroy_groups(scl_ens2d& e) {
   e.tw.clear();
 }
 
+// The groups' fields, zeroed.  A scheme 1 ensemble that does not fit takes the
+// smaller layout (split) for all its groups before it is refused.
+int32_t allocate_groups(scl_ens2d& e) {
+  for (;;) {
+    size_t refused = 0;
+    bool larger = false;
+    for (auto& gr : e.groups) {
+      const size_t bytes = (size_t)fields_of(e.p, gr) * gr.fs() * e.esize();
+      larger = larger || (e.p.scheme == 1 && !gr.split);
+      if (!refused && hipMalloc(&gr.base, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        gr.base = nullptr;
+        refused = bytes;
+      }
+    }
+    if (!refused) break;
+    if (!larger) return set_error("device allocation of %zu bytes failed", refused), SCL_ENOMEM;
+    for (auto& gr : e.groups) {
+      if (gr.base) (void)hipFree(gr.base);
+      gr.base = nullptr;
+      gr.split = true;
+    }
+  }
+  for (auto& gr : e.groups)
+    if (hipMemsetAsync(gr.base, 0, (size_t)fields_of(e.p, gr) * gr.fs() * e.esize(), e.stream) != hipSuccess)
+      return set_error("memset failed"), SCL_EHIP;
+  return SCL_OK;
+}
+
 template <class R>
 int32_t upload_twiddles(int n, void** out) {
   std::vector<double> re, im;
@@ -690,7 +719,6 @@ extern "C" int32_t scl_ens2d_create(int32_t prec, int32_t ngroups, const int32_t
       hipEventCreateWithFlags(&e->fork, hipEventDisableTiming) != hipSuccess || hipEventCreate(&e->t0) != hipSuccess ||
       hipEventCreate(&e->t1) != hipSuccess)
     return set_error("stream/event creation failed"), fail(SCL_EHIP);
-  const size_t es = e->esize();
   for (int ug = 0; ug < ngroups; ++ug) {
     const int n = sizes[ug];
     e->sizes.push_back(n);
@@ -717,16 +745,6 @@ extern "C" int32_t scl_ens2d_create(int32_t prec, int32_t ngroups, const int32_t
       gr.e = 8;  // at 1024 points: one 1024-thread workgroup per CU, 4 waves per SIMD
       gr.cw = prec == SCL_DP && n >= 1024 ? 4 : 8;  // FP64 1024: 4 columns (LDS)
       gr.split = params->scheme == 1 && turb_split(prec, n, nb);
-      const size_t bytes = (size_t)fields_of(*params, gr) * gr.fs() * es;
-      if (hipMalloc(&gr.base, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        e->groups.push_back(gr);
-        return set_error("device allocation of %zu bytes failed", bytes), fail(SCL_ENOMEM);
-      }
-      if (hipMemsetAsync(gr.base, 0, bytes, e->stream) != hipSuccess) {
-        e->groups.push_back(gr);
-        return set_error("memset failed"), fail(SCL_EHIP);
-      }
       if (!params->per_member && ngroups > 1) {
         if (hipStreamCreateWithFlags(&gr.stream, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&gr.done, hipEventDisableTiming) != hipSuccess) {
@@ -737,6 +755,7 @@ extern "C" int32_t scl_ens2d_create(int32_t prec, int32_t ngroups, const int32_t
       e->groups.push_back(gr);
     }
   }
+  if (const int32_t st = allocate_groups(*e); st != SCL_OK) return fail(st);
   if (hipMalloc((void**)&e->diag, 2 * sizeof(double) * e->total_members()) != hipSuccess)
     return set_error("device allocation failed"), fail(SCL_ENOMEM);
   if (hipStreamSynchronize(e->stream) != hipSuccess) return set_error("stream sync failed"), fail(SCL_EHIP);

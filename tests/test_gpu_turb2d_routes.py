@@ -72,3 +72,34 @@ def test_memory_of_a_batch_that_fills_the_chip(n, members, prec):
     f = members * n * (n // 2 + 1) * (8 if prec == scl.SP else 16)
     print(f"{used / f:.2f} fields of {f >> 20} MB", flush=True)
     assert used < 8 * f
+
+
+@pytest.mark.parametrize("n,members,per_member", [(256, 4096, False), (1024, 256, True)])
+def test_batches_that_only_fit_in_seven_fields(n, members, per_member):
+    """Sizes that take nine fields where there is room (forced off: the members
+    that are not set stay zero)."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU visible to torch")
+    w = field(n, 3).astype(np.complex64)
+    got = []
+    for fill in (False, True):
+        hold = None
+        m = members if fill else 2
+        if fill:
+            f = members * n * (n // 2 + 1) * 8
+            torch.cuda.empty_cache()
+            free = torch.cuda.mem_get_info()[0]
+            if free < 16 * f:
+                pytest.skip("not enough free memory on this device")
+            hold = torch.empty(free - 8 * f, dtype=torch.uint8, device="cuda")
+        try:
+            e = scl.Ensemble2D([(n, m)], prec=scl.SP, dt=1e-3, scheme=1, per_member=per_member, use_graph=False,
+                               forced=False, **par(n))
+            e.set_member(0, m - 1, w)
+            e.step(4)
+            got.append(e.get_member(0, m - 1).copy())
+            e.close()
+        finally:
+            del hold
+            torch.cuda.empty_cache()
+    assert np.abs(got[0] - got[1]).max() < 1e-5 * np.abs(got[0]).max()
