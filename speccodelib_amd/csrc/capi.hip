@@ -518,9 +518,53 @@ extern "C" int32_t scl_force_heli(scl_plan3d* p, void* fx, void* fy, void* fz, c
 // One RHS / one IF-RK4 step on device fields
 // Whether leaving out the modes beyond the truncation pays.  Where the fields
 // of a step sit in the caches a pass is bound by its longest chain of
-// instructions, not by its bytes: 32^3 (0.14 MB a field) was 5% slower with
-// it; 128^3 (8.5 MB) 1.14 times as fast.
+// instructions, not by its bytes.  us per step, all modes / truncated, by the
+// size of a field: below 0.6 MB slower (FP32 DNS 32^3 74/81, 64x64x32 105/113,
+// LES and scalar 64x32x32 215/228), about even at 1 MB (FP32 64^3 DNS 118/119,
+// LES 230/226, 128x64x32 DNS 124/131), faster from 2 MB on (FP32 64x64x128 DNS
+// 160/150, LES 302/298; FP64 64^3 DNS 180/172, scalar 252/258; 128^3 FP32 357/323).
 static bool trunc_pays(const scl_plan3d* p) { return (size_t)p->g.ntot * p->esize() >= ((size_t)2 << 20); }
+
+// Whether a solver's truncation radius keeps so much that leaving out the rest
+// does not pay for the conditional loads and stores.  The 2/3 radius never does
+// (it keeps at most 2/3 of the kx); a larger one, on a grid that is wide in x,
+// can keep everything.  All modes / truncated, by the kept part of the modes:
+//   DNS, FP32 256^3 0.67 1.02, 0.85 1.00, 0.96 0.99; 512x128x64 0.78 1.00, 0.88
+//     0.98, 0.98 0.96; 128^3 0.85 1.03, 0.96 1.02.  FP64 512x128x64 0.88 1.03, 1.00
+//     0.99; 256^3 0.85 1.00, 0.96 1.00
+//   DNS, RHS truncated, FP32 512x128x64 0.78 1.06, 0.88 0.97, 0.98 0.95; 128^3 0.85
+//     1.05, 0.96 1.02.  FP64 256x256x128 0.85 1.06, 0.96 1.01, 1.00 1.00
+//   scalar, FP32 512x128x64 0.78 1.06, 0.88 1.02, 1.00 0.98; FP64 256x256x128 0.72
+//     1.01, 0.85 0.99, 0.96 0.98; IF-AB2 FP64 128^3 0.85 1.05, 0.96 1.00, 1.00 0.97
+// With the Smagorinsky term the y-passes weigh most, so the kept (kx, ky) columns
+// tell:
+//   FP32 512x128x64 0.79 1.04, 0.89 1.02, 1.00 0.99; FP64 256^3 0.78 1.00, 0.89
+//     0.99, 0.97 0.98; 512x128x64 0.79 1.02, 0.89 1.00, 0.99 0.99
+//   IF-AB2 FP32 256x256x128 0.78 1.06, 0.89 0.99, 0.97 0.97; 512x128x64 0.89 1.04,
+//     0.99 0.96; FP64 128^3 0.89 1.04, 0.97 1.01, 1.00 0.98
+// Fields of up to 8 MB stay in the caches, and the truncated passes are slower only
+// where nothing at all is left out (FP64 512x64x32 IF-AB2 0.99 1.09; FP32, LES with
+// IF-AB2, 1.00 0.92, LES and scalar 1.00 0.95).
+static bool keeps_most(const scl_plan3d* p, const scl_dns_params& prm) {
+  const Geom& g = p->g;
+  if (!(prm.kcut > 2.0 * g.mx / 3.0)) return false;
+  const double kc2 = prm.kcut * prm.kcut;
+  double cols = 0, modes = 0;  // kept; ky and -ky, kz and -kz count together
+  for (int kx = 0; kx <= g.mx; ++kx)
+    for (int ky = 0; ky <= g.ny / 2; ++ky) {
+      const double rest = kc2 - (double)kx * kx - (double)ky * ky;
+      if (!(rest > 0)) break;
+      const double w = ky == 0 || ky == g.ny / 2 ? 1 : 2;
+      cols += w;
+      modes += w * std::min((double)g.nz, 2 * std::ceil(std::sqrt(rest)) - 1);
+    }
+  const double all = (double)(g.mx + 1) * g.ny;
+  const bool dp = p->prec == SCL_DP;
+  if ((size_t)g.ntot * p->esize() < ((size_t)12 << 20)) return modes > 0.995 * all * g.nz;
+  if (prm.sgs) return cols > (prm.stepper ? (dp ? 0.88 : 0.93) : dp ? 0.82 : 0.95) * all;
+  if (prm.stepper || prm.dealias_rhs) return modes > (dp || prm.stepper ? 0.95 : 0.87) * all * g.nz;
+  return modes > (prm.scalar ? (dp ? 0.87 : 0.95) : dp ? 0.95 : 0.92) * all * g.nz;
+}
 
 template <class R>
 static RhsParams<R> rhs_params(const scl_plan3d* p, double nu, double dt, int forced, double fkmax, int dealias) {
@@ -672,6 +716,7 @@ static int32_t rk4_step_dev(scl_plan3d* p, const DevFields& d, const scl_dns_par
   RhsParams<R> rp = rhs_params<R>(p, prm.nu, prm.dt, prm.forced, prm.fkmax, prm.dealias_rhs);
   apply_kcut<R>(rp, prm);
   rp.nonfinite = d.nonfinite;
+  rp.trunc = rp.trunc && !d.whole;
   const bool chain = chain_stages<R>(p, d);
   // primed: v was written by stage 4, so it is truncated; with the RHS
   // truncated too, so is every stage state (not where the forcing would have
@@ -754,7 +799,7 @@ static int32_t rk_stage_ext(scl_plan3d* p, const DevFields& d, int mode, const s
   apply_kcut<R>(ep.r, prm);
   ep.r.nonfinite = d.nonfinite;
   ep.r.ab = ab;
-  ep.r.trunc = mode > 0 && ext_trunc(p) && !d.separate;
+  ep.r.trunc = mode > 0 && ext_trunc(p) && !d.separate && !d.whole;
   ep.r.vcut = ep.r.trunc && vcut;
   // only stage 1 and the AB2 steps read the state itself
   const R kc2_in = !ep.r.trunc || (mode > 1 && mode < 5) ? (R)0 : ep.r.vcut ? ep.r.kc2 : std::numeric_limits<R>::infinity();
@@ -869,6 +914,7 @@ static unsigned* nonfinite_flag(const scl_dns* d) { return reinterpret_cast<unsi
 static DevFields dev_fields(const scl_dns* d) {
   DevFields f{d->fields, d->plan->fstride(), d->nc, d->coef};
   f.nonfinite = nonfinite_flag(d);
+  f.whole = d->whole;
   return f;
 }
 
@@ -944,6 +990,7 @@ extern "C" int32_t scl_dns_create(scl_plan3d* p, const scl_dns_params* prm, scl_
     d->nw = std::max(L.nin(), L.nout());
   }
   if (prm->sgs == 2) d->p.use_graph = 0;  // the update step differs from the others
+  d->whole = keeps_most(p, *prm);
   const size_t fb = (size_t)p->fstride() * p->esize();
   const size_t bytes = (size_t)(3 * d->nc + d->nw) * fb;
   auto fail = [&](size_t b) {
@@ -1129,7 +1176,7 @@ static int32_t dns_launch_steps(scl_dns* d, int nsteps, Timer* tm) {
     // step is the Adams-Bashforth one.  A LES / scalar state that the caller
     // holds (state_out) is taken as it is by every step, the captured one too
     while (nsteps > 0 && ((d->p.stepper && d->ab_steps < 2) || (!d->ext && !d->chained) ||
-                          (d->ext && ext_trunc(p) && !d->truncated && !d->state_out))) {
+                          (d->ext && ext_trunc(p) && !d->truncated && !d->state_out && !d->whole))) {
       SCL_CHECK(dns_step_once<R>(d, nullptr));
       d->steps += 1;
       --nsteps;

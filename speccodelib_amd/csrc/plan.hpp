@@ -75,6 +75,9 @@ struct scl_dns {
   // it at any time, so LES / scalar steps take it as it is (truncated stays
   // false)
   bool state_out = false;
+  // the truncation radius keeps nearly all modes: the passes leave none out
+  // (keeps_most)
+  bool whole = false;
   // IF-AB2 (p.stepper 1, 2): device state (AB_* slots), energy partials, and
   // the steps taken since the state was set (selects the bootstrap modes)
   double* ab = nullptr;

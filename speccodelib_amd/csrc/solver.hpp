@@ -21,6 +21,7 @@ struct DevFields {
   // the y- and x-passes in their separate form at every size, to the bit what
   // they give there (plan.hpp's plane off)
   bool separate = false;
+  bool whole = false;  // as scl_dns
   unsigned* nonfinite = nullptr;  // sticky flag: stage 4 found a non-finite v (null: not checked)
   template <class R>
   cpx<R>* f(int i) const {
