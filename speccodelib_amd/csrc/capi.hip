@@ -601,8 +601,8 @@ struct Timer {
 // (the fused five-pass DNS RHS; nc = 3).  in_cut: the stage state is zero
 // beyond the truncation, and W (primed) holds only its kept columns; the
 // passes leave the rest out.  After the products only the kept modes are
-// computed where the step ends (mode >= 4: the new v is truncated) or the
-// RHS is truncated.
+// computed where the step ends (mode 4: the new v is truncated) or the RHS is
+// truncated.  The IF-AB2 steps (mode >= 5) leave nothing out.
 template <class R>
 static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsParams<R>& rp, double eps, double eta,
                         double fkmax, const cpx<R>* st, Timer* tm, bool primed = false, bool fuse = false,
@@ -610,9 +610,9 @@ static int32_t rk_stage(scl_plan3d* p, const DevFields& d, int mode, const RhsPa
   const int64_t fs = d.fs;
   // where a pass is cut in some steps of a run and not in others (a run's
   // first step), the same kernels do both: the results do not depend on it
-  const bool may_cut = rp.trunc && (mode == 1 || mode >= 5 || rp.dealias);
+  const bool may_cut = rp.trunc && (mode == 1 || rp.dealias);
   const R kc2_in = in_cut ? rp.kc2 : may_cut ? std::numeric_limits<R>::infinity() : (R)0,
-          kc2_out = rp.trunc && (mode >= 4 || rp.dealias) ? rp.kc2 : (R)0;
+          kc2_out = rp.trunc && (mode == 4 || rp.dealias) ? rp.kc2 : (R)0;
   cpx<R>* V = d.V<R>();
   cpx<R>* DU = d.DU<R>();
   cpx<R>* S = d.S<R>();

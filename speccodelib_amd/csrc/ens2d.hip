@@ -118,7 +118,6 @@ int32_t with_col2d(int n, int e, int cw, F&& f) {
     return SCL_EINVAL;
   };
   switch (n) {
-    case 16: return go(Int<16>{});
     case 32: return go(Int<32>{});
     case 64: return go(Int<64>{});
     case 128: return go(Int<128>{});
@@ -127,14 +126,13 @@ int32_t with_col2d(int n, int e, int cw, F&& f) {
     case 1024: return go(Int<1024>{});
     default: break;
   }
-  set_error("2D size %d is not a power of two in [16, 1024]", n);
+  set_error("2D size %d is not a power of two in [32, 1024]", n);
   return SCL_EINVAL;
 }
 
 template <class R, class F>
 int32_t with_row2d(int m, F&& f) {
   switch (m) {
-    case 8: return f(Int<8>{});
     case 16: return f(Int<16>{});
     case 32: return f(Int<32>{});
     case 64: return f(Int<64>{});

@@ -826,9 +826,8 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_rhs(cpx<R>
 // The z-passes of the IF-AB2 steps (MODE 5..7; ab_apply), over all modes.  An
 // AB2 run of a field with energy up to its truncation multiplies any rounding
 // difference (8e-8 after 20 steps becomes 1e-5 and more within the next 20), so
-// these keep to the bit what the steps have always given; the passes that leave
-// modes out (k_zfwd_rhs<5..7>) made a 256^3 step 692 -> 622 us and moved such
-// runs by up to 3.5e-5.
+// these keep to the bit what the steps have always given; passes that leave modes
+// out made a 256^3 step 692 -> 622 us and moved such runs by up to 3.5e-5.
 template <class R, int N, int E, int CW, bool PARK, int ZS>
 __device__ inline void zinv_store_all(cpx<R> (&ux)[E], cpx<R> (&uy)[E], cpx<R> (&uz)[E], cpx<R>* lds, cpx<R>* park,
                                   const cpx<R>* twl, int rt, int c, R kx, R ky, int nz, ZOff<ZS> zo,
@@ -895,7 +894,8 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zinv_all(const 
                                     wstride);
 }
 
-template <class R, int N, int MODE, int CWZ, int EZ = 0, bool FUSED = false, int ZS = 0>
+// The z-forward with the AB2 update, always fused with the z-inverse of the new v.
+template <class R, int N, int MODE, int CWZ, int EZ = 0, int ZS = 0>
 __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_ab2(cpx<R>* W, int64_t fstride, cpx<R>* V,
                                                                     cpx<R>* DU, cpx<R>* S, const cpx<R>* st,
                                                                     const double* __restrict__ coef, RhsParams<R> p,
@@ -949,7 +949,6 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_ab2(cpx<R>
     const int z = L::out_pos(m, rt);
     const int iy = kwave(t.oth, g.ny), iz = kwave(z, g.nz);
     const int ik2 = t.kx * t.kx + iy * iy + iz * iz;
-    // MODE 4 reads du only inside the cut
     const bool cut = (ik2 == 0 ? std::numeric_limits<R>::min() : (R)ik2) >= p.kc2;
     const uint32_t o = zz.at(z);
     dst[0] = stage_load<MODE, R, uint32_t, NT>(o, V, DU, S, cut);
@@ -970,24 +969,18 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_ab2(cpx<R>
     fa = (R)coef[0];
     fb = (R)coef[1];
   }
-  R ab_dt = 0, ab_dto = 0, ab_s = 0, ab_ek = 0, ab_del = 0;
-  if constexpr (MODE >= 5) {
-    ab_dt = (R)p.ab[AB_DT];
-    ab_dto = (R)p.ab[AB_DTO];
-    ab_s = (R)p.ab[AB_S];
-    ab_ek = (R)p.ab[AB_EK];
-    ab_del = (R)p.ab[AB_DELTA];
-  }
+  const R ab_dt = (R)p.ab[AB_DT], ab_dto = (R)p.ab[AB_DTO], ab_s = (R)p.ab[AB_S], ab_ek = (R)p.ab[AB_EK],
+          ab_del = (R)p.ab[AB_DELTA];
   // With the park, the new x stage state goes back to its park slot (just
   // read) until the z-inverse, which keeps 2E registers free here.
   auto keep_x = [&](int m, cpx<R> v) {
-    if constexpr (PARK && FUSED) park[m * CC::BS + threadIdx.x] = v;
+    if constexpr (PARK) park[m * CC::BS + threadIdx.x] = v;
     else nx_[m] = v;
   };
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     StageIn<R> in[3];
-    if constexpr (MODE > 0) stage_in(m, ze, in);
+    stage_in(m, ze, in);
     const int z = L::out_pos(m, rt);
     const int ikz = kwave(z, g.nz);
     const R kz = (R)ikz;
@@ -1038,13 +1031,11 @@ __global__ __launch_bounds__((ColCfg<R, N, CWZ, EZ>::BS)) void k_zfwd_ab2(cpx<R>
                                  ab_del, e1, e2, cut, p.nonfinite);
     }
   }
-  if constexpr (FUSED && MODE > 0) {
-    if constexpr (PARK) {
+  if constexpr (PARK) {
 #pragma unroll
-      for (int m = 0; m < E; ++m) nx_[m] = park[m * CC::BS + threadIdx.x];
-    }
-    zinv_store_all<R, N, E, CW, PARK, ZS>(nx_, ny_, nz_, lds, park, twl, rt, c, kx, ky, g.nz, zo, W, fstride);
+    for (int m = 0; m < E; ++m) nx_[m] = park[m * CC::BS + threadIdx.x];
   }
+  zinv_store_all<R, N, E, CW, PARK, ZS>(nx_, ny_, nz_, lds, park, twl, rt, c, kx, ky, g.nz, zo, W, fstride);
 }
 
 // Forcing coefficients from the stage state: a reduction over the box of

@@ -29,20 +29,18 @@ struct ExtOps {
 
   // N(st) of the extended RHS into W (MODE 0) or one RK4 stage (MODE 1..4).
   // W holds max(nin, nout) fields.  phys_tape (optional): where the
-  // physical-space u, w, S_ij of this evaluation are kept (k_ext_phys).  fa:
+  // physical-space u, w, S_ij of this evaluation are kept, by the separate
+  // passes (k_row_ext, k_ext_phys).  fa:
   // the forcing coefficients the combine reads (type 0: there already, or not
   // forced).  begun(): called where the transforms start.  separate: as
   // DevFields.  kc2_in: the truncation st is known to have (infinite: it may
   // have one in another step; 0: none); ep.r.trunc: as RhsParams.
-  static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
-                     const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape = nullptr) {
-    return rhs(pl, mode, L, W, fs, V, DU, S, st, coef, ep, delta2, phys_tape, ForceArgs<R>{}, [] {}, false, (R)0);
-  }
   template <class F>
   static int32_t rhs(const scl_plan3d& pl, int mode, ExtLayout L, C* W, int64_t fs, C* V, C* DU, C* S, const C* st,
                      const double* coef, const ExtParams<R>& ep, R delta2, C* phys_tape, const ForceArgs<R>& fa,
                      F&& begun, bool separate, R kc2_in) {
     const Geom& g = pl.g;
+    separate = separate || phys_tape;
     const bool plane = !separate && pl.zfused && Ops<R>::plane_fits(pl, L.les, L.scalar);
     const bool sy = !separate && pl.zfused && !plane && Ops<R>::split_y(pl, L.les, L.scalar);
     if (fa.type && !plane && !sy) {
@@ -66,7 +64,7 @@ struct ExtOps {
     // physical products; y-forward
     const R scale = (R)1 / (R)((double)g.nx * g.ny * g.nz);
     if (plane) {
-      SCL_CHECK(Ops<R>::plane(pl, W, fs, L.les, L.scalar, scale, delta2, (R)(-ep.sign_phi), coef + 5, phys_tape, fa, kc2_in,
+      SCL_CHECK(Ops<R>::plane(pl, W, fs, L.les, L.scalar, scale, delta2, (R)(-ep.sign_phi), coef + 5, nullptr, fa, kc2_in,
                               kc2_out));
       return Ops<R>::ext_zfwd(pl, mode, W, fs, V, DU, S, st, coef, ep, L);
     }
@@ -74,7 +72,7 @@ struct ExtOps {
     else if (fused) SCL_CHECK(Ops<R>::ext_yinv(pl, W, fs, L, kc2_in));
     else SCL_CHECK(Ops<R>::colfft(pl, W, fs, L.nin(), 1, +1));
     if (!separate && Ops<R>::split_x(pl, L.les, L.scalar))
-      SCL_CHECK(Ops<R>::row_split(pl, W, fs, L.les, L.scalar, scale, delta2, coef + 5, phys_tape, kc2_in,
+      SCL_CHECK(Ops<R>::row_split(pl, W, fs, L.les, L.scalar, scale, delta2, coef + 5, nullptr, kc2_in,
                                   sy ? (R)0 : kc2_out));
     else
       SCL_CHECK(Ops<R>::row_ext(pl, W, fs, L, scale, delta2, coef + 5, phys_tape, kc2_in, sy ? (R)0 : kc2_out));

@@ -228,7 +228,7 @@ int32_t Ops<R>::zfwd_rhs(const scl_plan3d& pl, int mode, C* W, int64_t fstride, 
         // short lines come in both variants: their grids can be so small
         // that the instructions of the unused one are felt (Cut)
         if constexpr (MODE >= 5) {
-          go(k_zfwd_ab2<R, N, MODE, CW, EZ, FUSED, ZS>);
+          go(k_zfwd_ab2<R, N, MODE, CW, EZ, ZS>);
         } else {
           if constexpr (N <= 64) {
             if (!p.trunc) return go(k_zfwd_rhs<R, N, MODE, CW, EZ, FUSED, ZS, false>);
@@ -301,16 +301,20 @@ int32_t Ops<R>::ext_yinv(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout
     constexpr int N = decltype(NC)::value;
     using CC = ColCfg<R, N>;
     SCL_CHECK((check_cols<R, N>(g)));
-    const Cut<R> cut = cut_of<R>(g, kc2);
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(ycut_grid<CC::CW>(g, cut.nkx)), dim3(CC::BS), 0, pl.stream, W, fs, g, twp<R>(pl),
-                         pl.L / N, cut);
-      return check_launch("yinv_les");
-    };
-    SCL_CHECK(kc2 > 0 ? go(k_yinv_les<R, N, 0, true>) : go(k_yinv_les<R, N, 0>));
-    SCL_CHECK(kc2 > 0 ? go(k_yinv_les<R, N, 1, true>) : go(k_yinv_les<R, N, 1>));
-    // S_33 (= i kz u_z after the z-pass) and phi: a plain y-inverse
-    return colfft(pl, W + (L.s_in() + 5) * fs, fs, 1 + L.scalar, 1, +1, kc2);
+    if constexpr (N >= 1024) {
+      return set_error("fused LES y-pass: 1024-point lines take the unfused path"), SCL_EINVAL;
+    } else {
+      const Cut<R> cut = cut_of<R>(g, kc2);
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(ycut_grid<CC::CW>(g, cut.nkx)), dim3(CC::BS), 0, pl.stream, W, fs, g, twp<R>(pl),
+                           pl.L / N, cut);
+        return check_launch("yinv_les");
+      };
+      SCL_CHECK(kc2 > 0 ? go(k_yinv_les<R, N, 0, true>) : go(k_yinv_les<R, N, 0>));
+      SCL_CHECK(kc2 > 0 ? go(k_yinv_les<R, N, 1, true>) : go(k_yinv_les<R, N, 1>));
+      // S_33 (= i kz u_z after the z-pass) and phi: a plain y-inverse
+      return colfft(pl, W + (L.s_in() + 5) * fs, fs, 1 + L.scalar, 1, +1, kc2);
+    }
   });
 }
 
@@ -321,22 +325,26 @@ int32_t Ops<R>::ext_yfwd(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout
     constexpr int N = decltype(NC)::value;
     using CC = ColCfg<R, N>;
     SCL_CHECK((check_cols<R, N>(g)));
-    const Cut<R> cut = cut_of<R>(g, kc2);
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(ycut_grid<CC::CW>(g, cut.nkx)), dim3(CC::BS), 0, pl.stream, W, fs, g, sg,
-                         twp<R>(pl), pl.L / N, cut);
-      return check_launch("yfwd_ext");
-    };
-    if (!L.les && !L.scalar) return set_error("ext_yfwd: neither a Smagorinsky term nor a scalar"), SCL_EINVAL;
-    if (L.les) {
-      if (L.scalar) SCL_CHECK(kc2 > 0 ? go(k_yfwd_ext<R, N, 0, 1, true>) : go(k_yfwd_ext<R, N, 0, 1>));
-      else SCL_CHECK(kc2 > 0 ? go(k_yfwd_ext<R, N, 0, 0, true>) : go(k_yfwd_ext<R, N, 0, 0>));
+    if constexpr (N >= 1024) {
+      return set_error("fused LES y-pass: 1024-point lines take the unfused path"), SCL_EINVAL;
     } else {
-      SCL_CHECK(colfft(pl, W, fs, 3, 1, -1, kc2));  // N alone
+      const Cut<R> cut = cut_of<R>(g, kc2);
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(ycut_grid<CC::CW>(g, cut.nkx)), dim3(CC::BS), 0, pl.stream, W, fs, g, sg,
+                           twp<R>(pl), pl.L / N, cut);
+        return check_launch("yfwd_ext");
+      };
+      if (!L.les && !L.scalar) return set_error("ext_yfwd: neither a Smagorinsky term nor a scalar"), SCL_EINVAL;
+      if (L.les) {
+        if (L.scalar) SCL_CHECK(kc2 > 0 ? go(k_yfwd_ext<R, N, 0, 1, true>) : go(k_yfwd_ext<R, N, 0, 1>));
+        else SCL_CHECK(kc2 > 0 ? go(k_yfwd_ext<R, N, 0, 0, true>) : go(k_yfwd_ext<R, N, 0, 0>));
+      } else {
+        SCL_CHECK(colfft(pl, W, fs, 3, 1, -1, kc2));  // N alone
+      }
+      if (!L.scalar) return SCL_OK;
+      // the flux slots are W[3..5] with or without the Smagorinsky term
+      return kc2 > 0 ? go(k_yfwd_ext<R, N, 1, 1, true>) : go(k_yfwd_ext<R, N, 1, 1>);
     }
-    if (!L.scalar) return SCL_OK;
-    // the flux slots are W[3..5] with or without the Smagorinsky term
-    return kc2 > 0 ? go(k_yfwd_ext<R, N, 1, 1, true>) : go(k_yfwd_ext<R, N, 1, 1>);
   });
 }
 
@@ -547,6 +555,7 @@ template <class R>
 int32_t Ops<R>::plane(const scl_plan3d& pl, C* W, int64_t fs, int les, int sc, R scale, R d2, R sg,
                       const double* cs2p, C* tape, const ForceArgs<R>& fa, R kc2_in, R kc2_out) {
   const Geom& g = pl.g;
+  if (tape && (les || sc)) return set_error("plane pass: the LES tape is row_ext's"), SCL_EINVAL;
   const bool fits = with_plane<R>(pl, les, sc, [&](auto cfg, auto kern) {
     hipLaunchKernelGGL(kern, dim3(g.nz + (fa.type ? 1 : 0)), dim3(decltype(cfg)::BS), 0, pl.stream, W, fs, g, scale,
                        d2, sg, cs2p, twp<R>(pl), pl.L, cut_of<R>(g, kc2_in), cut_of<R>(g, kc2_out), tape, fa);
@@ -611,7 +620,7 @@ int32_t Ops<R>::yinv_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int 
   const Cut<R> in = cut_of<R>(g, kc2);
   return with_line<R>(g.ny, [&](auto NC) -> int32_t {
     constexpr int N = decltype(NC)::value;
-    if constexpr (N <= 512) {
+    if constexpr (N <= 256) {  // split_y
       return with_layout(les, sc, [&](auto LC, auto SC) -> int32_t {
         constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
         using C2 = SplitY<R, N, LES, S>;
@@ -631,7 +640,7 @@ int32_t Ops<R>::yfwd_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int 
   const Geom& g = pl.g;
   return with_line<R>(g.ny, [&](auto NC) -> int32_t {
     constexpr int N = decltype(NC)::value;
-    if constexpr (N <= 512) {
+    if constexpr (N <= 256) {  // split_y
       return with_layout(les, sc, [&](auto LC, auto SC) -> int32_t {
         constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
         using C2 = SplitY<R, N, LES, S>;
@@ -655,12 +664,18 @@ int32_t Ops<R>::row_split(const scl_plan3d& pl, C* W, int64_t fs, int les, int s
     constexpr int M = decltype(MC)::value;
     return with_layout(les, sc, [&](auto LC, auto SC) -> int32_t {
       constexpr int LES = decltype(LC)::value, S = decltype(SC)::value;
-      using C2 = SplitX<R, M, LES, S>;
-      if (g.nrow % C2::RW) return set_error("%lld rows: not whole groups of %d", (long long)g.nrow, C2::RW), SCL_EINVAL;
-      hipLaunchKernelGGL((k_row_split<R, M, LES, S>), dim3((unsigned)(g.nrow / C2::RW) + (fa.type ? 1 : 0)),
-                         dim3(64 * C2::NF), 0, pl.stream, W, fs, g, scale, d2, cs2p, tape, twp<R>(pl), pl.L / M,
-                         pl.L / g.nx, kin, kout, fa);
-      return check_launch("row_split");
+      if constexpr (M < 16) {  // split_x
+        return set_error("rows of %d entries: no wavefront per field", M), SCL_EINVAL;
+      } else {
+        using C2 = SplitX<R, M, LES, S>;
+        if (tape && (LES || S)) return set_error("row_split: the LES tape is row_ext's"), SCL_EINVAL;
+        if (g.nrow % C2::RW)
+          return set_error("%lld rows: not whole groups of %d", (long long)g.nrow, C2::RW), SCL_EINVAL;
+        hipLaunchKernelGGL((k_row_split<R, M, LES, S>), dim3((unsigned)(g.nrow / C2::RW) + (fa.type ? 1 : 0)),
+                           dim3(64 * C2::NF), 0, pl.stream, W, fs, g, scale, d2, cs2p, tape, twp<R>(pl), pl.L / M,
+                           pl.L / g.nx, kin, kout, fa);
+        return check_launch("row_split");
+      }
     });
   });
 }

@@ -4,7 +4,7 @@
 // (kx, ky) planes of all its fields fit in the 160 KB of one CU's LDS, one
 // workgroup takes a plane through the y-inverse, the c2r along x, the
 // physical products, the r2c and the y-forward: of the 26 F that the separate
-// passes of a DNS RHS move (F: one field), 8 F are left, and of its four
+// passes of a DNS RHS move (F: one field), 8 F are left, and of its five
 // launches (with the forcing coefficients', which a workgroup of their own
 // does on the side) one.  Small grids are bound by launches and by chains of
 // dependent passes: there each line transform belongs to one wavefront, which
@@ -117,8 +117,8 @@ __host__ __device__ constexpr PlaneForm plane_form() {
 
 // One workgroup per z-plane, and, with forcing, one more for its coefficients.
 // in, out: the truncation of the inputs (columns outside hold nothing) and of
-// the outputs (not wanted outside).  tape: u, w [, S_ij] in physical space, as
-// k_row_convec and k_row_ext leave them.  The workgroup reads all it needs of
+// the outputs (not wanted outside).  tape (DNS): u, w in physical space, as
+// k_row_convec leaves them.  The workgroup reads all it needs of
 // its plane of W before it writes any of it.
 template <class R, int M, int NY, int LES, int SC>
 __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
@@ -212,9 +212,8 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
 
   // x-lines: the rows of n planes in one list, RW of them a tile
   const int xs = lane / TX, xr = lane % TX;
-  // c2r of the planes from to on, in place; the physical rows also to the
-  // tape's fields from tf on (tf < 0: not)
-  auto c2r = [&](int to, int n, int tf) {
+  // c2r of the planes from to on, in place; the physical rows also to the tape
+  auto c2r = [&](int to, int n) {
     using Ln = Line<R, M, 8, +1, true>;
     const int rows = n * NY;
     for (int task = wave; task * RW < rows; task += NW) {
@@ -232,10 +231,12 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
       Ln::run(a, sh, xr, twM, 1, at);
 #pragma unroll
       for (int m = 0; m < 8; ++m) sh[at(Ln::out_pos(m, xr))] = a[m];
-      if (tape && tf >= 0 && ok) {
-        cpx<R>* const tb = tape + (tf + q) * fs + g.row(y, z) * M;
+      if constexpr (LES == 0 && SC == 0) {
+        if (tape && ok) {
+          cpx<R>* const tb = tape + (to + q) * fs + g.row(y, z) * M;
 #pragma unroll
-        for (int m = 0; m < 8; ++m) tb[Ln::out_pos(m, xr)] = a[m];
+          for (int m = 0; m < 8; ++m) tb[Ln::out_pos(m, xr)] = a[m];
+        }
       }
     }
   };
@@ -261,8 +262,8 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
   y_inverse(0, 6, 0, wave);
   if constexpr (SC != 0) y_inverse(X.phi_in(), 1, 6, wave);
   __syncthreads();
-  c2r(0, 6, 0);
-  if constexpr (SC != 0) c2r(6, 1, -1);
+  c2r(0, 6);
+  if constexpr (SC != 0) c2r(6, 1);
   __syncthreads();
   // u x w and u_j phi on the packed reals, in place (convec_dns.f90:30-42,
   // convecphi_dns.f90:23,33,42)
@@ -293,7 +294,7 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
     // wavefront after the last of the r2c's
     y_inverse(X.s_in(), 6, S0, (wave + NW - ((3 + 3 * SC) * NY / RW) % NW) % NW);
     __syncthreads();
-    c2r(S0, 6, 6);
+    c2r(S0, 6);
     __syncthreads();
     // tau_ij = -2 cs2 D^2 |S| S_ij (dynsmag.f90:206-225)
     const R c = (R)(-2.0 * cs2p[0]) * d2 * scale;
@@ -427,10 +428,7 @@ __global__ __launch_bounds__((PlaneCfg<R, M, NY, LES, SC>::BS)) void k_plane(
 // fields' transforms run side by side, and the products pass through LDS.
 // --------------------------------------------------------------------------
 
-// YINV of all the fields of a RHS (plane_form), in place: all wavefronts of
-// the workgroup have read their columns before any writes.  One workgroup more
-// than there are tiles computes the forcing coefficients (fa.type).  in: as
-// k_colfft's.
+// The y-passes with a wavefront per field.
 template <class R, int NY, int LES, int SC>
 struct SplitY {
   static constexpr int TY = NY / 8, CW = 64 / TY;
@@ -439,6 +437,10 @@ struct SplitY {
   static constexpr int LINE = lds_pad(NY) * CW;   // LDS entries of a wavefront
 };
 
+// YINV of all the fields of a RHS (plane_form), in place: all wavefronts of
+// the workgroup have read their columns before any writes.  One workgroup more
+// than there are tiles computes the forcing coefficients (fa.type).  in: as
+// k_colfft's.
 template <class R, int NY, int LES, int SC>
 __global__ __launch_bounds__((64 * SplitY<R, NY, LES, SC>::NF)) void k_yinv_split(cpx<R>* W, int64_t fs, Geom g,
                                                                                const cpx<R>* __restrict__ tw, int tws,
@@ -567,7 +569,7 @@ __global__ __launch_bounds__((64 * SplitY<R, NY, LES, SC>::KINDS)) void k_yfwd_s
 // XPASS with the products of k_row_convec / k_row_ext, a wavefront per field.
 // A wavefront holds 512/M rows of its field, every wavefront's lane the same
 // points, so the physical values pass through LDS as [field][slot][lane].
-// kin, kout, tape: as k_row_convec (k_row_ext: all).  One workgroup more than
+// kin, kout, tape (DNS): as k_row_convec.  One workgroup more than
 // there are row groups computes the forcing coefficients (fa.type).
 template <class R, int M, int LES, int SC>
 struct SplitX {
@@ -612,10 +614,12 @@ __global__ __launch_bounds__((64 * SplitX<R, M, LES, SC>::NF)) void k_row_split(
   }
   using Li = Line<R, M, 8, +1, true>;
   Li::run(v, ex, rt, twM, 1, LinIdx{});
-  if (tape && f < 6 + 6 * LES) {
-    cpx<R>* const tb = tape + f * fs + row * M;
+  if constexpr (LES == 0 && SC == 0) {
+    if (tape) {
+      cpx<R>* const tb = tape + f * fs + row * M;
 #pragma unroll
-    for (int m = 0; m < 8; ++m) tb[Li::out_pos(m, rt)] = v[m];
+      for (int m = 0; m < 8; ++m) tb[Li::out_pos(m, rt)] = v[m];
+    }
   }
 #pragma unroll
   for (int m = 0; m < 8; ++m) own[m * 64 + lane] = v[m];
