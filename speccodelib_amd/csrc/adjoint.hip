@@ -412,7 +412,9 @@ extern "C" int32_t scl_adjoint_create(scl_plan3d* p, const scl_dns_params* prm, 
     return set_error("SCL_ADJ_PHYS_TAPE=1: no physical tape (it needs z- and y-lines below 1024 points and memory)"),
            SCL_EINVAL;
   }
-  if (hipMemset(a->fields, 0, fb * (9 + a->nw)) != hipSuccess || hipMemset(a->coef, 0, 8 * sizeof(double)) != hipSuccess ||
+  // on the plan's stream, in order before the first forward's copies
+  if (hipMemsetAsync(a->fields, 0, fb * (9 + a->nw), p->stream) != hipSuccess ||
+      hipMemsetAsync(a->coef, 0, 8 * sizeof(double), p->stream) != hipSuccess ||
       hipEventCreate(&a->e0) != hipSuccess || hipEventCreate(&a->e1) != hipSuccess) {
     scl_adjoint_destroy(a);
     return set_error("adjoint set-up failed"), SCL_EHIP;

@@ -272,9 +272,12 @@ extern "C" int32_t scl_plan3d_create(int32_t nx, int32_t ny, int32_t nz, int32_t
     std::vector<cpx<R>> h(p->L);
     for (int j = 0; j < p->L; ++j) h[j] = mk<R>((R)re[j], (R)im[j]);
     SCL_HIP(hipMalloc(&p->tw, p->L * sizeof(cpx<R>)));
-    SCL_HIP(hipMemcpy(p->tw, h.data(), p->L * sizeof(cpx<R>), hipMemcpyHostToDevice));
     SCL_HIP(hipMalloc((void**)&p->coef, 8 * sizeof(double)));
-    SCL_HIP(hipMemset(p->coef, 0, 8 * sizeof(double)));
+    // on the plan's stream, which does not wait for the legacy stream; and the
+    // legacy stream would end a capture that another thread has going
+    SCL_HIP(hipMemcpyAsync(p->tw, h.data(), p->L * sizeof(cpx<R>), hipMemcpyHostToDevice, p->stream));
+    SCL_HIP(hipMemsetAsync(p->coef, 0, 8 * sizeof(double), p->stream));
+    SCL_HIP(hipStreamSynchronize(p->stream));
     return SCL_OK;
   });
   if (st != SCL_OK) {
@@ -1430,7 +1433,8 @@ extern "C" int32_t scl_dns_diagnostics(scl_dns* d, scl_diag* out) {
       out->scalar_dissipation = 2.0 * d->p.nu / d->p.schmidt * kvar;
     }
     double c[8];
-    SCL_HIP(hipMemcpy(c, d->coef, sizeof(c), hipMemcpyDeviceToHost));
+    SCL_HIP(hipMemcpyAsync(c, d->coef, sizeof(c), hipMemcpyDeviceToHost, p->stream));
+    SCL_HIP(hipStreamSynchronize(p->stream));
     out->cs2 = d->p.sgs ? c[5] : 0.0;
     SCL_CHECK(skewness_run<R>(p, v, &out->skewness));
     SCL_CHECK(divmax_run<R>(p, v, &out->divmax));

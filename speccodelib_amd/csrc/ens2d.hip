@@ -660,13 +660,15 @@ int32_t allocate_groups(scl_ens2d& e) {
 }
 
 template <class R>
-int32_t upload_twiddles(int n, void** out) {
+int32_t upload_twiddles(int n, void** out, hipStream_t st) {
   std::vector<double> re, im;
   twiddles(n, re, im);
   std::vector<cpx<R>> h(n);
   for (int j = 0; j < n; ++j) h[j] = mk<R>((R)re[j], (R)im[j]);
   SCL_HIP(hipMalloc(out, n * sizeof(cpx<R>)));
-  SCL_HIP(hipMemcpy(*out, h.data(), n * sizeof(cpx<R>), hipMemcpyHostToDevice));
+  // not on the legacy stream, which would end another thread's capture
+  SCL_HIP(hipMemcpyAsync(*out, h.data(), n * sizeof(cpx<R>), hipMemcpyHostToDevice, st));
+  SCL_HIP(hipStreamSynchronize(st));
   return SCL_OK;
 }
 
@@ -727,7 +729,7 @@ extern "C" int32_t scl_ens2d_create(int32_t prec, int32_t ngroups, const int32_t
       if (t.first == n) tw = t.second;
     if (!tw) {
       void* d = nullptr;
-      const int32_t st = prec == SCL_SP ? upload_twiddles<float>(n, &d) : upload_twiddles<double>(n, &d);
+      const int32_t st = prec == SCL_SP ? upload_twiddles<float>(n, &d, e->stream) : upload_twiddles<double>(n, &d, e->stream);
       if (st != SCL_OK) return fail(st);
       e->tw.push_back({n, d});
       tw = d;

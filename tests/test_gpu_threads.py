@@ -1,0 +1,95 @@
+"""Threads that each have their own solvers, ensembles and adjoints (GPU): making
+one does not disturb a step that another thread is capturing, and what a thread
+computes has the bits that it has alone."""
+import threading
+
+import numpy as np
+import pytest
+
+import speccodelib_amd as scl
+
+pytestmark = pytest.mark.gpu
+
+N = 32
+
+
+def dns():
+    p = scl.Plan3D(N, N, N, scl.SP)
+    d = scl.DNS(p, nu=0.02, dt=1e-3, forced=1, fkmax=2.5, eps=0.1)
+    d.set_velocity(*scl.initialize(N, N, N, 1, 4.0, 1.0, scl.SP))
+    d.step(3)
+    out = [*d.get_velocity(), d.diagnostics()["energy"]]
+    d.close()
+    p.close()
+    return out
+
+
+def les():
+    p = scl.Plan3D(N, N, N, scl.DP)
+    d = scl.DNS(p, nu=0.02, dt=1e-3, forced=1, fkmax=2.5, eps=0.1, sgs=1, cs2=0.03)
+    d.set_velocity(*scl.initialize(N, N, N, 2, 4.0, 1.0, scl.DP))
+    d.step(3)
+    out = [*d.get_velocity()]
+    d.close()
+    p.close()
+    return out
+
+
+def ensemble():
+    e = scl.Ensemble2D([(32, 2), (64, 1)], dt=1e-4)
+    e.initialize()
+    e.step(12)
+    out = [e.get_member(0, 1).copy(), e.get_member(1, 0).copy()]
+    e.close()
+    return out
+
+
+def adjoint():
+    p = scl.Plan3D(16, 16, 16, scl.SP)
+    a = scl.Adjoint(p, 2, 1, nu=0.02, dt=1e-3, sgs=1)
+    u = scl.initialize(16, 16, 16, 1, 4.0, 1.0, scl.SP)
+    out = [*a.forward(u, 0.03)]
+    g, c = a.backward(u)
+    a.close()
+    p.close()
+    return out + [*g, c]
+
+
+def test_threads_do_not_disturb_each_other():
+    work = [dns, les, ensemble, adjoint]
+    want = {f: f() for f in work}
+    failures = []
+
+    def run(k):
+        try:
+            for i in range(24):
+                f = work[(i + k) % len(work)]
+                for a, b in zip(f(), want[f]):
+                    np.testing.assert_array_equal(a, b)
+        except Exception as ex:
+            failures.append(f"thread {k}: {type(ex).__name__}: {ex}")
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, "\n".join(failures)
+
+
+def test_a_fresh_adjoint_gives_what_a_used_one_gives():
+    # its set-up has to be over before the first forward's copies: large work
+    # fields, a small first forward
+    n = 64
+    u = scl.initialize(n, n, n, 1, 4.0, 1.0, scl.DP)
+    p = scl.Plan3D(n, n, n, scl.DP)
+    used = scl.Adjoint(p, 1, 1, nu=0.02, dt=1e-3, sgs=1)
+    used.forward(u, 0.03)
+    want = used.forward(u, 0.03)
+    for _ in range(5):
+        a = scl.Adjoint(p, 1, 1, nu=0.02, dt=1e-3, sgs=1)
+        for x, y in zip(a.forward(u, 0.03), want):
+            np.testing.assert_array_equal(x, y)
+        a.close()
+    used.close()
+    p.close()
