@@ -98,8 +98,22 @@ int32_t staging_of(scl_plan3d* p, cpx<R>** st) {
   return SCL_OK;
 }
 
+// nf fields to evaluate a right-hand side with: the solver's, which are free
+// between IF-RK4 steps, or, where they hold an IF-AB2 run's history, the plan's.
+template <class R>
+int32_t rhs_fields(scl_dns* d, int nf, cpx<R>** out) {
+  if (!d->p.stepper) {
+    *out = DevFields{d->fields, d->plan->fstride(), d->nc, d->coef}.template DU<R>();
+    return SCL_OK;
+  }
+  void* s;
+  SCL_CHECK(plan_scratch(d->plan, nf, &s));
+  *out = reinterpret_cast<cpx<R>*>(s);
+  return SCL_OK;
+}
+
 // N(st) - nu k^2 st (linear = true) or N(st) into out (split layout, nc
-// fields), st = S of the solver.
+// fields).
 template <class R>
 int32_t rhs_split(scl_dns* d, const cpx<R>* st, cpx<R>* out, bool linear) {
   d->chained = false;  // W is overwritten
@@ -117,10 +131,10 @@ template <class R>
 int32_t dns_rhs(scl_dns* d, const void* const* y, void* const* dydt, bool dev) {
   scl_plan3d* p = d->plan;
   const int64_t fs = p->fstride();
-  DevFields f{d->fields, fs, d->nc, d->coef};
-  cpx<R>* S = f.S<R>();
-  cpx<R>* st = nullptr;
+  cpx<R>*out = nullptr, *st = nullptr;
+  SCL_CHECK(rhs_fields<R>(d, 2 * d->nc, &out));
   SCL_CHECK(staging_of<R>(p, &st));
+  cpx<R>* const S = out + d->nc * fs;
   for (int q = 0; q < d->nc; ++q) {
     if (!y[q] || !dydt[q]) return set_error("null array"), SCL_EINVAL;
     const cpx<R>* src = reinterpret_cast<const cpx<R>*>(y[q]);
@@ -130,8 +144,6 @@ int32_t dns_rhs(scl_dns* d, const void* const* y, void* const* dydt, bool dev) {
     }
     SCL_CHECK(Ops<R>::ref_to_split(*p, src, S + q * fs));
   }
-  // the result goes to DU (free between steps), then out in the reference layout
-  cpx<R>* out = f.DU<R>();
   SCL_CHECK(rhs_split<R>(d, S, out, true));
   for (int q = 0; q < d->nc; ++q) {
     if (dev) {
@@ -199,8 +211,8 @@ extern "C" int32_t scl_dns_derivs_cb(void* ctx, double t, const void* y, void* d
   return by_prec_p(p->prec, [&](auto zero) -> int32_t {
     using R = decltype(zero);
     const int64_t fs = p->fstride();
-    DevFields f{d->fields, fs, d->nc, d->coef};
-    cpx<R>* S = f.S<R>();
+    cpx<R>* S = nullptr;
+    SCL_CHECK(rhs_fields<R>(d, d->nc, &S));
     SCL_HIP(hipMemcpyAsync(S, y, d->nc * fs * sizeof(cpx<R>), hipMemcpyDeviceToDevice, p->stream));
     SCL_CHECK(rhs_split<R>(d, S, reinterpret_cast<cpx<R>*>(dydt), false));
     SCL_HIP(hipStreamSynchronize(p->stream));
