@@ -313,10 +313,13 @@ int32_t scl_dns_step_timed(scl_dns *d, int32_t nsteps, double *kind_ms, int32_t 
 int32_t scl_dns_rhs(scl_dns *d, double t, const void *const *y, void *const *dydt, int32_t on_device);
 /* The solver's state on the device: nc fields of the split layout, *n
  * complex entries in all (the layout of scl_dns_derivs_cb's arrays).  The
- * caller may change the state through the pointer before the next step.  A
- * solver with a Smagorinsky term or a scalar takes it as it is at every later
- * step too, and the pointer can be kept.  The others carry transforms of the
- * state from step to step: ask again before changing it after a step. */
+ * caller may read the state through the pointer after any step
+ * (scl_dns_sync), and change it before the next one.  To change it again
+ * after a step, ask for the pointer again: a solver carries what it knows of
+ * its state from step to step (transforms of it; that nothing is left beyond
+ * the truncation radius), and forgets it here, where a state is set, and
+ * where one of its right-hand sides is evaluated (scl_dns_rhs,
+ * scl_dns_derivs_cb). */
 int32_t scl_dns_state(scl_dns *d, void **state, int64_t *n);
 /* nu k^2 (scalar: nu/Sc k^2) per state entry into a device array of *n reals. */
 int32_t scl_dns_rates(scl_dns *d, void *rate);

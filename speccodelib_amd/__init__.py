@@ -510,7 +510,9 @@ class DNS:
         return tuple(out)
 
     def state(self):
-        """(device pointer, complex entries) of the state in the split layout."""
+        """(device pointer, complex entries) of the state in the split layout.
+        It can be read after any step; ask again before changing the state
+        through it after a step."""
         ptr = ctypes.c_void_p()
         n = ctypes.c_int64()
         _check(lib().scl_dns_state(self.h, ctypes.byref(ptr), ctypes.byref(n)))

@@ -1157,14 +1157,14 @@ static int32_t dns_step_once(scl_dns* d, Timer* tm) {
     SCL_CHECK(rk_stage_ext<R>(p, f, mode, prm, f.V<R>(), tm, d->ab, vcut));
     SCL_CHECK(ab_end(p, d->ab));
     d->ab_steps += 1;
-    d->truncated = !d->state_out;
+    d->truncated = true;
     return SCL_OK;
   }
   for (int stage = 1; stage <= 4; ++stage) {
     const cpx<R>* st = stage == 1 ? f.V<R>() : f.S<R>();
     SCL_CHECK(rk_stage_ext<R>(p, f, stage, prm, st, tm, nullptr, vcut));
   }
-  d->truncated = !d->state_out;
+  d->truncated = true;
   return SCL_OK;
 }
 
@@ -1176,10 +1176,9 @@ static int32_t dns_launch_steps(scl_dns* d, int nsteps, Timer* tm) {
     // The first step after the state was set runs eagerly: it starts the
     // chain and takes v as it was given, not truncated; the captured step is
     // the chained one.  IF-AB2: so do the two bootstrap steps; the captured
-    // step is the Adams-Bashforth one.  A LES / scalar state that the caller
-    // holds (state_out) is taken as it is by every step, the captured one too
+    // step is the Adams-Bashforth one
     while (nsteps > 0 && ((d->p.stepper && d->ab_steps < 2) || (!d->ext && !d->chained) ||
-                          (d->ext && ext_trunc(p) && !d->truncated && !d->state_out && !d->whole))) {
+                          (d->ext && ext_trunc(p) && !d->truncated && !d->whole))) {
       SCL_CHECK(dns_step_once<R>(d, nullptr));
       d->steps += 1;
       --nsteps;

@@ -116,7 +116,9 @@ int32_t rhs_fields(scl_dns* d, int nf, cpx<R>** out) {
 // fields).
 template <class R>
 int32_t rhs_split(scl_dns* d, const cpx<R>* st, cpx<R>* out, bool linear) {
-  d->chained = false;  // W is overwritten
+  // W is overwritten; and who evaluates right-hand sides of this solver may be
+  // stepping its state in place (scl_ifrk4_integrate)
+  d->chained = d->truncated = false;
   scl_plan3d* p = d->plan;
   DevFields f{d->fields, p->fstride(), d->nc, d->coef};
   SCL_CHECK(solver_stage<R>(p, f, 0, d->p, st));
@@ -173,18 +175,9 @@ extern "C" int32_t scl_dns_rhs(scl_dns* d, double t, const void* const* y, void*
 
 extern "C" int32_t scl_dns_state(scl_dns* d, void** state, int64_t* n) {
   if (!d || !state || !n) return set_error("null argument"), SCL_EINVAL;
-  if (d->ext && !d->state_out && d->exec) {
-    // the captured step takes the state to be truncated
-    SCL_HIP(hipStreamSynchronize(d->plan->stream));
-    (void)hipGraphExecDestroy(d->exec);
-    (void)hipGraphDestroy(d->graph);
-    d->exec = nullptr;
-    d->graph = nullptr;
-  }
   *state = d->fields;
   *n = (int64_t)d->nc * d->plan->fstride();
   d->chained = d->truncated = false;  // the caller may change the state through the pointer
-  d->state_out = true;
   return SCL_OK;
 }
 

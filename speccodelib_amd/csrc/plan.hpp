@@ -71,10 +71,6 @@ struct scl_dns {
   // LES / scalar: the state is zero beyond the truncation (a step has left it
   // so); cleared with chained
   bool truncated = false;
-  // scl_dns_state has given the state's address out: the caller may write to
-  // it at any time, so LES / scalar steps take it as it is (truncated stays
-  // false)
-  bool state_out = false;
   // the truncation radius keeps nearly all modes: the passes leave none out
   // (keeps_most)
   bool whole = false;
