@@ -551,22 +551,35 @@ static bool trunc_pays(const scl_plan3d* p) { return (size_t)p->g.ntot * p->esiz
 static bool keeps_most(const scl_plan3d* p, const scl_dns_params& prm) {
   const Geom& g = p->g;
   if (!(prm.kcut > 2.0 * g.mx / 3.0)) return false;
+  if (prm.stepper && !prm.sgs && !prm.scalar) return false;  // leaves nothing out anyway
   const double kc2 = prm.kcut * prm.kcut;
-  double cols = 0, modes = 0;  // kept; ky and -ky, kz and -kz count together
-  for (int kx = 0; kx <= g.mx; ++kx)
-    for (int ky = 0; ky <= g.ny / 2; ++ky) {
-      const double rest = kc2 - (double)kx * kx - (double)ky * ky;
-      if (!(rest > 0)) break;
-      const double w = ky == 0 || ky == g.ny / 2 ? 1 : 2;
-      cols += w;
-      modes += w * std::min((double)g.nz, 2 * std::ceil(std::sqrt(rest)) - 1);
-    }
+  const bool dp = p->prec == SCL_DP, small = (size_t)g.ntot * p->esize() < ((size_t)12 << 20);
+  // ky and -ky, kz and -kz count together; n: the first one beyond, up to n/2 + 1
+  auto both = [](int n, int all) { return (int64_t)std::min(all, 2 * n - 1); };
+  auto beyond = [&](int64_t k2, int& n) {
+    while (n > 0 && !((double)(k2 + (int64_t)(n - 1) * (n - 1)) < kc2)) --n;
+  };
+  int64_t cols = 0;
+  for (int kx = 0, ky = g.ny / 2 + 1; kx <= g.mx; ++kx) {
+    beyond((int64_t)kx * kx, ky);
+    if (ky == 0) break;
+    cols += both(ky, g.ny);
+  }
   const double all = (double)(g.mx + 1) * g.ny;
-  const bool dp = p->prec == SCL_DP;
-  if ((size_t)g.ntot * p->esize() < ((size_t)12 << 20)) return modes > 0.995 * all * g.nz;
-  if (prm.sgs) return cols > (prm.stepper ? (dp ? 0.88 : 0.93) : dp ? 0.82 : 0.95) * all;
-  if (prm.stepper || prm.dealias_rhs) return modes > (dp || prm.stepper ? 0.95 : 0.87) * all * g.nz;
-  return modes > (prm.scalar ? (dp ? 0.87 : 0.95) : dp ? 0.95 : 0.92) * all * g.nz;
+  if (prm.sgs && !small) return cols > (prm.stepper ? (dp ? 0.88 : 0.93) : dp ? 0.82 : 0.95) * all;
+  const double part = small ? 0.995
+                      : prm.stepper || prm.dealias_rhs ? (dp || prm.stepper ? 0.95 : 0.87)
+                      : prm.scalar ? (dp ? 0.87 : 0.95)
+                                   : (dp ? 0.95 : 0.92);
+  if (cols <= part * all) return false;  // so are the modes
+  int64_t modes = 0;
+  for (int kx = 0; kx <= g.mx; ++kx)
+    for (int ky = 0, kz = g.nz / 2 + 1; ky <= g.ny / 2; ++ky) {
+      beyond((int64_t)kx * kx + (int64_t)ky * ky, kz);
+      if (kz == 0) break;
+      modes += (ky == 0 || ky == g.ny / 2 ? 1 : 2) * both(kz, g.nz);
+    }
+  return modes > part * all * g.nz;
 }
 
 template <class R>
