@@ -545,6 +545,8 @@ static bool trunc_pays(const scl_plan3d* p) { return (size_t)p->g.ntot * p->esiz
 //     0.99, 0.97 0.98; 512x128x64 0.79 1.02, 0.89 1.00, 0.99 0.99
 //   IF-AB2 FP32 256x256x128 0.78 1.06, 0.89 0.99, 0.97 0.97; 512x128x64 0.89 1.04,
 //     0.99 0.96; FP64 128^3 0.89 1.04, 0.97 1.01, 1.00 0.98
+// unless the box is long in z and few modes of those columns are kept (FP64
+// 128x64x512, LES and scalar, 0.97 of the columns and a fifth of the modes: 1.05).
 // Fields of up to 8 MB stay in the caches, and the truncated passes are slower only
 // where nothing at all is left out (FP64 512x64x32 IF-AB2 0.99 1.09; FP32, LES with
 // IF-AB2, 1.00 0.92, LES and scalar 1.00 0.95).
@@ -566,8 +568,10 @@ static bool keeps_most(const scl_plan3d* p, const scl_dns_params& prm) {
     cols += both(ky, g.ny);
   }
   const double all = (double)(g.mx + 1) * g.ny;
-  if (prm.sgs && !small) return cols > (prm.stepper ? (dp ? 0.88 : 0.93) : dp ? 0.82 : 0.95) * all;
+  const bool les = prm.sgs && !small;
+  if (les && cols <= (prm.stepper ? (dp ? 0.88 : 0.93) : dp ? 0.82 : 0.95) * all) return false;
   const double part = small ? 0.995
+                      : les ? 0.6
                       : prm.stepper || prm.dealias_rhs ? (dp || prm.stepper ? 0.95 : 0.87)
                       : prm.scalar ? (dp ? 0.87 : 0.95)
                                    : (dp ? 0.95 : 0.92);
