@@ -51,16 +51,21 @@ struct PlaneCfg {
   // 32^3 134/73, 64^3 169/117, 64x64x1024 641/548, 16x256x512 421/292, FP64 32^3
   // 160/96, 16x128x512 353/251; LES 32^3 280/138, 64x16x512 473/289, FP64
   // 16x64x256 437/283; scalar 64x64x256 386/285.  With a scalar or the
-  // Smagorinsky term and y-lines of 128 points and more, planes of many entries
-  // are slower: 15232 (scalar, 32x128x64) 256/257, 13824 (both, 16x128x512)
-  // 654/845, 19584 (LES, 32x128x64) 373/428, where 10368 (LES, 16x128x512) are
-  // not: 527/411.
+  // Smagorinsky term the other side is the passes with a wavefront per field,
+  // which spread a plane's lines over the chip, and with y-lines of 128 points
+  // and more a workgroup has too many tiles of them in turn once the planes hold
+  // some 13,000 entries.  A wavefront per field / this: 8064 entries (scalar,
+  // 16x128x64) 167/143, 10368 (LES, 16x128x64) 194/172, 13824 (both, 16x128x64)
+  // 247/320, 15232 (scalar, 32x128x64) 203/258, 19584 (LES, 32x128x64) 249/368;
+  // even again at 256 points, 16128 (scalar, 16x256x64) 254/242.
   static constexpr bool fits = TY <= 32 && TX >= 1 && TX <= 16 && (size_t)LDS * sizeof(cpx<R>) <= 160 * 1024 &&
                                !((LES || SC) && NY >= 128 && NP * X1 * NY > 12000);
   // FP32 with a scalar or the Smagorinsky term: where one workgroup fills a CU's
   // LDS and there are as many as CUs, solvers running side by side are faster
   // with the separate passes (64x64 planes, scalar: 128 of them 133/123, 256
-  // 214/247; 64x32, LES and scalar: 64 of them 137/92, 256 205/251).
+  // 214/247; 64x32, LES and scalar: 64 of them 137/92, 256 205/251), though one
+  // alone is not yet (64x64, scalar: 128 of them 263/243, 256 312/284; 64x32, both:
+  // 256 350/339, 512 523/555).
   static constexpr int max_nz = sizeof(R) == 4 && (LES || SC) && LDS * 8 > 100 * 1024 ? 128 : 1024;
 };
 
