@@ -127,7 +127,9 @@ def cpu_baseline(n, steps, scl):
 # dt = 5e-4, 1000 IF-RK4 steps.  Per RHS 15 F2 (y-inverse 1 in + 3 out,
 # x-pass 3 + 2, y-forward 2 + state and stage I/O), 58 F2 per step with
 # F2 = 8 (n/2 + 1) n bytes per member (the model the roofline fraction is
-# priced against; the stage chain moves 51 F2 per step).
+# priced against, every mode through every pass; the stage chain, which leaves
+# out what lies beyond the 2/3 cut, moves about 30 F2 per step: x-pass 3.3,
+# fused y-forward 4.0 to 4.4 a stage).
 ENS2D_GROUPS = [(256, 192), (512, 48), (1024, 16)]
 ENS2D_KW = dict(dt=5e-4, c_hyper=1e-5, n_hyper=8, damp=0.1, fkmin=4.0, fkmax=5.0, eps=0.01)
 ENS2D_STEP_F2 = 58.0
@@ -329,9 +331,11 @@ def bench_ab2(scl, steps, n=512):
     }
 
 
-# turb_2d.f90's scheme on the configs[2] groups: per step an unshifted and a
-# shifted half RHS, 28 F2 (y-inverse 1 + 3 twice, x-pass 3 + 2 twice,
-# y-forward 2 + 1 then 2 + 1 + state and owz in and out).
+# turb_2d.f90's scheme on the same ensembles: per step an unshifted and a
+# shifted half RHS.  One after the other (the 512^2 and 1024^2 groups): 28 F2
+# (y-inverse 1 + 3 twice, x-pass 3 + 2 twice, y-forward 2 + 1, then 2 + 1 + state
+# and owz in and out).  Both in each pass (the 256^2 group): 24 F2 (x-pass twice,
+# y-forward 4 + state and owz in and out + 6).  The model takes 28 for all.
 TURB2D_STEP_F2 = 28
 
 
@@ -454,6 +458,9 @@ def bench_main(scl, a):
         "data": "synthetic",
         "config": {"workload": f"forced DNS {n}^3 FP32, Lawson IF-RK4 (dns-deform.f90), nu=0.01, dt=0.002, "
                    "force k^2<4 eps=0.1, 2/3 cut, IC k0=4 u0=1 iseed=1", "n": n, "parallelism": "single GPU"},
+        # against the model: every mode through every pass.  What the kernels
+        # move (impl_*) is less, as they leave out what the truncation zeroes:
+        # impl_bandwidth_frac_step is the share of the HBM peak
         "hbm_roofline_frac_step": step_bytes / (ms_per_step * 1e-3) / HBM_PEAK,
         "step_alg_bytes": step_bytes,
         "impl_step_bytes": IMPL_STEP_BYTES_F * F,
