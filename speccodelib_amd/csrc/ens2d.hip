@@ -659,17 +659,16 @@ int32_t allocate_groups(scl_ens2d& e) {
   return SCL_OK;
 }
 
-// host: kept until the stream is synchronised
 template <class R>
-int32_t upload_twiddles(int n, void** out, hipStream_t st, std::vector<std::vector<char>>& host) {
+int32_t upload_twiddles(int n, void** out, hipStream_t st) {
   std::vector<double> re, im;
   twiddles(n, re, im);
-  host.emplace_back(n * sizeof(cpx<R>));
-  cpx<R>* const h = reinterpret_cast<cpx<R>*>(host.back().data());
+  std::vector<cpx<R>> h(n);
   for (int j = 0; j < n; ++j) h[j] = mk<R>((R)re[j], (R)im[j]);
   SCL_HIP(hipMalloc(out, n * sizeof(cpx<R>)));
   // not on the legacy stream, which would end another thread's capture
-  SCL_HIP(hipMemcpyAsync(*out, h, n * sizeof(cpx<R>), hipMemcpyHostToDevice, st));
+  SCL_HIP(hipMemcpyAsync(*out, h.data(), n * sizeof(cpx<R>), hipMemcpyHostToDevice, st));
+  SCL_HIP(hipStreamSynchronize(st));
   return SCL_OK;
 }
 
@@ -699,7 +698,6 @@ extern "C" int32_t scl_ens2d_create(int32_t prec, int32_t ngroups, const int32_t
     (void)hipGetLastError();
     return set_error("no HIP device"), SCL_ENODEV;
   }
-  std::vector<std::vector<char>> tables;  // the sizes' twiddles, copied until the end
   auto* e = new scl_ens2d();
   e->prec = prec;
   e->p = *params;
@@ -731,8 +729,7 @@ extern "C" int32_t scl_ens2d_create(int32_t prec, int32_t ngroups, const int32_t
       if (t.first == n) tw = t.second;
     if (!tw) {
       void* d = nullptr;
-      const int32_t st = prec == SCL_SP ? upload_twiddles<float>(n, &d, e->stream, tables)
-                                         : upload_twiddles<double>(n, &d, e->stream, tables);
+      const int32_t st = prec == SCL_SP ? upload_twiddles<float>(n, &d, e->stream) : upload_twiddles<double>(n, &d, e->stream);
       if (st != SCL_OK) return fail(st);
       e->tw.push_back({n, d});
       tw = d;
