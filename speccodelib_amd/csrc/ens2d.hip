@@ -219,16 +219,9 @@ Cut<R> cut2d(const scl_ens2d& e, const Group& gr, bool trunc) {
 template <class R, int M, bool CUT>
 int64_t row_grid_size(const scl_ens2d& e, const Group& gr) {
   using RC = RowCfg<R, M>;
-  static int resident = 0;
-  if (!resident) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_row_adv2d<R, M, CUT>, RC::BS, 0) != hipSuccess ||
-        per_cu < 1)
-      per_cu = 1;
-    resident = per_cu;
-  }
+  static const int per_cu = blocks_per_cu(k_row_adv2d<R, M, CUT>, RC::BS);
   const int64_t ngroups = gr.g.nrow / RC::RPW;
-  return gr.row_grid ? ngroups : std::min<int64_t>(ngroups, (int64_t)resident * e.ncu);
+  return gr.row_grid ? ngroups : std::min<int64_t>(ngroups, (int64_t)per_cu * e.ncu);
 }
 
 // halves = 2 (here and in row_launch): the shifted half of scheme 1 as well;

@@ -432,15 +432,9 @@ int32_t Ops<R>::row_convec(const scl_plan3d& pl, C* W, int64_t fstride, C* tape,
     // tag gives each variant its own cached occupancy)
     auto go = [&](auto tag, auto kern) -> int32_t {
       (void)tag;
-      static int resident = 0;
-      if (!resident) {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, RC::BS, 0) != hipSuccess || per_cu < 1)
-          per_cu = 1;
-        resident = per_cu;
-      }
+      static const int per_cu = blocks_per_cu(kern, RC::BS);
       const int64_t groups = g.nrow / RC::RPW;
-      const int64_t grid = std::min<int64_t>(groups, (int64_t)resident * pl.ncu);
+      const int64_t grid = std::min<int64_t>(groups, (int64_t)per_cu * pl.ncu);
       hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(RC::BS), 0, pl.stream, W, fstride, g, scale, twp<R>(pl),
                          pl.L / M, pl.L / g.nx, tape, kin, kout);
       return check_launch("row_convec");
@@ -464,10 +458,7 @@ int32_t Ops<R>::row_ext(const scl_plan3d& pl, C* W, int64_t fs, const ExtLayout&
     // cached occupancy)
     auto go = [&](auto tag, auto kern) -> int32_t {
       (void)tag;
-      static int per_cu = 0;
-      if (!per_cu && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, RC::BS, 0) != hipSuccess ||
-                      per_cu < 1))
-        per_cu = 1;
+      static const int per_cu = blocks_per_cu(kern, RC::BS);
       const int64_t groups = g.nrow / RC::RPW;
       const int64_t grid = std::min<int64_t>(groups, (int64_t)per_cu * pl.ncu);
       hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(RC::BS), 0, pl.stream, W, fs, g, scale, d2, cs2p, tape,
@@ -500,10 +491,7 @@ int32_t Ops<R>::row_adj(const scl_plan3d& pl, C* W, int64_t fs, R scale, R c, R 
     // persistent grid, as for row_convec
     auto go = [&](auto tag, auto kern) -> int32_t {
       (void)tag;
-      static int per_cu = 0;
-      if (!per_cu && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, RC::BS, 0) != hipSuccess ||
-                      per_cu < 1))
-        per_cu = 1;
+      static const int per_cu = blocks_per_cu(kern, RC::BS);
       const int64_t groups = g.nrow / RC::RPW;
       const int64_t grid = std::min<int64_t>(groups, (int64_t)per_cu * pl.ncu);
       hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(RC::BS), 0, pl.stream, W, fs, g, scale, c, cc, part, P,

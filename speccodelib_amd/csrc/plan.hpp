@@ -47,6 +47,14 @@ struct scl_plan3d {
 namespace scl {
 int32_t plan_scratch(scl_plan3d* p, size_t nfields, void** out);
 int32_t plan_diag(scl_plan3d* p, size_t bytes, void** out);
+
+// Workgroups of bs threads of kern that a CU holds at once.  A launch keeps it in
+// a static const, which one of the threads that launch kern first initialises.
+template <class K>
+int blocks_per_cu(K kern, int bs) {
+  int n = 0;
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, bs, 0) == hipSuccess && n > 0 ? n : 1;
+}
 }  // namespace scl
 
 struct scl_dns {
