@@ -53,6 +53,8 @@ int32_t scl_version(void);
  * ------------------------------------------------------------------- */
 /* explicit handle */
 int32_t scl_plan3d_create(int32_t nx, int32_t ny, int32_t nz, int32_t prec, scl_plan3d **plan);
+/* The solvers and adjoints made on a plan keep it until they are destroyed
+ * themselves, in any order. */
 int32_t scl_plan3d_destroy(scl_plan3d *plan);
 /* Use an existing HIP stream (hipStream_t passed as void*), NULL = own. */
 int32_t scl_plan3d_set_stream(scl_plan3d *plan, void *stream);

@@ -350,6 +350,7 @@ extern "C" int32_t scl_adjoint_destroy(scl_adjoint* a) {
   if (a->acc) (void)hipFree(a->acc);
   if (a->e0) (void)hipEventDestroy(a->e0);
   if (a->e1) (void)hipEventDestroy(a->e1);
+  (void)scl_plan3d_destroy(a->plan);
   delete a;
   return SCL_OK;
 }
@@ -364,6 +365,7 @@ extern "C" int32_t scl_adjoint_create(scl_plan3d* p, const scl_dns_params* prm, 
   if (nsteps < 1 || ckpt_every < 1) return set_error("nsteps and ckpt_every must be >= 1"), SCL_EINVAL;
   auto* a = new scl_adjoint();
   a->plan = p;
+  ++p->holds;
   a->p = *prm;
   a->nsteps = nsteps;
   a->ckpt = std::min(ckpt_every, nsteps);

@@ -291,6 +291,7 @@ extern "C" int32_t scl_plan3d_create(int32_t nx, int32_t ny, int32_t nz, int32_t
 extern "C" int32_t scl_plan3d_destroy(scl_plan3d* p) {
   if (!p) return SCL_OK;
   if (p->stream) (void)hipStreamSynchronize(p->stream);
+  if (p->holds.fetch_sub(1) > 1) return SCL_OK;
   if (p->tw) (void)hipFree(p->tw);
   if (p->coef) (void)hipFree(p->coef);
   if (p->scratch) (void)hipFree(p->scratch);
@@ -967,6 +968,7 @@ static void free_dns(scl_dns* d) {
   if (d->coef) (void)hipFree(d->coef);
   if (d->ab) (void)hipFree(d->ab);
   if (d->ab_part) (void)hipFree(d->ab_part);
+  (void)scl_plan3d_destroy(d->plan);
   delete d;
 }
 
@@ -1001,6 +1003,7 @@ extern "C" int32_t scl_dns_create(scl_plan3d* p, const scl_dns_params* prm, scl_
   if (prm->scalar && !(prm->schmidt > 0)) return set_error("scalar needs schmidt > 0"), SCL_EINVAL;
   auto* d = new scl_dns();
   d->plan = p;
+  ++p->holds;
   d->p = *prm;
   d->ext = prm->sgs != 0 || prm->scalar != 0;
   d->nc = prm->scalar ? 4 : 3;

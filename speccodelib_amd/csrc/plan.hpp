@@ -1,6 +1,7 @@
 // Host-side plan and solver objects behind the opaque C handles.
 #pragma once
 
+#include <atomic>
 #include <vector>
 
 #include "scl_core.hpp"
@@ -15,6 +16,9 @@
 #endif
 
 struct scl_plan3d {
+  // the owner's handle and the solvers and adjoints on the plan: it is freed with
+  // the last of them, in whatever order they are destroyed
+  std::atomic<int> holds{1};
   int prec = SCL_SP;
   scl::Geom g{};
   int device = 0;
